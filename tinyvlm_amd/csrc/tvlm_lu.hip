@@ -5,13 +5,15 @@
 // column, info = first exactly-zero pivot (1-based), factorisation continues past it.
 //
 // getrf is blocked right-looking; each panel (64 columns, 32 while more than 2048 rows remain):
-//   1. k_panel_reg  : one work-group factors the panel (register-resident sub-panels, DPP argmax,
+//   1. k_panel_spec : the panel with the pivots of a few candidate rows, checked against all rows (three
+//                     rounds); the matrices for which no round stood take
+//      k_panel_reg  : one work-group factors the panel (register-resident sub-panels, DPP argmax,
 //                     LDS-only barriers) and lists the panel's composed row interchanges; panels
 //                     of more than 1024 rows of one matrix (or of a few) are factored by several
 //                     work-groups together instead (k_panel_coop, 64 columns, one exchange through
 //                     global memory per column);
 //   2. k_swap_trsm  : the interchanges on the columns left and right of the panel, and
-//                     U12 = L11^{-1} A12 for the columns right of it;
+//                     U12 = L11^{-1} A12 for the columns right of it, on the matrix cores;
 //   3. k_update     : A22 -= L21 U12 on the matrix cores (double-buffered 16-deep k-slices).
 // Panels taller than the cooperative groups hold (and taller than 8192 rows) use the
 // column-by-column k_panel + k_laswp + k_trsm instead.
@@ -262,12 +264,638 @@ __device__ int wave_compose_swaps(int first, int cnt, const int* piv, int* pd, i
     return ni + __popcll(mo);
 }
 
+// ---- speculative panel ----------------------------------------------------------------------------
+// Partial pivoting has one exchange over all rows per column; on the influence matrices of wings
+// nearly every pivot lies in the panel's diagonal block.  k_panel_spec factors a small set of
+// candidate rows on its own, eliminates all other rows against the resulting U11 and checks that
+// none of them would have been a pivot: every multiplier |l| <= 1.  When that holds everywhere, the
+// candidates' pivots are the ones partial pivoting over all rows picks (on a tie the first row, which
+// is the diagonal block's), so nothing had to be exchanged.  Three rounds:
+//   round 1 (R = 1): candidates = the panel's kb diagonal rows, no interchange among them;
+//   rounds 2, 3 (R = 2): only for matrices whose earlier rounds failed: plus up to 64 rows that broke
+//                    the check in them, column by column the worst first (keys).
+// A column whose pivot is zero or not finite, a tie among candidates, an |l| above 1 (within rounding
+// of 1 in rounds 2 and 3, where a tie is not settled by the row order) or a NaN fails the round.
+// The rounds write their result to sp.w and leave the matrix as it is: the next round copies the
+// result of one that stood, the panel kernel launched after them (k_panel_coop / k_panel_reg) copies
+// round 3's, or factors the panel itself where all failed.  A matrix whose panels failed kSpecFails
+// times in a row skips the rounds from then on.
+// On the influence matrices of rectangular and 25-degree swept wings every panel stands in round 1;
+// on the elliptic ones (pivots at the tip panels, up to 1538 rows below the diagonal) up to half in
+// round 1, most others in round 2 and, at 64 x 64, a quarter in round 3.
+//
+// Every work-group factors the candidates for itself (a 64-step chain in registers and LDS: one
+// launch and no exchange) and then takes its share of the other rows, 16 per wave and step on the
+// matrix cores: with Y = L21^T, 16 columns of the panel at a time, Y_b = Uinv_bb^T (A_b^T - sum_{c<b}
+// U_cb^T Y_c) (Uinv_bb: inverse of the 16 x 16 diagonal block).  The MFMA output layout is the
+// second operand's layout, so the blocks chain without moving between lanes.  What bounds it is the
+// candidates' chain, 64 dependent pivot steps.  Per 4096-row FP64 panel of one matrix, round 1 takes 21 us
+// (loads 2.3, chain 12.8, inverses and staging 2.8, rows 2.9; FP32 17 us) and a later round 52 us (its
+// chain 41: the pivot search and v_readlane broadcasts); the cooperative panel with an exchange per panel
+// took 153 us, with an exchange per column 327 us.
+typedef float vf4 __attribute__((ext_vector_type(4)));
+typedef double vd4 __attribute__((ext_vector_type(4)));
+
+template <typename T>
+struct Mf16;
+template <>
+struct Mf16<float> {
+    typedef vf4 vacc;
+    static __device__ __forceinline__ vacc mfma(float p, float q, vacc c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(p, q, c, 0, 0, 0);
+    }
+    // row of D in register r of lane l; also the k index lane l stands for when register r of a
+    // result is the second operand (the contraction may run in any order, the same in both operands)
+    static __device__ __forceinline__ int k(int l, int r) { return 4 * (l >> 4) + r; }
+};
+template <>
+struct Mf16<double> {
+    typedef vd4 vacc;
+    static __device__ __forceinline__ vacc mfma(double p, double q, vacc c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(p, q, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int k(int l, int r) { return (l >> 4) + 4 * r; }
+};
+
+constexpr int kSpecFails = 2;  // failed panels in a row after which a matrix skips the rounds
+// Rows that round 1 keeps per column: the one breaking the check by most among the row tiles of 16
+// with index i mod kSpecSlots.  A wing's tip rows break it in a handful of columns (up to 6), in each of
+// which the next pivots are mostly among its top rows: with one row per column 39 of the 63 panels of the
+// elliptic 64 x 64 wing need round 3, with these 17.
+constexpr int kSpecSlots = 16;
+constexpr int kSpecRounds = 3;
+constexpr int kSpecMaxRows = 32768;  // rows of a panel (the cooperative panels hold no more)
+
+// Buffers of one panel's speculative rounds (device); sets are zeroed once per factorisation.
+template <typename T>
+struct SpecBufs {
+    bool on = false;
+    T* w = nullptr;                      // results: matrix z at w + z ldw NB, {rows, NB} column-major
+    int64_t ldw = 0;
+    // this panel's [kSpecRounds - 1][batch][kSpecSlots][NB]: largest |l| > 1, with its row
+    unsigned long long* keys = nullptr;
+    int32_t* fail = nullptr;    // this panel's [kSpecRounds][batch]: the round failed
+    int32_t* ostate = nullptr;  // [batch]: failed panels in a row
+    int batch = 1;
+};
+
+// The round (1-based) whose result stands for matrix z among the first `rounds`, 0 if none.
+template <typename T>
+__device__ __forceinline__ int spec_stood(const SpecBufs<T>& sp, int z, int rounds) {
+    for (int r = 0; r < rounds; r++)
+        if (sp.fail[r * sp.batch + z] == 0) return r + 1;
+    return 0;
+}
+
+// Whether one of the rounds stood for matrix z (the failure count is kept by the one `keeper` thread).
+template <typename T>
+__device__ __forceinline__ bool spec_settled(const SpecBufs<T>& sp, int z, bool keeper) {
+    const bool ok = spec_stood(sp, z, kSpecRounds) != 0;
+    if (keeper) {
+        if (ok)
+            sp.ostate[z] = 0;
+        else if (sp.ostate[z] < kSpecFails)
+            sp.ostate[z]++;
+    }
+    return ok;
+}
+
+// Copies a round's result into the panel; thread id of count.
+template <typename T>
+__device__ __forceinline__ void spec_commit(const SpecBufs<T>& sp, int z, T* a, int64_t lda, int n, int k0, int kb,
+                                            int id, int count) {
+    const T* w = sp.w + (int64_t)z * sp.ldw * NB;
+    const int m = n - k0;
+    for (int r = id; r < m; r += count)
+#pragma unroll 8
+        for (int j = 0; j < kb; j++) a[(k0 + r) + (int64_t)(k0 + j) * lda] = w[r + (int64_t)j * sp.ldw];
+}
+
+__device__ __forceinline__ double lane_value(double v, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+__device__ __forceinline__ float lane_value(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// 1/v to about an ulp (the hardware estimate and Newton steps); spec_pivot_ok bounds v so that none of
+// the steps overflows.
+__device__ __forceinline__ double spec_recip(double v) {
+    double y = __builtin_amdgcn_rcp(v);
+    y = fma(y, fma(-v, y, 1.0), y);
+    return fma(y, fma(-v, y, 1.0), y);
+}
+__device__ __forceinline__ float spec_recip(float v) {
+    const float y = __builtin_amdgcn_rcpf(v);
+    return fmaf(y, fmaf(-v, y, 1.0f), y);
+}
+__device__ __forceinline__ bool spec_pivot_ok(double v) { return fabs(v) > 1e-290 && fabs(v) < 1e290; }
+__device__ __forceinline__ bool spec_pivot_ok(float v) { return fabsf(v) > 1e-30f && fabsf(v) < 1e30f; }
+
+// Lane N of every row of 16 lanes, to the whole row.
+template <int N>
+__device__ __forceinline__ double row_value(double v) {
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, 0x150 + N, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(lo, lo, 0x150 + N, 0xf, 0xf, true));
+}
+template <int N>
+__device__ __forceinline__ float row_value(float v) {
+    const int q = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(q, q, 0x150 + N, 0xf, 0xf, true));
+}
+
+// x[i] += nl u_i and rt[i] += nrl u_i, u_i = row_value<N>(rt[i]), for four values: one multiply-add with
+// a DPP operand each.  The leading s_nop covers the two wait
+// states between a vector write of rt and its use as a DPP operand.
+template <int N>
+__device__ __forceinline__ void row_fmac4(double* x, double* rt, double nl, double nrl) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %4, %8 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %1, %5, %8 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %2, %6, %8 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %3, %7, %8 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %4, %4, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %5, %5, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %6, %6, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %7, %7, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf"
+        : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(rt[0]), "+v"(rt[1]), "+v"(rt[2]), "+v"(rt[3])
+        : "v"(nl), "v"(nrl), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void row_fmac4(float* x, float* rt, float nl, float nrl) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %4, %8 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %5, %8 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %6, %8 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %7, %8 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %4, %4, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %5, %5, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %6, %6, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %7, %7, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf"
+        : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(rt[0]), "+v"(rt[1]), "+v"(rt[2]), "+v"(rt[3])
+        : "v"(nl), "v"(nrl), "n"(N));
+}
+
+// Steps of the candidates' chain in round 1, for one 16-column block (columns base + 0..15, a row per
+// lane in x).  rt holds the block's 16 pivot rows in every row of 16 lanes (lane n: row base + n of the
+// panel), so that a pivot row's value reaches all lanes as one DPP operand; reading it with v_readlane
+// instead took 2.5 times as long.
+template <typename T>
+struct SpecChain {
+    // factors the block: multipliers to x, rt and sl[k][lane]
+    template <int K>
+    static __device__ __forceinline__ void factor_step(T (&x)[16], T (&rt)[16], T (*sl)[64], int lane, int rel, int ln) {
+        const T rinv = spec_recip(row_value<K>(rt[K]));
+        const T l = rel > K ? x[K] * rinv : T(0);
+        const T rl = ln > K ? rt[K] * rinv : T(0);
+        x[K] = rel > K ? l : x[K];
+        sl[K][lane] = l;
+        constexpr int first = (K + 4) / 4 * 4;  // the next column group
+#pragma unroll
+        for (int kk = K + 1; kk < first; kk++) {
+            const T u = row_value<K>(rt[kk]);
+            rt[kk] -= rl * u;
+            x[kk] -= l * u;
+        }
+#pragma unroll
+        for (int kk = first; kk < 16; kk += 4) row_fmac4<K>(x + kk, rt + kk, -l, -rl);
+    }
+    // applies the block's step K (multipliers l, for the pivot rows rl) to another block
+    template <int K>
+    static __device__ __forceinline__ void apply_step(T (&x)[16], T (&rt)[16], T l, T rl) {
+#pragma unroll
+        for (int kk = 0; kk < 16; kk += 4) row_fmac4<K>(x + kk, rt + kk, -l, -rl);
+    }
+    // step P of X = U^{-1}, X U = I with a row of X per lane: s holds I - X_{<P} U so far, rt U's rows,
+    // rd the reciprocals of its diagonal
+    template <int P>
+    static __device__ __forceinline__ void inverse_step(T (&s)[16], const T (&rt)[16], T rd) {
+        s[P] *= row_value<P>(rd);
+#pragma unroll
+        for (int j = P + 1; j < 16; j++) s[j] -= s[P] * row_value<P>(rt[j]);
+    }
+    template <int... K>
+    static __device__ __forceinline__ void factor(T (&x)[16], T (&rt)[16], T (*sl)[64], int lane, int rel, int ln,
+                                                  std::integer_sequence<int, K...>) {
+        (factor_step<K>(x, rt, sl, lane, rel, ln), ...);
+    }
+    template <int... K>
+    static __device__ __forceinline__ void apply(T (&x)[16], T (&rt)[16], const T (*sl)[64], int lane, int pl,
+                                                 std::integer_sequence<int, K...>) {
+        (apply_step<K>(x, rt, sl[K][lane], sl[K][pl]), ...);
+    }
+    template <int... P>
+    static __device__ __forceinline__ void inverse(T (&s)[16], const T (&rt)[16], T rd,
+                                                   std::integer_sequence<int, P...>) {
+        (inverse_step<P>(s, rt, rd), ...);
+    }
+};
+
+// R rows per lane: 64 R candidates.  Grid (x: shares of the rows, z: matrices), 256 threads.
+template <typename T, int R>
+__global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t lda, int n, int k0, int kb,
+                                                    int32_t* __restrict__ ipiv, int32_t* __restrict__ perm, int64_t sb,
+                                                    SpecBufs<T> sp, int round) {
+    using M = Mf16<T>;
+    constexpr int KC = NB / 4;  // columns per wave: wave g holds columns [16 g, 16 g + 16)
+    const int z = blockIdx.z, t = threadIdx.x, lane = t & 63;
+    const int g = __builtin_amdgcn_readfirstlane(t >> 6);
+    a += (int64_t)z * sb;
+    if constexpr (R == 2) {
+        const int stood = spec_stood(sp, z, round - 1);
+        if (stood == round - 1) spec_commit(sp, z, a, lda, n, k0, kb, blockIdx.x * 256 + t, gridDim.x * 256);
+        if (stood != 0) return;
+    }
+    int32_t* fail = sp.fail + (round - 1) * sp.batch + z;
+    if (sp.ostate[z] >= kSpecFails) {
+        if (blockIdx.x == 0 && t == 0) *fail = 1;
+        return;
+    }
+    const int m = n - k0;
+    __shared__ T sU[NB][NB + 1];     // the factored diagonal block, rows in pivot order, U negated
+    __shared__ T sInv[4][16][17];    // inverses of U's 16 x 16 diagonal blocks
+    __shared__ T s_l[2][KC][64 * R];  // multipliers of a column block
+    __shared__ int s_pv[2][KC];      // its pivots
+    __shared__ int s_row[64 * R];    // candidate -> row (relative to k0), -1: none
+    __shared__ int s_pos[64 * R];    // candidate -> final row (candidates that became no pivot)
+    __shared__ uint32_t s_cmap[R == 2 ? kSpecMaxRows / 32 : 1];  // rows that are candidates below the diagonal block
+    __shared__ int s_bad;
+    // candidates: the diagonal rows, from round 2 on also rows of the earlier rounds' keys
+    int crow = -1;  // row of candidate 64 + lane
+    if constexpr (R == 2) {
+        for (int e = t; e < (m + 31) / 32; e += 256) s_cmap[e] = 0u;
+        // round by round, lane = column: its worst row first, then its other rows; entry e of the list
+        // sits in lane e
+        int count = 0;
+        for (int rd = 0; rd < round - 1; rd++) {
+            const unsigned long long* keys = sp.keys + ((int64_t)(rd * sp.batch + z) * kSpecSlots) * NB + lane;
+            unsigned long long key[kSpecSlots + 1];
+            key[0] = 0ull;
+#pragma unroll
+            for (int s = 1; s <= kSpecSlots; s++) key[s] = keys[(s - 1) * NB];
+#pragma unroll
+            for (int s = 1; s <= kSpecSlots; s++) key[0] = key[s] > key[0] ? key[s] : key[0];
+#pragma unroll
+            for (int s = 0; s <= kSpecSlots; s++) {
+                const int row = key[s] != 0ull ? (int)~(uint32_t)key[s] : -1;
+                for (unsigned long long todo = __ballot(row >= kb && row < m); todo != 0ull && count < 64;
+                     todo &= todo - 1) {
+                    const int r = __builtin_amdgcn_readlane(row, __ffsll((long long)todo) - 1);
+                    if (__ballot(crow == r) != 0ull) continue;
+                    crow = lane == count ? r : crow;
+                    count++;
+                }
+            }
+        }
+    }
+    if (t < 64) {
+        s_row[lane] = lane < kb ? lane : -1;
+        if constexpr (R == 2) s_row[64 + lane] = crow;
+        if (lane == 0) s_bad = 0;
+    }
+    __syncthreads();
+    if constexpr (R == 2)
+        if (t < 64 && crow >= 0) atomicOr(&s_cmap[crow >> 5], 1u << (crow & 31));
+    T x[R][KC];
+    bool act[R];
+    int step[R];  // column at which this row became the pivot
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+        const int row = s_row[64 * q + lane];
+        act[q] = row >= 0;
+        step[q] = -1;
+#pragma unroll
+        for (int k = 0; k < KC; k++) {
+            const int c = KC * g + k;
+            x[q][k] = (act[q] && c < kb) ? a[(k0 + row) + (int64_t)(k0 + c) * lda]
+                                         : (R == 1 && lane == c ? T(1) : T(0));  // round 1: identity beyond kb
+        }
+    }
+    // the wave's first 16 other rows, in flight while the candidates are factored: lane l holds row
+    // l % 16, columns M::k(l, r) of each 16-block
+    const int tiles = (m - kb + 15) / 16, ln = lane & 15;
+    typename M::vacc y[4];
+    auto load_rows = [&](int tile) {
+        const int row = kb + 16 * tile + ln;
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                y[b][r] = (tile < tiles && row < m)
+                              ? a[(k0 + row) + (int64_t)(k0 + 16 * b + M::k(lane, r)) * lda]
+                              : T(0);
+    };
+    // with more than one work-group, the first writes the candidates' result instead
+    const int share = gridDim.x > 1 ? (int)blockIdx.x - 1 : 0, shares = gridDim.x > 1 ? gridDim.x - 1 : 1;
+    if (share >= 0) load_rows(4 * share + g);
+    // where the rows are as the interchanges go on: src = candidate now at position `lane`, oval =
+    // candidate now at the place of candidate 64 + lane; pp = the position pivot `lane` came from
+    int src = lane, oval = 64 + lane, pp = lane;
+    bool bad = false, over1 = false;
+    // candidate p becomes the pivot of column j
+    auto take = [&](int j, int p) {
+        if constexpr (R == 2) {
+            const int did = __builtin_amdgcn_readlane(src, j);
+            if (p != did) {  // position j's row and p change places
+                const unsigned long long in = __ballot(src == p);
+                if (in != 0ull) {
+                    const int jj = __ffsll((long long)in) - 1;
+                    pp = lane == j ? jj : pp;
+                    src = lane == j ? p : (lane == jj ? did : src);
+                } else {
+                    const int e = (__ffsll((long long)__ballot(oval == p)) - 1) & 63;
+                    const int place = __builtin_amdgcn_readlane(crow, e);
+                    pp = lane == j ? place : pp;
+                    src = lane == j ? p : src;
+                    oval = lane == e ? did : oval;
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < R; q++)
+            if (64 * q + lane == p) {
+                act[q] = false;
+                step[q] = j;
+            }
+    };
+    if constexpr (R == 1) {
+        constexpr auto k16 = std::make_integer_sequence<int, KC>{};
+#pragma unroll 1
+        for (int b = 0; b < 4; b++) {
+            const int buf = b & 1, pl = KC * b + ln;  // lane of the block's pivot row ln
+            if (g >= b) {
+                // this wave's columns in the block's pivot rows, for every row of 16 lanes
+                T rt[KC];
+                if (g == b) {  // factor the block; the waves right of it apply it after the barrier
+#pragma unroll
+                    for (int k = 0; k < KC; k++) rt[k] = __shfl(x[0][k], pl);
+                    SpecChain<T>::factor(x[0], rt, s_l[buf], lane, lane - KC * b, ln, k16);
+                }
+                lds_sync();
+                if (g > b) {
+#pragma unroll
+                    for (int k = 0; k < KC; k++) rt[k] = __shfl(x[0][k], pl);
+                    SpecChain<T>::apply(x[0], rt, s_l[buf], lane, pl, k16);
+                }
+            } else {
+                lds_sync();
+            }
+        }
+        step[0] = lane;
+    } else {
+#pragma unroll 1
+        for (int b = 0; b < 4; b++) {
+            if (KC * b >= kb) break;
+            const int buf = b & 1;
+            if (g == b) {
+#pragma unroll
+                for (int k = 0; k < KC; k++) {
+                    const int j = KC * b + k;
+                    if (j < kb) {
+                        const int did = __builtin_amdgcn_readlane(src, j);  // the row at position j
+                        T v[R];
+#pragma unroll
+                        for (int q = 0; q < R; q++) v[q] = act[q] ? (T)fabs(x[q][k]) : T(-1);
+                        const T dv = did >= 64 ? lane_value(v[R - 1], did & 63) : lane_value(v[0], did);
+                        int p = did;
+                        if (__ballot(v[0] > dv || v[R - 1] > dv) != 0ull) {
+                            T best = v[0];
+                            int bi = lane;
+                            argmax_merge(best, bi, v[R - 1], 64 + lane);
+                            wave_argmax(best, bi);
+                            p = bi;
+                            bad = bad || __popcll(__ballot(v[0] == best)) + __popcll(__ballot(v[R - 1] == best)) != 1;
+                        }
+                        take(j, p);
+                        // xr: the pivot's row among the lane's R rows
+                        auto eliminate = [&](T (&xr)[KC]) {
+                            const T rinv = spec_recip(lane_value(xr[k], p & 63));
+                            T l[R];
+#pragma unroll
+                            for (int q = 0; q < R; q++) {
+                                l[q] = act[q] ? x[q][k] * rinv : T(0);
+                                x[q][k] = act[q] ? l[q] : x[q][k];
+                                s_l[buf][k][64 * q + lane] = l[q];
+                            }
+                            if (lane == 0) s_pv[buf][k] = p;
+                            T u[KC];
+#pragma unroll
+                            for (int kk = k + 1; kk < KC; kk++) u[kk] = lane_value(xr[kk], p & 63);
+#pragma unroll
+                            for (int kk = k + 1; kk < KC; kk++)
+#pragma unroll
+                                for (int q = 0; q < R; q++) x[q][kk] -= l[q] * u[kk];
+                        };
+                        if (p < 64)
+                            eliminate(x[0]);
+                        else
+                            eliminate(x[R - 1]);
+                    }
+                }
+            }
+            lds_sync();
+            if (g != b) {
+                const int kn = min(KC, kb - KC * b);
+                int pn = __builtin_amdgcn_readfirstlane(s_pv[buf][0]);
+                T lnx[R];
+#pragma unroll
+                for (int q = 0; q < R; q++) lnx[q] = s_l[buf][0][64 * q + lane];
+                for (int k = 0; k < kn; k++) {
+                    const int p = pn, kx = k + 1 < kn ? k + 1 : k;
+                    T l[R];
+#pragma unroll
+                    for (int q = 0; q < R; q++) {
+                        l[q] = lnx[q];
+                        lnx[q] = s_l[buf][kx][64 * q + lane];
+                    }
+                    const int pv = s_pv[buf][kx];
+                    take(KC * b + k, p);
+                    if (g > b) {
+                        T u[KC];
+                        if (p < 64) {
+#pragma unroll
+                            for (int kk = 0; kk < KC; kk++) u[kk] = lane_value(x[0][kk], p & 63);
+                        } else {
+#pragma unroll
+                            for (int kk = 0; kk < KC; kk++) u[kk] = lane_value(x[R - 1][kk], p & 63);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int kk = 0; kk < KC; kk++)
+#pragma unroll
+                            for (int q = 0; q < R; q++) x[q][kk] -= l[q] * u[kk];
+                    }
+                    pn = __builtin_amdgcn_readfirstlane(pv);
+                }
+            }
+        }
+    }
+    // every multiplier of the candidates (columns before a row's own pivot) is at most 1
+#pragma unroll
+    for (int q = 0; q < R; q++)
+#pragma unroll
+        for (int k = 0; k < KC; k++) {
+            const int c = KC * g + k;
+            const bool mult = (R == 1 ? step[q] > c : act[q] || step[q] > c) && c < kb;
+            over1 = over1 || (mult && !(fabs(x[q][k]) <= T(1)));
+        }
+    // round 1 goes on to the other rows after an |l| above 1 among the candidates (they are all
+    // candidates again, the keys of the others are wanted)
+    if (R == 1 && __ballot(over1) != 0ull && lane == 0) *fail = 1;
+    bad = bad || (R == 2 && over1);
+    if (__ballot(bad) != 0ull && lane == 0) s_bad = 1;
+    // the diagonal block in pivot order (identity beyond kb), U negated for the products below
+    if (R == 2 && kb < NB)
+        for (int e = t; e < NB * NB; e += 256) {
+            const int r = e & 63, c = e >> 6;
+            if (r >= kb || c >= kb) sU[r][c] = r == c ? T(-1) : T(0);
+        }
+#pragma unroll
+    for (int q = 0; q < R; q++)
+        if (step[q] >= 0)
+#pragma unroll
+            for (int k = 0; k < KC; k++) {
+                const int c = KC * g + k;
+                if (R == 1 || c < kb) sU[step[q]][c] = c >= step[q] ? -x[q][k] : x[q][k];
+            }
+    if (g == 0) {
+        s_pos[lane] = -1;
+        if constexpr (R == 2) {
+            s_pos[64 + lane] = -1;
+            if (crow >= 0) s_pos[oval] = crow;
+        }
+    }
+    __syncthreads();
+    const bool badp = !spec_pivot_ok(sU[lane][lane]);
+    if (s_bad != 0 || __ballot(badp) != 0ull) {
+        if (blockIdx.x == 0 && t == 0) *fail = 1;
+        // with a pivot that is not finite or zero the products below mean nothing
+        return;
+    }
+    T* w = sp.w + (int64_t)z * sp.ldw * NB;
+    if (blockIdx.x == 0) {
+        for (int e = t; e < NB * kb; e += 256) {
+            const int r = e % NB, c = e / NB;
+            if (r < kb) w[r + (int64_t)c * sp.ldw] = c >= r ? -sU[r][c] : sU[r][c];
+        }
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+            const int pos = s_pos[64 * q + lane];
+            if (pos >= 0 && step[q] < 0)
+#pragma unroll
+                for (int k = 0; k < KC; k++)
+                    if (KC * g + k < kb) w[pos + (int64_t)(KC * g + k) * sp.ldw] = x[q][k];
+        }
+        if (g == 0) {
+            if (lane < kb) ipiv[(int64_t)z * n + k0 + lane] = k0 + pp + 1;
+            // composed interchanges (destination, source), as wave_compose_swaps lists them
+            int32_t* out = perm + (int64_t)z * kPermInts;
+            const bool in_pair = lane < kb && src != lane;
+            const bool out_pair = R == 2 && crow >= 0 && oval != 64 + lane;
+            const unsigned long long mi = __ballot(in_pair), mo = __ballot(out_pair);
+            const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+            const int ni = __popcll(mi);
+            if (in_pair) {
+                const int e = __popcll(mi & below);
+                out[1 + 2 * e] = k0 + lane;
+                out[2 + 2 * e] = k0 + s_row[src];
+            }
+            if (out_pair) {
+                const int e = ni + __popcll(mo & below);
+                out[1 + 2 * e] = k0 + crow;
+                out[2 + 2 * e] = k0 + s_row[oval];
+            }
+            if (lane == 0) out[0] = ni + __popcll(mo);
+        }
+    }
+    if (m <= kb || share < 0) return;
+    // inverse of U's diagonal block g, a row per lane (in every row of 16 lanes)
+    {
+        T rt[16], s[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            rt[i] = -sU[16 * g + ln][16 * g + i];  // (the multipliers below the diagonal are not read)
+            s[i] = i == ln ? T(1) : T(0);
+        }
+        const T rd = T(-1) / sU[16 * g + ln][16 * g + ln];
+        SpecChain<T>::inverse(s, rt, rd, std::make_integer_sequence<int, 16>{});
+        if (lane < 16)
+#pragma unroll
+            for (int i = 0; i < 16; i++) sInv[g][ln][i] = s[i];
+    }
+    __syncthreads();
+    // the other rows, 16 per wave and step
+    const T one = T(1), strict = R == 2 ? T(1) - T(64) * (sizeof(T) == 8 ? (T)2.2e-16 : (T)1.2e-7f) : T(1);
+    bool failed = false;
+    for (int tile = 4 * share + g; tile < tiles; tile += 4 * shares) {
+        if (tile >= 4 * shares) load_rows(tile);  // the first tile is here already
+        const int row = kb + 16 * tile + ln;
+        bool use = row < m;
+        if constexpr (R == 2) use = use && ((s_cmap[row >> 5] >> (row & 31)) & 1u) == 0u;
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+#pragma unroll
+            for (int c = 0; c < b; c++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    y[b] = M::mfma(sU[16 * c + M::k(lane, r)][16 * b + ln], y[c][r], y[b]);
+            typename M::vacc s = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+            for (int r = 0; r < 4; r++) s = M::mfma(sInv[b][M::k(lane, r)][ln], y[b][r], s);
+            y[b] = s;
+        }
+        bool over = false;
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                over = over || !((T)fabs(y[b][r]) <= (R == 2 ? strict : one));
+                if (use) w[row + (int64_t)(16 * b + M::k(lane, r)) * sp.ldw] = y[b][r];
+            }
+        over = over && use;
+        if (__ballot(over) != 0ull) {
+            failed = true;
+            if (round < kSpecRounds) {  // per column the row of the largest |l| among the wave's 16
+#pragma unroll
+                for (int b = 0; b < 4; b++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const T v = use ? (T)fabs(y[b][r]) : T(0);
+                        const float f = v <= (R == 2 ? strict : one) ? 0.0f : (v < T(3e38) ? (float)v : 3.4e38f);
+                        unsigned long long key =
+                            f > 0.0f ? ((unsigned long long)__float_as_uint(f) << 32) | (uint32_t)~row : 0ull;
+#pragma unroll
+                        for (int o = 8; o > 0; o >>= 1) {
+                            const unsigned long long ok = __shfl_xor(key, o, 16);
+                            key = ok > key ? ok : key;
+                        }
+                        if (ln == 0 && key != 0ull)
+                            atomicMax(&sp.keys[((int64_t)((round - 1) * sp.batch + z) * kSpecSlots + tile % kSpecSlots) * NB + 16 * b +
+                                               M::k(lane, r)],
+                                      key);
+                    }
+            }
+        }
+    }
+    if (failed && lane == 0) *fail = 1;
+}
+
 template <typename T, int NT, int Q, int IB>
 __global__ __launch_bounds__(NT) void k_panel_reg(T* __restrict__ a, int64_t lda, int n, int k0, int kb,
                                                   int32_t* __restrict__ ipiv, int32_t* __restrict__ info,
-                                                  int32_t* __restrict__ perm, int64_t sb) {
+                                                  int32_t* __restrict__ perm, int64_t sb, SpecBufs<T> sp) {
     constexpr int NW = NT / 64;
     a += (int64_t)blockIdx.z * sb;  // batch: one matrix per blockIdx.z
+    // after a speculative panel: nothing to do where one of its earlier rounds stood; where the last did,
+    // the launch's work-groups copy its result; work-group 0 factors the panel where all failed
+    if (sp.on && spec_settled(sp, blockIdx.z, blockIdx.x == 0 && threadIdx.x == 0)) {
+        if (spec_stood(sp, blockIdx.z, kSpecRounds - 1) == 0)
+            spec_commit(sp, blockIdx.z, a, lda, n, k0, kb, blockIdx.x * NT + threadIdx.x, gridDim.x * NT);
+        return;
+    }
+    if (blockIdx.x != 0) return;
     ipiv += (int64_t)blockIdx.z * n;
     info += blockIdx.z;
     perm += (int64_t)blockIdx.z * kPermInts;
@@ -528,24 +1156,14 @@ __global__ __launch_bounds__(NT) void k_panel_reg(T* __restrict__ a, int64_t lda
 // leaves info = kCoopStalled instead of waiting for ever or indexing out of bounds.
 // Group 0 writes ipiv and the panel's composed interchanges for k_swap_trsm, as k_panel_reg does.
 //
-// Before the column-by-column exchange, an attempt with two exchanges in all: group 0 factors its
-// own NT rows with partial pivoting among them and publishes U11 (its first kb rows); every other
-// group eliminates its rows against U11 (the same operations, in the same order, as the exchange
-// loop with those pivots) and checks |a(r, c)| <= |U(c, c)| for every row and column before
-// scaling.  When that holds everywhere, partial pivoting over all rows picks exactly group 0's
-// pivots (on a tie the first row, which is group 0's), so the result is the exchange loop's; the
-// groups vote, and on any failure every group reloads its rows and runs the exchange loop.
-// Influence matrices of rectangular and swept planforms never pivot outside the diagonal block and
-// pass throughout; after kCoopOptFails failed attempts in a row the matrix (ostate, per matrix,
-// zeroed with the counters) skips them.  Counters per panel and matrix: ctr[0, NB) the columns,
-// ctr[NB] U11 published, ctr[NB + 1] the votes, ctr[NB + 2] a failed vote.
+// After a speculative panel (k_panel_spec) it factors only the matrices for which all rounds failed;
+// where the last round stood, the groups copy its result into the matrix instead.
 constexpr int kCoopMaxGroups = 64;   // work-groups of one launch; all of them must be resident at once
 constexpr int kCoopMinRows = 1024;   // shorter panels stay in one work-group (k_panel_reg)
 constexpr unsigned kCoopSpinLimit = 1u << 22;  // default bound of every wait (tvlm_lu_set_coop_spin_limit)
 constexpr int kCoopStalled = -999;
-constexpr int kCoopCtr = NB + 4;                                                      // counters per panel and matrix
-constexpr int64_t kCoopXrow = (int64_t)NB * (kCoopMaxGroups + 1) * NB + NB * NB;  // xrow per matrix (+ U11)
-constexpr int kCoopOptFails = 2;
+constexpr int kCoopCtr = NB + 4;                                         // counters per panel and matrix
+constexpr int64_t kCoopXrow = (int64_t)NB * (kCoopMaxGroups + 1) * NB;  // xrow per matrix
 
 template <typename T>
 __device__ __forceinline__ void st_agent(T* p, T v) {
@@ -562,89 +1180,19 @@ constexpr int coop_threads() {
     return sizeof(T) == 4 ? 512 : 256;
 }
 
-// Column J of the first group's local factorisation (k_panel_coop's single-exchange attempt); cols()
-// runs all NB of them in order, one instantiation per column, so the row stays in registers.
-template <typename T, int NT>
-struct CoopLocal {
-    T* r;
-    int k0, n, i;
-    bool mine;
-    int t, lane, w, wu;
-    T* s_val;
-    int *s_idx;
-    T *s_prow, *s_crow;
-    int *s_arg, *s_piv, *s_zero;
-
-    template <int J>
-    __device__ __forceinline__ void col() {
-        constexpr int NW = NT / 64;
-        const int c = k0 + J;
-        T best = T(-1);
-        int bi = n;
-        if (mine && i >= J) {
-            best = (T)fabs(r[J]);
-            bi = k0 + i;
-        }
-        wave_argmax(best, bi);
-        if (lane == 0) {
-            s_val[w] = best;
-            s_idx[w] = bi;
-        }
-        __syncthreads();
-        best = s_val[0];
-        bi = s_idx[0];
-#pragma unroll
-        for (int ww = 1; ww < NW; ww++) argmax_merge(best, bi, s_val[ww], s_idx[ww]);
-        const int pl = (bi >= k0 + J && bi < k0 + NT && bi < n) ? bi - k0 : J;
-        if (wu == (pl >> 6) && lane == (pl & 63)) {
-#pragma unroll
-            for (int jj = 0; jj < NB; jj++) s_prow[jj] = r[jj];
-        }
-        if (pl != J && wu == 0 && lane == J) {
-#pragma unroll
-            for (int jj = 0; jj < NB; jj++) s_crow[jj] = r[jj];
-        }
-        __syncthreads();
-        const T piv = s_prow[J];
-        const bool nz = piv != T(0);
-        if (t == 0) {
-            s_arg[J] = k0 + pl;
-            s_piv[J] = nz ? k0 + pl : c;
-            if (!nz && *s_zero == 0) *s_zero = c + 1;
-        }
-        if (nz && pl != J) {
-            if (wu == 0 && lane == J) {
-#pragma unroll
-                for (int jj = 0; jj < NB; jj++) r[jj] = s_prow[jj];
-            }
-            if (wu == (pl >> 6) && lane == (pl & 63)) {
-#pragma unroll
-                for (int jj = 0; jj < NB; jj++) r[jj] = s_crow[jj];
-            }
-        }
-        if (nz && mine && i > J) {
-            const T l = r[J] * (T(1) / piv);
-            r[J] = l;
-#pragma unroll
-            for (int jj = J + 1; jj < NB; jj++) r[jj] -= l * s_prow[jj];
-        }
-        __syncthreads();  // s_val, s_prow and s_crow are rewritten for the next column
-    }
-
-    template <int... J>
-    __device__ __forceinline__ void cols(std::integer_sequence<int, J...>) {
-        (col<J>(), ...);
-    }
-};
-
 template <typename T, int NT>
 __global__ __launch_bounds__(NT) void k_panel_coop(T* __restrict__ a, int64_t lda, int n, int k0, int kb, int G,
                                                    int32_t* __restrict__ ipiv, int32_t* __restrict__ info,
                                                    int32_t* __restrict__ perm, int64_t sb, int32_t* ctr, T* cval,
-                                                   int32_t* crow, T* xrow, int32_t* ostate, unsigned spin_limit,
-                                                   int32_t* fail) {
+                                                   int32_t* crow, T* xrow, unsigned spin_limit, int32_t* fail,
+                                                   SpecBufs<T> sp) {
     constexpr int NW = NT / 64, MG = kCoopMaxGroups;
     const int z = blockIdx.z, g = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
+    if (sp.on && spec_settled(sp, z, g == 0 && t == 0)) {
+        if (spec_stood(sp, z, kSpecRounds - 1) == 0)
+            spec_commit(sp, z, a + (int64_t)z * sb, lda, n, k0, kb, g * NT + t, G * NT);
+        return;
+    }
     a += (int64_t)z * sb;
     ipiv += (int64_t)z * n;
     info += z;
@@ -661,105 +1209,14 @@ __global__ __launch_bounds__(NT) void k_panel_coop(T* __restrict__ a, int64_t ld
     __shared__ int s_idx[NW];
     __shared__ T s_prow[NB], s_crow[NB];
     __shared__ int s_p, s_fail, s_zero, s_arg[NB], s_piv[NB];
-    __shared__ int s_pd[2 * NB], s_ps[2 * NB], s_pcnt, s_opt;
-    __shared__ T s_u[NB * (NB + 1) / 2];  // U11 of the attempt, row r from column r on, rows packed
+    __shared__ int s_pd[2 * NB], s_ps[2 * NB], s_pcnt;
     if (t == 0) {
         s_fail = 0;
         s_zero = 0;
     }
     for (int jj = 0; jj < kb; jj++) xs[jj * NT + t] = mine ? a[k0 + i + (int64_t)(k0 + jj) * lda] : T(0);
     __syncthreads();
-    bool settled = false;
-    const int fails = ld_agent(&ostate[z]);
-    if (kb == NB && fails < kCoopOptFails) {
-        int32_t* octr = ctr + NB;
-        T* xu = xrow + (int64_t)NB * (MG + 1) * NB;
-        bool ok = true;
-        if (g == 0) {
-            // partial pivoting among this group's rows (all NT of them hold rows: m > kCoopMinRows),
-            // each row in its thread's registers (one instantiation per column: every index is a
-            // constant); the pivot row is broadcast through s_prow, the row it displaces through s_crow
-            T r[NB];
-#pragma unroll
-            for (int jj = 0; jj < NB; jj++) r[jj] = xs[jj * NT + t];
-            CoopLocal<T, NT> L{r, k0, n, i, mine, t, lane, w, __builtin_amdgcn_readfirstlane(w), s_val, s_idx, s_prow,
-                               s_crow, s_arg, s_piv, &s_zero};
-            L.cols(std::make_integer_sequence<int, NB>{});
-#pragma unroll
-            for (int jj = 0; jj < NB; jj++) xs[jj * NT + t] = r[jj];
-            __syncthreads();
-            for (int e = t; e < kb * kb; e += NT) {
-                const int r = e / kb, cc = e % kb;
-                if (cc >= r) st_agent(&xu[r * NB + cc], xs[cc * NT + r]);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            __syncthreads();
-            if (t == 0) __hip_atomic_fetch_add(&octr[0], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            if (t == 0) {
-                unsigned spins = 0;
-                while (__hip_atomic_load(&octr[0], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < 1) {
-                    if (++spins > spin_limit) {
-                        s_fail = 1;
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                }
-            }
-            __syncthreads();
-            for (int e = t; e < kb * kb; e += NT) {
-                const int r = e / kb, cc = e % kb;
-                if (cc >= r) s_u[r * NB - r * (r - 1) / 2 + (cc - r)] = ld_agent(&xu[r * NB + cc]);
-            }
-            __syncthreads();
-            bool okr = s_fail == 0;
-            if (mine) {  // the row in registers (kb == NB here: every index below is a constant)
-                T r[NB];
-#pragma unroll
-                for (int jj = 0; jj < NB; jj++) r[jj] = xs[jj * NT + t];
-#pragma unroll
-                for (int j = 0; j < NB; j++) {
-                    const int b = j * NB - j * (j - 1) / 2;
-                    const T piv = s_u[b];
-                    okr = okr && ((T)fabs(r[j]) <= (T)fabs(piv));
-                    if (piv != T(0)) {
-                        const T l = r[j] * (T(1) / piv);
-                        r[j] = l;
-#pragma unroll
-                        for (int jj = j + 1; jj < NB; jj++) r[jj] -= l * s_u[b + (jj - j)];
-                    }
-                }
-#pragma unroll
-                for (int jj = 0; jj < NB; jj++) xs[jj * NT + t] = r[jj];
-            }
-            ok = __syncthreads_and(okr) != 0;
-        }
-        // the vote: every group counts in, a failing one first raises the flag
-        if (t == 0) {
-            if (!ok) st_agent(&octr[2], 1);
-            __hip_atomic_fetch_add(&octr[1], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-            unsigned spins = 0;
-            bool stalled = false;
-            while (__hip_atomic_load(&octr[1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < G) {
-                if (++spins > spin_limit) {
-                    stalled = true;
-                    s_fail = 1;
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-            }
-            s_opt = (!stalled && ld_agent(&octr[2]) == 0) ? 1 : 0;
-        }
-        __syncthreads();
-        settled = s_opt != 0;
-        if (g == 0 && t == 0) st_agent(&ostate[z], settled ? 0 : fails + 1);
-        if (!settled) {  // back to the rows as loaded
-            if (t == 0) s_zero = 0;
-            for (int jj = 0; jj < kb; jj++) xs[jj * NT + t] = mine ? a[k0 + i + (int64_t)(k0 + jj) * lda] : T(0);
-            __syncthreads();
-        }
-    }
-    for (int j = 0; j < kb && !settled; j++) {
+    for (int j = 0; j < kb; j++) {
         const int c = k0 + j;
         // this group's candidate: largest |a(r, c)| over its rows r >= c, first row on ties
         T best = T(-1);
@@ -875,9 +1332,14 @@ __global__ __launch_bounds__(NT) void k_panel_coop(T* __restrict__ a, int64_t ld
 }
 
 // Row interchanges of one panel on the columns outside it, then for the columns right of the panel
-// U12 = L11^{-1} A12 (L11 unit lower).  A work-group of 256 threads takes 64 columns: the swap pairs
-// are gathered for all columns at once, then scattered; U12's 64 x 64 block and L11 sit in LDS and
-// the forward substitution runs one row per step over all 64 columns.
+// U12 = L11^{-1} A12 (L11 unit lower).  A wave takes 16 columns, which no other wave touches: every
+// value it needs is read before any is written, so the waves meet only once, for L11.  U12 is formed
+// on the matrix cores, 16 rows at a time: Z_b = Linv_bb (A_b - sum_{c<b} L_bc Z_c), Linv_bb the
+// inverse of L11's 16 x 16 diagonal block (each work-group inverts the four, a wave each); the MFMA
+// output layout is the second operand's, so the blocks chain in registers, and the block's rows are
+// read through the interchanges and written once.
+// Bound by the latency of the scattered column reads: 15.4 us per launch (mean over a factorisation of
+// N = 4096, FP64) against 60.7 us for forward substitution of a 64 x 64 block in LDS, one row per step.
 // mode: 0 = interchanges on both sides and U12 on the right; 1 = interchanges only; 2 = U12 only
 // (the right blocks, no interchanges).  With gtab, the left blocks before column left0 take the
 // interchanges into their gather lists instead of their columns (deferred interchanges, below).  The
@@ -887,13 +1349,15 @@ __global__ __launch_bounds__(256) void k_swap_trsm(T* __restrict__ a, int64_t ld
                                                    const int32_t* __restrict__ perm, int64_t sb, int mode = 0,
                                                    int left0 = 0, int32_t* __restrict__ gtab = nullptr, int lbase = 0,
                                                    int rbase = -1) {
+    using M = Mf16<T>;
     a += (int64_t)blockIdx.z * sb;
     perm += (int64_t)blockIdx.z * kPermInts;
-    constexpr int kPer = 2 * NB * 64 / 256;  // gathered elements per thread
     __shared__ int s_pd[2 * NB], s_ps[2 * NB];
-    __shared__ T s_x[NB][64 + 1];
-    __shared__ T s_l[NB][NB + 1];
-    const int t = threadIdx.x;
+    __shared__ int s_map[NB];        // row of the block -> the row it comes from
+    __shared__ T s_l[NB][NB + 1];    // -L11 below the diagonal
+    __shared__ T s_inv[4][16][17];   // inverses of its 16 x 16 diagonal blocks
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     const bool left = (int)blockIdx.x < nleft;
     const int col0 = left ? lbase + blockIdx.x * 64 : (rbase < 0 ? k0 + kb : rbase) + (blockIdx.x - nleft) * 64;
     const int colend = left ? k0 : n;
@@ -906,47 +1370,80 @@ __global__ __launch_bounds__(256) void k_swap_trsm(T* __restrict__ a, int64_t ld
         if (t < cnt) g[perm[1 + 2 * t]] = v;
         return;
     }
+    const bool solve = !left && mode != 1;
+    if (cnt == 0 && !solve) return;
     for (int e = t; e < cnt; e += 256) {
         s_pd[e] = perm[1 + 2 * e];
         s_ps[e] = perm[2 + 2 * e];
     }
-    __syncthreads();
-    T v[kPer];
-#pragma unroll
-    for (int u = 0; u < kPer; u++) {
-        const int e = t + 256 * u, pr = e >> 6, col = col0 + (e & 63);
-        v[u] = (pr < cnt && col < colend) ? a[s_ps[pr] + (int64_t)col * lda] : T(0);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < kPer; u++) {
-        const int e = t + 256 * u, pr = e >> 6, col = col0 + (e & 63);
-        if (pr < cnt && col < colend) a[s_pd[pr] + (int64_t)col * lda] = v[u];
-    }
-    if (left || mode == 1) return;
-    __syncthreads();
-    for (int e = t; e < NB * 64; e += 256) {
-        const int r = e % NB, c = e / NB;
-        s_x[r][c] = (r < kb && col0 + c < colend) ? a[(k0 + r) + (int64_t)(col0 + c) * lda] : T(0);
-    }
-    for (int e = t; e < kb * kb; e += 256) {
-        const int r = e % kb, c = e / kb;
-        s_l[r][c] = a[(k0 + r) + (int64_t)(k0 + c) * lda];
-    }
-    __syncthreads();
-    const int c = t & 63, g = t >> 6;
-    for (int k = 0; k < kb - 1; k++) {
-        const T xk = s_x[k][c];
-#pragma unroll
-        for (int m = 0; m < NB / 4; m++) {
-            const int r = g + 4 * m;
-            if (r > k && r < kb) s_x[r][c] -= s_l[r][k] * xk;
+    if (t < NB) s_map[t] = k0 + t;
+    if (solve)
+        for (int e = t; e < NB * NB; e += 256) {
+            const int r = e & 63, c = e >> 6;
+            s_l[r][c] = (r < kb && c < r) ? -a[(k0 + r) + (int64_t)(k0 + c) * lda] : T(0);
         }
-        lds_sync();
+    __syncthreads();
+    if (solve) {
+        if (t < cnt && s_pd[t] >= k0 && s_pd[t] < k0 + kb) s_map[s_pd[t] - k0] = s_ps[t];
+        // unit lower: X_ij = delta_ij - sum_{p < i} L_ip X_pj, one column per lane (lanes 0..15)
+        const int b0 = 16 * w, jc = lane & 15;
+        T y[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            T s = i == jc ? T(1) : T(0);
+#pragma unroll
+            for (int p = 0; p < i; p++) s += s_l[b0 + i][b0 + p] * y[p];
+            y[i] = s;
+        }
+        if (lane < 16)
+#pragma unroll
+            for (int i = 0; i < 16; i++) s_inv[w][i][jc] = y[i];
+        __syncthreads();
     }
-    for (int e = t; e < NB * 64; e += 256) {
-        const int r = e % NB, cc = e / NB;
-        if (r < kb && col0 + cc < colend) a[(k0 + r) + (int64_t)(col0 + cc) * lda] = s_x[r][cc];
+    const int ln = lane & 15, col = col0 + 16 * w + ln;
+    const bool act = col < colend;
+    T* ac = a + (int64_t)col * lda;
+    typename M::vacc x[4];
+    if (solve) {
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int row = 16 * b + M::k(lane, r);
+                x[b][r] = (act && row < kb) ? ac[s_map[row]] : T(0);
+            }
+    }
+    // the interchanges (with U12: those into rows below the block), 32 pairs per lane group of 16
+    T v[2 * NB / 4];
+#pragma unroll
+    for (int u = 0; u < 2 * NB / 4; u++) {
+        const int e = 4 * u + (lane >> 4);
+        if (4 * u < cnt) v[u] = (act && e < cnt) ? ac[s_ps[e]] : T(0);
+    }
+#pragma unroll
+    for (int u = 0; u < 2 * NB / 4; u++) {
+        const int e = 4 * u + (lane >> 4);
+        if (4 * u < cnt && act && e < cnt) {
+            const int d = s_pd[e];
+            if (!solve || d < k0 || d >= k0 + kb) ac[d] = v[u];
+        }
+    }
+    if (!solve) return;
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+#pragma unroll
+        for (int c = 0; c < b; c++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) x[b] = M::mfma(s_l[16 * b + ln][16 * c + M::k(lane, r)], x[c][r], x[b]);
+        typename M::vacc s = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+        for (int r = 0; r < 4; r++) s = M::mfma(s_inv[b][ln][M::k(lane, r)], x[b][r], s);
+        x[b] = s;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int row = 16 * b + M::k(lane, r);
+            if (act && row < kb) ac[k0 + row] = x[b][r];
+        }
     }
 }
 
@@ -1105,9 +1602,11 @@ void launch_update(T* C, int64_t ldc, const T* A, int64_t lda, const T* B, int64
 
 template <typename T, int NT, int Q, int IB>
 int launch_panel_reg(T* a, int64_t lda, int n, int k0, int kb, int32_t* ipiv, int32_t* info, int32_t* perm,
-                     hipStream_t st, int batch, int64_t sb) {
-    hipLaunchKernelGGL((k_panel_reg<T, NT, Q, IB>), dim3(1, 1, batch), dim3(NT), 0, st, a, lda, n, k0, kb, ipiv, info,
-                       perm, sb);
+                     hipStream_t st, int batch, int64_t sb, const SpecBufs<T>& sp) {
+    // after a speculative panel, further work-groups that copy its last round's result where it stood
+    const int copies = sp.on ? (n - k0 + NT - 1) / NT : 1;
+    hipLaunchKernelGGL((k_panel_reg<T, NT, Q, IB>), dim3(copies, 1, batch), dim3(NT), 0, st, a, lda, n, k0, kb, ipiv,
+                       info, perm, sb, sp);
     TVLM_LAUNCHED();
     return TVLM_OK;
 }
@@ -1116,20 +1615,86 @@ int launch_panel_reg(T* a, int64_t lda, int n, int k0, int kb, int32_t* ipiv, in
 // per thread Q and sub-panel width IB per panel height, chosen so that the sub-panel (Q x IB values
 // per thread) and its L-block buffers stay in registers.
 template <typename T>
-int panel_fast(T* a, int64_t lda, int n, int k0, int kb, int32_t* ipiv, int32_t* info, int32_t* perm, hipStream_t st,
-               int batch, int64_t sb) {
+int panel_one_group(T* a, int64_t lda, int n, int k0, int kb, int32_t* ipiv, int32_t* info, int32_t* perm,
+                    hipStream_t st, int batch, int64_t sb, const SpecBufs<T>& sp) {
     const int m = n - k0;
-    if (m <= 256) return launch_panel_reg<T, 256, 1, 8>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb);
-    if (m <= 512) return launch_panel_reg<T, 256, 2, 8>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb);
-    if (m <= 1024) return launch_panel_reg<T, 256, 4, 8>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb);
-    if (m <= 2048) return launch_panel_reg<T, 256, 8, 8>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb);
+    if (m <= 256) return launch_panel_reg<T, 256, 1, 8>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb, sp);
+    if (m <= 512) return launch_panel_reg<T, 256, 2, 8>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb, sp);
+    if (m <= 1024) return launch_panel_reg<T, 256, 4, 8>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb, sp);
+    if (m <= 2048) return launch_panel_reg<T, 256, 8, 8>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb, sp);
     if constexpr (sizeof(T) == 8) {
-        if (m <= 4096) return launch_panel_reg<T, 256, 16, 4>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb);
-        return launch_panel_reg<T, 256, 32, 2>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb);
+        if (m <= 4096) return launch_panel_reg<T, 256, 16, 4>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb, sp);
+        return launch_panel_reg<T, 256, 32, 2>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb, sp);
     } else {
-        if (m <= 4096) return launch_panel_reg<T, 256, 16, 4>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb);
-        return launch_panel_reg<T, 256, 32, 4>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb);
+        if (m <= 4096) return launch_panel_reg<T, 256, 16, 4>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb, sp);
+        return launch_panel_reg<T, 256, 32, 4>(a, lda, n, k0, kb, ipiv, info, perm, st, batch, sb, sp);
     }
+}
+
+// Device buffers of a factorisation's speculative panels (one set of keys and flags per panel, cleared
+// once): SpecWork::panel(kp) gives the panel's, the results' buffer is shared.
+template <typename T>
+struct SpecWork {
+    SpecBufs<T> base;  // base.on = false: panels without speculation
+    SpecBufs<T> panel(int kp) const {
+        SpecBufs<T> b = base;
+        const int64_t s = kp / NB, batch = base.batch;
+        b.keys += s * (kSpecRounds - 1) * batch * kSpecSlots * NB;
+        b.fail += s * kSpecRounds * batch;
+        return b;
+    }
+    // bytes of the flags, the failure counts and the keys (zeroed before the first panel), and in all
+    static size_t zeroed(int n, int batch) {
+        const size_t panels = (size_t)(n + NB - 1) / NB;
+        return (sizeof(unsigned long long) * panels * (kSpecRounds - 1) * kSpecSlots * NB +
+                sizeof(int32_t) * (kSpecRounds * panels + 1)) * batch;
+    }
+    static size_t bytes(int n, int batch) {
+        return (zeroed(n, batch) + 255) / 256 * 256 + sizeof(T) * (size_t)n * NB * batch;
+    }
+    void place(void* ws, int n, int batch) {
+        base.batch = batch;
+        const size_t panels = (size_t)(n + NB - 1) / NB;
+        base.on = true;
+        base.keys = static_cast<unsigned long long*>(ws);
+        base.fail = reinterpret_cast<int32_t*>(base.keys + panels * (kSpecRounds - 1) * batch * kSpecSlots * NB);
+        base.ostate = base.fail + kSpecRounds * panels * batch;
+        base.w = reinterpret_cast<T*>(static_cast<char*>(ws) + (zeroed(n, batch) + 255) / 256 * 256);
+        base.ldw = n;
+    }
+};
+
+// The speculative rounds of the panel at kp; what they leave open (and the copy of the last round's
+// result) is the caller's next launch: panel_one_group or panel_coop with the same buffers.
+// Shares of the rows: 64 rows per work-group, but at most one work-group per CU in all: each factors the
+// candidates again, and a second one on a CU has its chain on the same SIMD at the same time (32 FP32
+// matrices of 4096 rows: rounds 2 and 3 took 189 us on average with two per CU).
+template <typename T>
+int panel_spec(T* a, int64_t lda, int n, int kp, int kb, int32_t* ipiv, int32_t* perm, hipStream_t st, int batch,
+               int64_t sb, const SpecBufs<T>& sp) {
+    int shares = (n - kp - kb + 63) / 64;
+    const int most = batch < 128 ? 256 / batch - 1 : 1;
+    if (shares > most) shares = most;
+    const dim3 grid(shares + 1, 1, batch);  // one more for the candidates' result
+    hipLaunchKernelGGL((k_panel_spec<T, 1>), grid, dim3(256), 0, st, a, lda, n, kp, kb, ipiv, perm, sb, sp, 1);
+    TVLM_LAUNCHED();
+    for (int round = 2; round <= kSpecRounds; round++) {
+        hipLaunchKernelGGL((k_panel_spec<T, 2>), grid, dim3(256), 0, st, a, lda, n, kp, kb, ipiv, perm, sb, sp, round);
+        TVLM_LAUNCHED();
+    }
+    return TVLM_OK;
+}
+
+// One panel in one work-group per matrix, after the speculative rounds where the factorisation has them.
+template <typename T>
+int panel_fast(T* a, int64_t lda, int n, int kp, int kb, int32_t* ipiv, int32_t* info, int32_t* perm, hipStream_t st,
+               int batch, int64_t sb, const SpecWork<T>& spec) {
+    SpecBufs<T> sp;
+    if (spec.base.on) {
+        sp = spec.panel(kp);
+        TVLM_TRY(panel_spec<T>(a, lda, n, kp, kb, ipiv, perm, st, batch, sb, sp));
+    }
+    return panel_one_group<T>(a, lda, n, kp, kb, ipiv, info, perm, st, batch, sb, sp);
 }
 
 constexpr int kFastPanelRows = 8192;  // taller panels take the column-by-column panel
@@ -1229,8 +1794,8 @@ __global__ void k_coop_fail_info(const int32_t* __restrict__ fail, int32_t* __re
 
 template <typename T>
 int panel_coop(T* a, int64_t lda, int n, int k0, int kb, int G, int32_t* ipiv, int32_t* info, int32_t* perm,
-               hipStream_t st, int batch, int64_t sb, int32_t* ctr, T* cval, int32_t* crow, T* xrow, int32_t* ostate,
-               int32_t* fail) {
+               hipStream_t st, int batch, int64_t sb, int32_t* ctr, T* cval, int32_t* crow, T* xrow, int32_t* fail,
+               const SpecBufs<T>& sp) {
     constexpr int NT = coop_threads<T>();
     static const hipError_t lds_attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_panel_coop<T, NT>),
                                                            hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1238,9 +1803,9 @@ int panel_coop(T* a, int64_t lda, int n, int k0, int kb, int G, int32_t* ipiv, i
     TVLM_HIP(lds_attr);
     TVLM_REQUIRE(G >= 2 && G * batch <= kCoopMaxGroups && kb <= NB && (int64_t)G * NT >= (int64_t)(n - k0),
                  "cooperative panel: %d groups for %d rows", G, n - k0);
-    TVLM_REQUIRE(ctr && cval && crow && xrow && ostate && fail, "cooperative panel without exchange buffers");
+    TVLM_REQUIRE(ctr && cval && crow && xrow && fail, "cooperative panel without exchange buffers");
     hipLaunchKernelGGL((k_panel_coop<T, NT>), dim3(G, 1, batch), dim3(NT), kCoopLdsBytes, st, a, lda, n, k0, kb, G,
-                       ipiv, info, perm, sb, ctr, cval, crow, xrow, ostate, g_coop_spin_limit.load(), fail);
+                       ipiv, info, perm, sb, ctr, cval, crow, xrow, g_coop_spin_limit.load(), fail, sp);
     TVLM_LAUNCHED();
     return TVLM_OK;
 }
@@ -1296,7 +1861,7 @@ constexpr double kLookaheadPairBytes = 256.0 * 1024 * 1024;
 
 template <typename T>
 int getrf_lookahead(T* a, int64_t lda, int n, int batch, int64_t sb, int32_t* ipiv, int32_t* info, int32_t* perm,
-                    hipStream_t st) {
+                    hipStream_t st, const SpecWork<T>& spec) {
     LookaheadStreams* L = nullptr;
     TVLM_TRY(lookahead_streams(st, &L));
     int32_t* perm2 = perm + (size_t)batch * kPermInts;
@@ -1313,7 +1878,7 @@ int getrf_lookahead(T* a, int64_t lda, int n, int batch, int64_t sb, int32_t* ip
     auto blocks = [](int cols) { return cols > 0 ? (cols + 63) / 64 : 0; };
     auto at = [&](int r, int c) { return a + r + (int64_t)c * lda; };
     int k0 = 0, j1 = n < NB ? n : NB;
-    TVLM_TRY(panel_fast<T>(a, lda, n, k0, j1, ipiv, info, perm, st, batch, sb));
+    TVLM_TRY(panel_fast<T>(a, lda, n, k0, j1, ipiv, info, perm, st, batch, sb, spec));
     TVLM_TRY(swaps(k0, j1, perm, 0, 0, 0, j1, blocks(n - j1)));
     while (j1 < n) {
         const int kr = j1 - k0, m = n - j1;  // rank of the pending update; trailing size
@@ -1331,7 +1896,7 @@ int getrf_lookahead(T* a, int64_t lda, int n, int batch, int64_t sb, int32_t* ip
             TVLM_HIP(hipEventRecord(L->rest_done, L->side));
         }
         if (!pair) {
-            TVLM_TRY(panel_fast<T>(a, lda, n, j1, w, ipiv, info, perm, st, batch, sb));
+            TVLM_TRY(panel_fast<T>(a, lda, n, j1, w, ipiv, info, perm, st, batch, sb, spec));
             if (rest) TVLM_HIP(hipStreamWaitEvent(st, L->rest_done, 0));
             TVLM_TRY(swaps(j1, w, perm, 0, 0, blocks(j1), jw, blocks(n - jw)));
             k0 = j1;
@@ -1339,11 +1904,11 @@ int getrf_lookahead(T* a, int64_t lda, int n, int batch, int64_t sb, int32_t* ip
             continue;
         }
         const int jA = j1 + NB;  // panel A = [j1, jA), panel B = [jA, jw)
-        TVLM_TRY(panel_fast<T>(a, lda, n, j1, NB, ipiv, info, perm, st, batch, sb));
+        TVLM_TRY(panel_fast<T>(a, lda, n, j1, NB, ipiv, info, perm, st, batch, sb, spec));
         TVLM_TRY(swaps(j1, NB, perm, 0, 0, 0, jA, 1));
         launch_update<T>(at(jA, jA), lda, at(jA, j1), lda, at(j1, jA), lda, n - jA, NB, NB, sb, batch, st);
         TVLM_LAUNCHED();
-        TVLM_TRY(panel_fast<T>(a, lda, n, jA, NB, ipiv, info, perm2, st, batch, sb));
+        TVLM_TRY(panel_fast<T>(a, lda, n, jA, NB, ipiv, info, perm2, st, batch, sb, spec));
         TVLM_TRY(swaps(jA, NB, perm2, 1, j1, 1, 0, 0));
         if (rest) TVLM_HIP(hipStreamWaitEvent(st, L->rest_done, 0));
         TVLM_TRY(swaps(j1, NB, perm, 1, 0, blocks(j1), jw, blocks(n - jw)));
@@ -1481,7 +2046,7 @@ GetrfPlan getrf_plan(int n, int batch, bool allow_coop) {
 template <typename T>
 int getrf_coop_pairs(T* a, int64_t lda, int n, int batch, int64_t sb, int32_t* ipiv, int32_t* info, int32_t* perm,
                      hipStream_t st, const GetrfPlan& plan, int32_t* ctr, T* cval, int32_t* crow, T* xrow,
-                     int32_t* gtab, int32_t* ostate, int32_t* fail) {
+                     int32_t* gtab, int32_t* fail, const SpecWork<T>& spec) {
     if (n > NB) {
         const int64_t total = (int64_t)batch * ((n + NB - 1) / NB) * n;
         hipLaunchKernelGGL(k_iota_lists, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, gtab, n, total);
@@ -1493,11 +2058,16 @@ int getrf_coop_pairs(T* a, int64_t lda, int n, int batch, int64_t sb, int32_t* i
         TVLM_REQUIRE(kp % NB == 0 && s < (int)plan.steps.size() && plan.steps[s].kp == kp && plan.steps[s].kb == kb,
                      "panel at column %d (width %d) is not in the factorisation plan", kp, kb);
         const GetrfStep& p = plan.steps[s];
-        if (p.groups == 0) return panel_fast<T>(a, lda, n, kp, kb, ipiv, info, perm, st, batch, sb);
+        if (p.groups == 0) return panel_fast<T>(a, lda, n, kp, kb, ipiv, info, perm, st, batch, sb, spec);
         TVLM_REQUIRE(p.ctr_set >= 0 && p.ctr_set < plan.ctr_sets, "cooperative panel %d: counter set %d of %d", s,
                      p.ctr_set, plan.ctr_sets);
+        SpecBufs<T> sp;
+        if (spec.base.on) {
+            sp = spec.panel(kp);
+            TVLM_TRY(panel_spec<T>(a, lda, n, kp, kb, ipiv, perm, st, batch, sb, sp));
+        }
         return panel_coop<T>(a, lda, n, kp, kb, p.groups, ipiv, info, perm, st, batch, sb,
-                             ctr + (size_t)p.ctr_set * batch * kCoopCtr, cval, crow, xrow, ostate, fail);
+                             ctr + (size_t)p.ctr_set * batch * kCoopCtr, cval, crow, xrow, fail, sp);
     };
     // the left columns before left0 take the interchanges into their gather lists
     auto swap_trsm = [&](int kp, int kb, int mode, int left0) -> int {
@@ -1561,7 +2131,20 @@ int getrf(const tvlm_view* av, int32_t* ipiv, int32_t* info, void* stream, bool 
     TVLM_TRY(device_workspace(sizeof(int32_t) * kPermInts * 2 * (size_t)batch, &ws, kWsLuPerm, st));
     int32_t* perm = static_cast<int32_t*>(ws);
     const GetrfPlan plan = getrf_plan<T>(n, batch, allow_coop);
-    if (plan.path == kPathLookahead) return getrf_lookahead<T>(a, lda, n, batch, sb, ipiv, info, perm, st);
+    // Speculative panels wherever a panel kernel of at most kFastPanelRows rows or a cooperative one
+    // follows them.  With a spin limit set (a diagnostic), cooperative factorisations go without, so that
+    // the waits it bounds are run.
+    SpecWork<T> spec;
+    if (n > 0 && n <= kSpecMaxRows && (plan.path == kPathCoopPairs ? g_coop_spin_limit.load() == kCoopSpinLimit : n <= kFastPanelRows)) {
+        void* sws = nullptr;
+        TVLM_TRY(device_workspace(SpecWork<T>::bytes(n, batch), &sws, kWsLuSpec, st));
+        spec.place(sws, n, batch);
+        const int64_t words = (int64_t)(SpecWork<T>::zeroed(n, batch) / sizeof(int32_t));
+        hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st,
+                           static_cast<int32_t*>(sws), words);
+        TVLM_LAUNCHED();
+    }
+    if (plan.path == kPathLookahead) return getrf_lookahead<T>(a, lda, n, batch, sb, ipiv, info, perm, st, spec);
     if (plan.path == kPathCoopPairs) {
         // Buffers (sized by the plan): per cooperative panel and matrix kCoopCtr counters, per matrix
         // the attempt counter and the failure word (all zeroed here, once for the whole
@@ -1578,22 +2161,21 @@ int getrf(const tvlm_view* av, int32_t* ipiv, int32_t* info, void* stream, bool 
         hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)((plan.nctr + 255) / 256)), dim3(256), 0, st, ctr,
                            (int64_t)plan.nctr);
         TVLM_LAUNCHED();
-        int32_t* ostate = ctr + (size_t)plan.ctr_sets * batch * kCoopCtr;  // per matrix: failed attempts in a row
-        int32_t* fail = ostate + batch;                                     // per matrix: a wait gave up
+        int32_t* fail = ctr + (size_t)plan.ctr_sets * batch * kCoopCtr;  // per matrix: a wait gave up
         return getrf_coop_pairs<T>(a, lda, n, batch, sb, ipiv, info, perm, st, plan, ctr, cval, crow, xrow, gtab,
-                                   ostate, fail);
+                                   fail, spec);
     }
     for (int k0 = 0; k0 < n;) {
         // tall panels of one matrix are narrower: the in-panel left-looking traffic grows with width
         // squared.  A batch is bound by the trailing updates instead, whose traffic (the whole
         // trailing matrix read and written per panel) halves with the full width.
-        const int width = (n - k0 > 2048 && batch < kWidePanelBatch) ? NB / 2 : NB;
+        const int width = (!spec.base.on && n - k0 > 2048 && batch < kWidePanelBatch) ? NB / 2 : NB;
         const int kb = (n - k0 < width) ? n - k0 : width;
         const int j1 = k0 + kb;
         const int kp = k0;  // this panel's first column
         k0 = j1;
         if (n - kp <= kFastPanelRows) {
-            TVLM_TRY(panel_fast<T>(a, lda, n, kp, kb, ipiv, info, perm, st, batch, sb));
+            TVLM_TRY(panel_fast<T>(a, lda, n, kp, kb, ipiv, info, perm, st, batch, sb, spec));
             const int nleft = (kp + 63) / 64, nright = (n - j1 + 63) / 64;
             if (nleft + nright > 0) {
                 hipLaunchKernelGGL(k_swap_trsm<T>, dim3(nleft + nright, 1, batch), dim3(256), 0, st, a, lda, n, kp, kb,
