@@ -406,6 +406,13 @@ __device__ __forceinline__ float row_value(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(q, q, 0x150 + N, 0xf, 0xf, true));
 }
 
+// Lane l - N of every row of 16 lanes (cyclic).
+template <int N>
+__device__ __forceinline__ float row_rotated(float v) {
+    const int q = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(q, q, 0x120 + N, 0xf, 0xf, true));
+}
+
 // x[i] += nl u_i and rt[i] += nrl u_i, u_i = row_value<N>(rt[i]), for four values: one multiply-add with
 // a DPP operand each.  The leading s_nop covers the two wait
 // states between a vector write of rt and its use as a DPP operand.
@@ -864,17 +871,17 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
                     for (int r = 0; r < 4; r++) {
                         const T v = use ? (T)fabs(y[b][r]) : T(0);
                         const float f = v <= (R == 2 ? strict : one) ? 0.0f : (v < T(3e38) ? (float)v : 3.4e38f);
-                        unsigned long long key =
-                            f > 0.0f ? ((unsigned long long)__float_as_uint(f) << 32) | (uint32_t)~row : 0ull;
-#pragma unroll
-                        for (int o = 8; o > 0; o >>= 1) {
-                            const unsigned long long ok = __shfl_xor(key, o, 16);
-                            key = ok > key ? ok : key;
-                        }
-                        if (ln == 0 && key != 0ull)
-                            atomicMax(&sp.keys[((int64_t)((round - 1) * sp.batch + z) * kSpecSlots + tile % kSpecSlots) * NB + 16 * b +
-                                               M::k(lane, r)],
-                                      key);
+                        float top = fmaxf(f, row_rotated<8>(f));
+                        top = fmaxf(top, row_rotated<4>(top));
+                        top = fmaxf(top, row_rotated<2>(top));
+                        top = fmaxf(top, row_rotated<1>(top));
+                        const bool hit = f > 0.0f && f == top;
+                        const uint32_t first = (uint32_t)(__ballot(hit) >> (lane & 48)) & ((1u << ln) - 1u);
+                        if (hit && first == 0u)
+                            atomicMax(&sp.keys[((int64_t)((round - 1) * sp.batch + z) * kSpecSlots + tile % kSpecSlots) *
+                                                   NB +
+                                               16 * b + M::k(lane, r)],
+                                      ((unsigned long long)__float_as_uint(f) << 32) | (uint32_t)~row);
                     }
             }
         }
