@@ -215,12 +215,11 @@ inline void fl_tile_shape(int ns, int rows, int recv_blocks, int& sw, int& rh, i
 // circulation shed at step i - q, in slot (i - q) mod slots.  Same tiling and arithmetic as
 // k_wake_lattice.
 template <int RH>
-__global__ __launch_bounds__(kThreads) void k_fl_wake(FlConst c, FlBufs d, const FlState* __restrict__ st,
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_fl_wake(FlConst c, FlBufs d, const FlState* __restrict__ st,
                                                       double* __restrict__ partial, int64_t spart, int step, int rows,
                                                       int sw, int tiles_span) {
-    constexpr int SWG = kWaves * kLatChunkMax;
-    __shared__ double sverts[(RH + 1) * (SWG + 1) * 3];
-    __shared__ double sgam[RH * SWG];
+    __shared__ LatTile<RH> tile_s;
+    double *const sverts = tile_s.verts, *const sgam = tile_s.gam;
     __shared__ double sred[kWaves][kRecv];
     const int b = blockIdx.z;
     if (st[b].done) return;
@@ -248,6 +247,8 @@ __global__ __launch_bounds__(kThreads) void k_fl_wake(FlConst c, FlBufs d, const
         sgam[e] = WG[(int64_t)slot * ns + s0 + sp];
     }
     __syncthreads();
+    lattice_segments<RH>(tile_s, swe, rhe);
+    __syncthreads();
     const int lane = threadIdx.x & (kRecv - 1);
     const int wave = threadIdx.x / kRecv;
     const int p = blockIdx.x * kRecv + lane;
@@ -258,7 +259,7 @@ __global__ __launch_bounds__(kThreads) void k_fl_wake(FlConst c, FlBufs d, const
         const double* C = d.colloc + b * d.sp3;
         const double* Nn = d.normals + b * d.sp3;
         double ax = 0.0, ay = 0.0, az = 0.0;
-        lattice_chunk<RH>(sverts, sgam, swe, rhe, vw, sa, sb, C[p], C[p + N], C[p + 2 * N], ax, ay, az);
+        lattice_chunk<RH>(tile_s, swe, rhe, sa, sb, C[p], C[p + N], C[p + 2 * N], ax, ay, az);
         part = ax * Nn[p] + ay * Nn[p + N] + az * Nn[p + 2 * N];
     }
     sred[wave][lane] = part;

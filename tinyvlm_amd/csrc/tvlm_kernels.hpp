@@ -439,50 +439,150 @@ __device__ __forceinline__ void lat_pair(double& ax, double& ay, double& az, con
 
 constexpr int kLatChunkMax = 16;  // spans per wave
 
-// The lattice walk of one wave over its span chunk [sa, sb) of a staged tile (vertex rows 0..rhe,
-// vw = swe + 1 vertex columns, 3 coordinates each in sverts; circulations rhe x swe in sgam) for
-// the receiver (cx, cy, cz): chordwise segments of each vertex column with the circulation
-// difference of the two ring columns beside it, spanwise segments of each vertex row with the
-// difference of the two ring rows, the previous vertex column's terms kept in registers; the tile's
-// right edge only when sb == swe.  Adds the induced velocity to (vx, vy, vz).
+// A segment a -> b of a staged tile: b - a, and the difference of the circulations beside it.
+struct LatSegment {
+    double x, y, z, g;
+};
+
+// What a work-group stages of a tile of RH rings x 4 kLatChunkMax spans.
 template <int RH>
-__device__ __forceinline__ void lattice_chunk(const double* sverts, const double* sgam, int swe, int rhe, int vw,
-                                              int sa, int sb, double cx, double cy, double cz, double& vx, double& vy,
-                                              double& vz) {
-    double ax = 0.0, ay = 0.0, az = 0.0;  // 4 pi x the induced velocity (lat_pair leaves the factor out)
-    LatVertex prev[RH + 1], cur[RH + 1];
+struct LatTile {
+    static constexpr int kSpans = kWaves * kLatChunkMax;
+    double verts[(RH + 1) * (kSpans + 1) * 3];  // vertex rows 0..rhe x vw = swe + 1 columns
+    double gam[RH * kSpans];                    // circulations rhe x swe
+    LatSegment span[(RH + 1) * kSpans];         // vertex row q, from vertex column s to s + 1: q * swe + s
+    LatSegment chord[RH * (kSpans + 1)];        // vertex column s, from vertex row q to q + 1: q * vw + s
+};
+
+// The segments of a tile whose vertices and circulations are staged (between two barriers).  Rings
+// outside the tile count 0 in the differences: their own tile adds them.
+template <int RH>
+__device__ __forceinline__ void lattice_segments(LatTile<RH>& t, int swe, int rhe) {
+    const int vw = swe + 1;
+    for (int e = threadIdx.x; e < (rhe + 1) * swe; e += kThreads) {
+        const int q = e / swe, s = e % swe;
+        const double* v = t.verts + 3 * (q * vw + s);
+        double g = 0.0;
+        if (q < rhe) g += t.gam[q * swe + s];
+        if (q > 0) g -= t.gam[(q - 1) * swe + s];
+        t.span[e] = {v[3] - v[0], v[4] - v[1], v[5] - v[2], g};
+    }
+    for (int e = threadIdx.x; e < rhe * vw; e += kThreads) {
+        const int q = e / vw, s = e % vw;
+        const double *v = t.verts + 3 * e, *w = v + 3 * vw;
+        double g = 0.0;
+        if (s < swe) g -= t.gam[q * swe + s];
+        if (s > 0) g += t.gam[q * swe + s - 1];
+        t.chord[e] = {w[0] - v[0], w[1] - v[1], w[2] - v[2], g};
+    }
+}
+
+__device__ __forceinline__ uint32_t hi_word(double v) { return (uint32_t)__double2hiint(v); }
+
+// A staged segment for the receiver and its image, as lat_pair but without its cutoffs: low_sq keeps
+// the smallest high word of |r1 x r2|^2 met, so that the walk learns at its end whether any segment came
+// near a cutoff.  The image shares every term without a y component and the one reciprocal,
+// 1/(sq sq') = the seeded estimate, of which each takes its part: 46 issue slots (of one FP64
+// multiply-add) a pair of segments, where lat_pair with its compares and selects takes 58.
+__device__ __forceinline__ void lat_pair_fast(double& ax, double& ay, double& az, const LatVertex& a,
+                                              const LatVertex& b, const LatSegment& r, uint32_t& low_sq) {
+    const double cry = a.z * b.x - a.x * b.z;
+    const double cry2 = cry * cry;
+    const double d1xz = r.x * a.x + r.z * a.z;
+    const double d2xz = r.x * b.x + r.z * b.z;
+    const double crx = a.y * b.z - a.z * b.y, crz = a.x * b.y - a.y * b.x;
+    const double mrx = a.ym * b.z - a.z * b.ym, mrz = a.x * b.ym - a.ym * b.x;
+    const double sq = crx * crx + (crz * crz + cry2), sqm = mrx * mrx + (mrz * mrz + cry2);
+    const double inv = rcp_seeded(sq * sqm) * r.g;
+    const double t = ((d1xz + r.y * a.y) * a.ri - (d2xz + r.y * b.y) * b.ri) * (inv * sqm);
+    const double tm = ((d1xz + r.y * a.ym) * a.rim - (d2xz + r.y * b.ym) * b.rim) * (inv * sq);
+    low_sq = min(min(low_sq, hi_word(sq)), hi_word(sqm));
+    ax += t * crx;
+    ay += t * cry;
+    az += t * crz;
+    ax += tm * mrx;
+    ay -= tm * cry;
+    az += tm * mrz;
+}
+
+// lat_vertex, with the smallest high word of |r|^2 kept in low_r2.
+__device__ __forceinline__ LatVertex lat_vertex_fast(double cx, double cy, double cz, const double* v,
+                                                     uint32_t& low_r2) {
+    LatVertex f;
+    f.x = cx - v[0];
+    f.y = cy - v[1];
+    f.z = cz - v[2];
+    f.ym = -cy - v[1];
+    const double xz = f.x * f.x + f.z * f.z;
+    const double r2 = xz + f.y * f.y, r2m = xz + f.ym * f.ym;
+    f.ri = rsqrt_seeded(r2);
+    f.rim = rsqrt_seeded(r2m);
+    low_r2 = min(min(low_r2, hi_word(r2)), hi_word(r2m));
+    return f;
+}
+
+// The lattice walk of one wave over its span chunk [sa, sb) of a staged tile for the receiver
+// (cx, cy, cz): chordwise segments of each vertex column, spanwise segments of each vertex row, the
+// previous vertex column's terms kept in registers; the tile's right edge only when sb == swe.  Adds
+// the induced velocity to (vx, vy, vz).  This form applies every cutoff where it stands.
+template <int RH>
+__device__ __forceinline__ void lattice_chunk_cutoffs(const LatTile<RH>& t, int swe, int rhe, int sa, int sb, double cx,
+                                                      double cy, double cz, double& ax, double& ay, double& az) {
+    const int vw = swe + 1;
+    ax = ay = az = 0.0;  // 4 pi x the induced velocity (lat_pair leaves the factor out)
+    // per vertex column: its rhe chordwise segments, then the rhe + 1 spanwise ones to the next column
+#pragma unroll 1
+    for (int s = sa; s <= sb; s++)
+#pragma unroll 1
+        for (int e = s < sb || sb == swe ? 0 : rhe; e < (s < sb ? 2 * rhe + 1 : rhe); e++) {
+            const bool chord = e < rhe;
+            const int q = chord ? e : e - rhe, from = q * vw + s;
+            lat_pair(ax, ay, az, lat_vertex(cx, cy, cz, t.verts + 3 * from),
+                     lat_vertex(cx, cy, cz, t.verts + 3 * (from + (chord ? vw : 1))),
+                     chord ? t.chord[from].g : t.span[q * swe + s].g);
+        }
+}
+
+// The same walk without the cutoffs (lat_pair_fast); where some lane's smallest |r1 x r2|^2 or |r|^2 is
+// within a rounding of its cutoff or below it, or a result is not finite (an input that is not, or a
+// product that overflowed), the wave walks again with them.  Wakes and wings in use keep clear of the
+// cutoffs (1e-10), so that the second walk is rare.
+// Bound by FP64 VALU issue.  Per (receiver, ring) pair at RH = 4: 2.25 segment pairs of 46 slots and
+// 1.25 vertices of 25 against 58 and 24 with the cutoffs inside.
+template <int RH>
+__device__ __forceinline__ void lattice_chunk(const LatTile<RH>& t, int swe, int rhe, int sa, int sb, double cx,
+                                              double cy, double cz, double& vx, double& vy, double& vz) {
+    const int vw = swe + 1;
+    double ax = 0.0, ay = 0.0, az = 0.0;
+    uint32_t low_sq = 0xffffffffu, low_r2 = 0xffffffffu;
+    LatVertex prev[RH + 1];
 #pragma unroll
     for (int q = 0; q <= RH; q++)
-        if (q <= rhe) prev[q] = lat_vertex(cx, cy, cz, sverts + 3 * (q * vw + sa));
+        if (q <= rhe) prev[q] = lat_vertex_fast(cx, cy, cz, t.verts + 3 * (q * vw + sa), low_r2);
     for (int s = sa; s < sb; s++) {
         // chordwise segments of vertex column s (left edge of ring column s)
 #pragma unroll
-        for (int q = 0; q < RH; q++) {
-            if (q < rhe) {
-                double g = -sgam[q * swe + s];
-                if (s > 0) g += sgam[q * swe + s - 1];
-                lat_pair(ax, ay, az, prev[q], prev[q + 1], g);
-            }
-        }
+        for (int q = 0; q < RH; q++)
+            if (q < rhe) lat_pair_fast(ax, ay, az, prev[q], prev[q + 1], t.chord[q * vw + s], low_sq);
         // vertex column s+1 and the spanwise segments of ring column s
 #pragma unroll
         for (int q = 0; q <= RH; q++) {
             if (q <= rhe) {
-                cur[q] = lat_vertex(cx, cy, cz, sverts + 3 * (q * vw + s + 1));
-                double g = 0.0;
-                if (q < rhe) g += sgam[q * swe + s];
-                if (q > 0) g -= sgam[(q - 1) * swe + s];
-                lat_pair(ax, ay, az, prev[q], cur[q], g);
+                const LatVertex cur = lat_vertex_fast(cx, cy, cz, t.verts + 3 * (q * vw + s + 1), low_r2);
+                lat_pair_fast(ax, ay, az, prev[q], cur, t.span[q * swe + s], low_sq);
+                prev[q] = cur;
             }
         }
-#pragma unroll
-        for (int q = 0; q <= RH; q++) prev[q] = cur[q];
     }
     if (sb == swe) {  // right edge of the work-group tile: chordwise segments of vertex column swe
 #pragma unroll
         for (int q = 0; q < RH; q++)
-            if (q < rhe) lat_pair(ax, ay, az, prev[q], prev[q + 1], sgam[q * swe + swe - 1]);
+            if (q < rhe) lat_pair_fast(ax, ay, az, prev[q], prev[q + 1], t.chord[q * vw + swe], low_sq);
     }
+    constexpr double cut_r2 = BS<double>::cut_norm * BS<double>::cut_norm;
+    const bool near = (low_sq <= hi_word(BS<double>::cut_cross)) | (low_r2 <= hi_word(cut_r2)) |
+                      !(fabs(ax) + fabs(ay) + fabs(az) < __builtin_huge_val());
+    if (__ballot(near) != 0ull) lattice_chunk_cutoffs<RH>(t, swe, rhe, sa, sb, cx, cy, cz, ax, ay, az);
     constexpr double inv_fourpi = 1.0 / BS<double>::fourpi;
     vx += ax * inv_fourpi;
     vy += ay * inv_fourpi;
@@ -491,17 +591,14 @@ __device__ __forceinline__ void lattice_chunk(const double* sverts, const double
 
 // zs: simulations (blockIdx.z) of one launch find their receivers, wake and circulations z * zs
 // elements after simulation 0's (the tables' pointers) and write their partials z * wzs after.
-// At least 4 waves per SIMD: the hint once held the 4-row form at 128 registers when it needed 130
-// unhinted (3 waves); since a segment and its image share their y-free terms it takes 126 either way,
-// and the hint keeps a later change from dropping a wave unnoticed.
+// At least 4 waves per SIMD (the hint keeps a later change from dropping a wave unnoticed).
 template <typename TS, int RH>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_wake_lattice(TS* __restrict__ partial, RecvTable<TS> rt,
                                                            WakeTable<TS> wt, int64_t zs = 0, int64_t wzs = 0) {
     const int64_t zo = (int64_t)blockIdx.z * zs;
     partial += (int64_t)blockIdx.z * wzs;
-    constexpr int SWG = kWaves * kLatChunkMax;
-    __shared__ double sverts[(RH + 1) * (SWG + 1) * 3];
-    __shared__ double sgam[RH * SWG];
+    __shared__ LatTile<RH> st;
+    double *const sverts = st.verts, *const sgam = st.gam;
     __shared__ double sred[kWaves][kRecv];
     const int tile = blockIdx.y;
     int w = 0;
@@ -539,6 +636,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         }
     }
     __syncthreads();
+    lattice_segments<RH>(st, swe, rhe);
+    __syncthreads();
     const int lane = threadIdx.x & (kRecv - 1);
     const int wave = threadIdx.x / kRecv;
     const int p = blockIdx.x * kRecv + lane;
@@ -553,7 +652,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         const TS* no = rc.normals + zo;
         const double cx = co[li], cy = co[li + rc.cs2], cz = co[li + 2 * rc.cs2];
         double ax = 0.0, ay = 0.0, az = 0.0;
-        lattice_chunk<RH>(sverts, sgam, swe, rhe, vw, sa, sb, cx, cy, cz, ax, ay, az);
+        lattice_chunk<RH>(st, swe, rhe, sa, sb, cx, cy, cz, ax, ay, az);
         part = ax * (double)no[li] + ay * (double)no[li + rc.ns2] + az * (double)no[li + 2 * rc.ns2];
     }
     sred[wave][lane] = part;
