@@ -1,17 +1,17 @@
 // tvlm_assembly.hip -- influence-matrix assembly and wake induction on gfx950.
 //
-// lhs_assemble: every (receiver, ring) pair is independent.  A work-group owns 64 receivers
-// (one per lane, colloc + normal in registers) and TC rings whose 12 vertex coordinates are staged
-// in LDS; its 4 waves take every 4th ring, so each wave reads LDS as a broadcast and writes one
-// coalesced 64-element column segment per ring.  The work is VALU-bound (16 sqrt + 8 div per pair
-// in the exact forms, 16 rsq + 8 rcp in the fast FP32 form).
+// lhs_assemble: a work-group owns 64 receivers (one per lane, colloc + normal in registers) and a tile
+// of rings whose vertices are staged in LDS; its 4 waves walk the tile's lattice, every segment and vertex
+// once per receiver, and write one coalesced 64-element column segment per ring.
 //
 // rhs_assemble_wake_influence: receivers x wake rings with a Gamma-weighted sum per receiver.
-// The wake rings are cut into tiles of RH rows x SW spans; a work-group stages one tile's vertex
-// rows and circulations in LDS and reduces its 4 waves in LDS to one partial per receiver.  A
-// second kernel sums the partials of all tiles in a fixed order, so results are bitwise
-// reproducible (the CUDA reference uses float atomics, vlm_backend_cuda_kernels.cuh:370).
+// The wake rings are cut into tiles of rows x spans; a work-group stages one tile's vertex rows and
+// circulations in LDS, walks its lattice (every segment once, with the difference of the circulations
+// beside it) and reduces its 4 waves in LDS to one partial per receiver.  A second kernel sums the
+// partials of all tiles in a fixed order, so results are bitwise reproducible (the CUDA reference uses
+// float atomics, vlm_backend_cuda_kernels.cuh:370).
 #include <mutex>
+#include <type_traits>
 
 #include "tvlm_kernels.hpp"
 
@@ -52,7 +52,6 @@ int lhs_sections(const tvlm_view* lhs, int32_t n_surf, const tvlm_view* colloc, 
     TVLM_REQUIRE(lhs->shape[0] >= total && lhs->shape[1] >= total, "lhs smaller than the total panel count %lld",
                  (long long)total);
     const int64_t ld = lhs->stride[1];
-    constexpr int TC = sizeof(T) == 8 ? 32 : 64;
     int64_t offset_j = 0;
     for (int mj = 0; mj < n_surf; mj++) {
         RingSource<T> src;
@@ -77,7 +76,8 @@ int lhs_sections(const tvlm_view* lhs, int32_t n_surf, const tvlm_view* colloc, 
             sec.lhs = static_cast<T*>(lhs->ptr) + offset_i + offset_j * ld;
             sec.ld = ld;
             sec.tiles_x = (sec.rc.m + kRecv - 1) / kRecv;
-            const int64_t tiles_y = (n_rings + TC - 1) / TC;
+            lhs_tile_shape(sec.rc.m, src.ns, src.nc, sec.rh, sec.spans);
+            const int64_t tiles_y = lhs_tiles_y(sec);
             TVLM_REQUIRE(tiles + (int64_t)sec.tiles_x * tiles_y < (int64_t)1 << 31, "more than 2^31 tiles");
             sec.tile0 = (int32_t)tiles;
             tiles += (int64_t)sec.tiles_x * tiles_y;
@@ -100,29 +100,32 @@ int lhs_assemble(const tvlm_view* lhs, int32_t n_surf, const tvlm_view* colloc, 
     int64_t tiles = 0;
     TVLM_TRY(lhs_sections<T>(lhs, n_surf, colloc, normals, verts_wing, verts_wake, iteration, secs, tiles));
     hipStream_t st = as_stream(stream);
-    constexpr int TC = sizeof(T) == 8 ? 32 : 64;
     for (const LhsSection<T>& sc : secs) {
         T* section = sc.lhs;
         const int64_t ld = sc.ld;
         const Receivers<T>& rc = sc.rc;
         const RingSource<T>& src = sc.src;
-        dim3 grid(sc.tiles_x, (src.ns * src.nc + TC - 1) / TC);
-        if constexpr (sizeof(T) == 4) {
-            if (sigma != T(0)) {
-                // the fast form has no core model; use the exact float form for sigma != 0
-                hipLaunchKernelGGL((k_lhs_block<T, TC, 1>), grid, dim3(kThreads), 0, st, section, ld, rc, src, sigma);
-            } else {
-                hipLaunchKernelGGL((k_lhs_block<T, TC, 2>), grid, dim3(kThreads), 0, st, section, ld, rc, src, sigma);
-            }
-        } else {
-            if (sigma != T(0)) {
-                hipLaunchKernelGGL((k_lhs_block<T, TC, 1>), grid, dim3(kThreads), 0, st, section, ld, rc, src, sigma);
-            } else if (seeded) {
-                hipLaunchKernelGGL((k_lhs_block<T, TC, 3>), grid, dim3(kThreads), 0, st, section, ld, rc, src, sigma);
-            } else {
-                hipLaunchKernelGGL((k_lhs_block<T, TC, 0>), grid, dim3(kThreads), 0, st, section, ld, rc, src, sigma);
-            }
-        }
+        const dim3 grid(sc.tiles_x, (unsigned)lhs_tiles_y(sc));
+        auto launch = [&](auto mode) {
+            constexpr int MODE = decltype(mode)::value;
+            if (sc.rh == 4)
+                hipLaunchKernelGGL((k_lhs_block<T, 4, MODE>), grid, dim3(kThreads), 0, st, section, ld, rc, src, sigma,
+                                   sc.spans);
+            else if (sc.rh == 2)
+                hipLaunchKernelGGL((k_lhs_block<T, 2, MODE>), grid, dim3(kThreads), 0, st, section, ld, rc, src, sigma,
+                                   sc.spans);
+            else
+                hipLaunchKernelGGL((k_lhs_block<T, 1, MODE>), grid, dim3(kThreads), 0, st, section, ld, rc, src, sigma,
+                                   sc.spans);
+        };
+        if (sigma != T(0))  // the FP32 rsqrt and FP64 seeded forms have no core model
+            launch(std::integral_constant<int, 1>{});
+        else if constexpr (sizeof(T) == 4)
+            launch(std::integral_constant<int, 2>{});
+        else if (seeded)
+            launch(std::integral_constant<int, 3>{});
+        else
+            launch(std::integral_constant<int, 0>{});
         TVLM_LAUNCHED();
     }
     return TVLM_OK;
@@ -230,17 +233,10 @@ int wake_influence(const tvlm_view* rhs, int32_t n_surf, const tvlm_view* gamma_
             return TVLM_OK;
         }
     }
-    if constexpr (sizeof(T) == 4) {
-        if (sigma != T(0))
-            hipLaunchKernelGGL((k_wake_partials<T, T, 1>), grid, dim3(kThreads), 0, st, (T*)ws, rt, wt, sigma);
-        else
-            hipLaunchKernelGGL((k_wake_partials<T, T, 2>), grid, dim3(kThreads), 0, st, (T*)ws, rt, wt, sigma);
-    } else {
-        if (sigma != T(0))
-            hipLaunchKernelGGL((k_wake_partials<T, T, 1>), grid, dim3(kThreads), 0, st, (T*)ws, rt, wt, sigma);
-        else
-            hipLaunchKernelGGL((k_wake_partials<T, T, 0>), grid, dim3(kThreads), 0, st, (T*)ws, rt, wt, sigma);
-    }
+    if (sigma != T(0))
+        launch_wake_partials<T, 1>(grid, st, (T*)ws, rt, wt, sigma);
+    else
+        launch_wake_partials<T, sizeof(T) == 4 ? 2 : 0>(grid, st, (T*)ws, rt, wt, sigma);
     TVLM_LAUNCHED();
     launch_wake_reduce<T>(static_cast<T*>(rhs->ptr), rhs->stride[0], (const T*)ws, tiles, total, st);
     TVLM_LAUNCHED();
@@ -360,13 +356,13 @@ int tvlm_lhs_group_assemble_f64(tvlm_lhs_group* G, int32_t n_items, int32_t seed
     using tvlm::k_lhs_grouped;
     const dim3 grid((unsigned)tiles);
     if (sigma != 0.0)
-        hipLaunchKernelGGL((k_lhs_grouped<double, 32, 1>), grid, dim3(tvlm::kThreads), 0, st, G->secs, G->tile0,
+        hipLaunchKernelGGL((k_lhs_grouped<double, 1>), grid, dim3(tvlm::kThreads), 0, st, G->secs, G->tile0,
                            G->chunk, (int)tiles, sigma);
     else if (seeded)
-        hipLaunchKernelGGL((k_lhs_grouped<double, 32, 3>), grid, dim3(tvlm::kThreads), 0, st, G->secs, G->tile0,
+        hipLaunchKernelGGL((k_lhs_grouped<double, 3>), grid, dim3(tvlm::kThreads), 0, st, G->secs, G->tile0,
                            G->chunk, (int)tiles, sigma);
     else
-        hipLaunchKernelGGL((k_lhs_grouped<double, 32, 0>), grid, dim3(tvlm::kThreads), 0, st, G->secs, G->tile0,
+        hipLaunchKernelGGL((k_lhs_grouped<double, 0>), grid, dim3(tvlm::kThreads), 0, st, G->secs, G->tile0,
                            G->chunk, (int)tiles, sigma);
     TVLM_LAUNCHED();
     return TVLM_OK;

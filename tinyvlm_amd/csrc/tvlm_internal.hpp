@@ -130,57 +130,6 @@ struct BS<float> {
     static constexpr float cut_norm = 1e-5f;    // RCUT2 on |r1|, |r2|
 };
 
-// Exact form of one unit straight segment a->b at c (Katz-Plotkin eq. 10.115), operation for
-// operation as kernel_biosavart / dkernel_biosavart (kernels.ispc:69-89 / :382-402) with IEEE
-// sqrt and division.  With sigma == 0 the core term sqrt(sq*sq + 0) equals sq exactly in IEEE
-// arithmetic, so the SIGMA=false instantiation skips that square root.
-template <typename T, bool SIGMA>
-__device__ __forceinline__ v3<T> segment_exact(const v3<T>& c, const v3<T>& a, const v3<T>& b, T sigma) {
-    const v3<T> r0 = b - a;
-    const v3<T> r1 = c - a;
-    const v3<T> r2 = c - b;
-    const v3<T> cr = cross(r1, r2);
-    const T r1n = sqrt(dot(r1, r1));
-    const T r2n = sqrt(dot(r2, r2));
-    const T sq = dot(cr, cr);
-    if ((sq < BS<T>::cut_cross) || (r1n < BS<T>::cut_norm) || (r2n < BS<T>::cut_norm)) return {T(0), T(0), T(0)};
-    T core;
-    if constexpr (SIGMA) {
-        const T sm = sigma * sigma * dot(r0, r0);
-        core = sqrt(sq * sq + sm * sm);
-    } else {
-        core = sq;
-    }
-    const T coeff = (dot(r0, r1) * r2n - dot(r0, r2) * r1n) / (BS<T>::fourpi * core * r1n * r2n);
-    return coeff * cr;
-}
-
-// Segment + its image across y = 0 (kernel_symmetry, kernels.ispc:91-102).
-template <typename T, bool SIGMA>
-__device__ __forceinline__ void symmetry_exact(v3<T>& inf, const v3<T>& c, const v3<T>& a, const v3<T>& b, T sigma) {
-    const v3<T> s = segment_exact<T, SIGMA>(c, a, b, sigma);
-    inf.x += s.x;
-    inf.y += s.y;
-    inf.z += s.z;
-    const v3<T> cm = {c.x, -c.y, c.z};
-    const v3<T> t = segment_exact<T, SIGMA>(cm, a, b, sigma);
-    inf.x += t.x;
-    inf.y -= t.y;
-    inf.z += t.z;
-}
-
-// Unit vortex ring v0->v1->v2->v3->v0 with images (kernel_influence body, kernels.ispc:127-133).
-template <typename T, bool SIGMA>
-__device__ __forceinline__ v3<T> ring_exact(const v3<T>& c, const v3<T>& v0, const v3<T>& v1, const v3<T>& v2,
-                                            const v3<T>& v3_, T sigma) {
-    v3<T> inf = {T(0), T(0), T(0)};
-    symmetry_exact<T, SIGMA>(inf, c, v0, v1, sigma);
-    symmetry_exact<T, SIGMA>(inf, c, v1, v2, sigma);
-    symmetry_exact<T, SIGMA>(inf, c, v2, v3_, sigma);
-    symmetry_exact<T, SIGMA>(inf, c, v3_, v0, sigma);
-    return inf;
-}
-
 // ---- panel metrics (vlm_backend_cpu.cpp:391-433, vlm_backend_cpud.cpp:258-300) -----------------
 // Normal normalize((v3-v1) x (v2-v0)); area 0.5(|f x b| + |b x e|); collocation point
 // 0.5(v0+v1) + k * 0.5(v2+v3-v0-v1), k = 1/2 below EPS_f else alpha / (2 (sin alpha + EPS_f)).
@@ -209,44 +158,6 @@ __device__ __forceinline__ T displace_row(const T* M, int64_t m0, int64_t m1, in
     return s;
 }
 
-// ---- FP32 fast form ---------------------------------------------------------------------------
-// Same mathematics with the hardware reciprocal square root: coeff = (d1/|r1| - d2/|r2|) / (4 pi sq),
-// which equals the reference's (d1 |r2| - d2 |r1|) / (4 pi sq |r1| |r2|).  Cutoffs are tested on
-// squared norms: |r| < 1e-5  <=>  |r|^2 < 1e-10, and sq < 1e-10 as in the reference.  Each ring
-// vertex difference and its rsqrt is computed once and shared by the two segments that meet there.
-struct FastVertex {
-    float x, y, z, r2, rinv;  // c - v, |c - v|^2, 1/|c - v|
-};
-
-__device__ __forceinline__ FastVertex fast_vertex(float cx, float cy, float cz, float vx, float vy, float vz) {
-    FastVertex f;
-    f.x = cx - vx;
-    f.y = cy - vy;
-    f.z = cz - vz;
-    f.r2 = f.x * f.x + f.y * f.y + f.z * f.z;
-    f.rinv = __builtin_amdgcn_rsqf(f.r2);
-    return f;
-}
-
-// Accumulates s * (velocity of segment a->b) into acc; s = +1 / -1 mixes the y image sign.
-__device__ __forceinline__ void fast_segment(float& ax, float& ay, float& az, const FastVertex& r1, const FastVertex& r2,
-                                             float sy) {
-    const float crx = r1.y * r2.z - r1.z * r2.y;
-    const float cry = r1.z * r2.x - r1.x * r2.z;
-    const float crz = r1.x * r2.y - r1.y * r2.x;
-    const float sq = crx * crx + cry * cry + crz * crz;
-    // r0 = b - a = r1 - r2 (as points: (c-a) - (c-b))
-    const float r0x = r1.x - r2.x, r0y = r1.y - r2.y, r0z = r1.z - r2.z;
-    const float d1 = r0x * r1.x + r0y * r1.y + r0z * r1.z;
-    const float d2 = r0x * r2.x + r0y * r2.y + r0z * r2.z;
-    const bool ok = (sq >= 1e-10f) & (r1.r2 >= 1e-10f) & (r2.r2 >= 1e-10f);
-    const float t = (d1 * r1.rinv - d2 * r2.rinv) * __builtin_amdgcn_rcpf(BS<float>::fourpi * sq);
-    const float coeff = ok ? t : 0.0f;
-    ax += coeff * crx;
-    ay += sy * (coeff * cry);
-    az += coeff * crz;
-}
-
 // ---- FP64 seeded form ---------------------------------------------------------------------------
 // FP64 arithmetic throughout, but 1/sqrt and 1/x from the hardware estimates (v_rsq_f64,
 // v_rcp_f64) refined by one Newton step in FP64 instead of the multi-instruction correctly rounded
@@ -260,92 +171,6 @@ __device__ __forceinline__ double rsqrt_seeded(double x) {
 __device__ __forceinline__ double rcp_seeded(double x) {
     const double y = __builtin_amdgcn_rcp(x);  // v_rcp_f64 estimate
     return y * (2.0 - x * y);
-}
-
-struct SeedVertex {
-    double x, y, z, r2, rinv;
-};
-
-__device__ __forceinline__ SeedVertex seed_vertex(double cx, double cy, double cz, double vx, double vy, double vz) {
-    SeedVertex f;
-    f.x = cx - vx;
-    f.y = cy - vy;
-    f.z = cz - vz;
-    f.r2 = f.x * f.x + f.y * f.y + f.z * f.z;
-    f.rinv = rsqrt_seeded(f.r2);
-    return f;
-}
-
-__device__ __forceinline__ void seed_segment(double& ax, double& ay, double& az, const SeedVertex& r1,
-                                             const SeedVertex& r2, double sy) {
-    const double crx = r1.y * r2.z - r1.z * r2.y;
-    const double cry = r1.z * r2.x - r1.x * r2.z;
-    const double crz = r1.x * r2.y - r1.y * r2.x;
-    const double sq = crx * crx + cry * cry + crz * crz;
-    const double r0x = r1.x - r2.x, r0y = r1.y - r2.y, r0z = r1.z - r2.z;
-    const double d1 = r0x * r1.x + r0y * r1.y + r0z * r1.z;
-    const double d2 = r0x * r2.x + r0y * r2.y + r0z * r2.z;
-    constexpr double cut2 = BS<double>::cut_norm * BS<double>::cut_norm;
-    const bool ok = (sq >= BS<double>::cut_cross) & (r1.r2 >= cut2) & (r2.r2 >= cut2);
-    const double t = (d1 * r1.rinv - d2 * r2.rinv) * rcp_seeded(BS<double>::fourpi * sq);
-    const double coeff = ok ? t : 0.0;
-    ax += coeff * crx;
-    ay += sy * (coeff * cry);
-    az += coeff * crz;
-}
-
-// Segment a->b of strength g (r1 = c - a, r2 = c - b), accumulated with image sign sy on y.
-__device__ __forceinline__ void seed_segment_w(double& ax, double& ay, double& az, const SeedVertex& r1,
-                                               const SeedVertex& r2, double sy, double g) {
-    const double crx = r1.y * r2.z - r1.z * r2.y;
-    const double cry = r1.z * r2.x - r1.x * r2.z;
-    const double crz = r1.x * r2.y - r1.y * r2.x;
-    const double sq = crx * crx + cry * cry + crz * crz;
-    const double r0x = r1.x - r2.x, r0y = r1.y - r2.y, r0z = r1.z - r2.z;
-    const double d1 = r0x * r1.x + r0y * r1.y + r0z * r1.z;
-    const double d2 = r0x * r2.x + r0y * r2.y + r0z * r2.z;
-    constexpr double cut2 = BS<double>::cut_norm * BS<double>::cut_norm;
-    const bool ok = (sq >= BS<double>::cut_cross) & (r1.r2 >= cut2) & (r2.r2 >= cut2);
-    const double t = (d1 * r1.rinv - d2 * r2.rinv) * rcp_seeded(BS<double>::fourpi * sq) * g;
-    const double coeff = ok ? t : 0.0;
-    ax += coeff * crx;
-    ay += sy * (coeff * cry);
-    az += coeff * crz;
-}
-
-__device__ __forceinline__ void seed_ring(double& ax, double& ay, double& az, double cx, double cy, double cz,
-                                          const double* v0, const double* v1, const double* v2, const double* v3) {
-#pragma unroll
-    for (int m = 0; m < 2; m++) {
-        const double y = m == 0 ? cy : -cy;
-        const double sy = m == 0 ? 1.0 : -1.0;
-        const SeedVertex a = seed_vertex(cx, y, cz, v0[0], v0[1], v0[2]);
-        const SeedVertex b = seed_vertex(cx, y, cz, v1[0], v1[1], v1[2]);
-        const SeedVertex c = seed_vertex(cx, y, cz, v2[0], v2[1], v2[2]);
-        const SeedVertex d = seed_vertex(cx, y, cz, v3[0], v3[1], v3[2]);
-        seed_segment(ax, ay, az, a, b, sy);
-        seed_segment(ax, ay, az, b, c, sy);
-        seed_segment(ax, ay, az, c, d, sy);
-        seed_segment(ax, ay, az, d, a, sy);
-    }
-}
-
-// Ring with image; vertices given as coordinates.
-__device__ __forceinline__ void fast_ring(float& ax, float& ay, float& az, float cx, float cy, float cz, const float* v0,
-                                          const float* v1, const float* v2, const float* v3) {
-#pragma unroll
-    for (int m = 0; m < 2; m++) {
-        const float y = m == 0 ? cy : -cy;
-        const float sy = m == 0 ? 1.0f : -1.0f;
-        const FastVertex a = fast_vertex(cx, y, cz, v0[0], v0[1], v0[2]);
-        const FastVertex b = fast_vertex(cx, y, cz, v1[0], v1[1], v1[2]);
-        const FastVertex c = fast_vertex(cx, y, cz, v2[0], v2[1], v2[2]);
-        const FastVertex d = fast_vertex(cx, y, cz, v3[0], v3[1], v3[2]);
-        fast_segment(ax, ay, az, a, b, sy);
-        fast_segment(ax, ay, az, b, c, sy);
-        fast_segment(ax, ay, az, c, d, sy);
-        fast_segment(ax, ay, az, d, a, sy);
-    }
 }
 
 }  // namespace tvlm

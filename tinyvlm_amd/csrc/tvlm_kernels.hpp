@@ -1,13 +1,14 @@
 // tvlm_kernels.hpp -- Biot-Savart assembly kernels shared by the Backend entry points and the
 // device-resident solver loops.
 //
-// lhs block: a work-group owns 64 receivers (one per lane, colloc + normal in registers) and TC
-// rings whose 12 vertex coordinates are staged in LDS; its 4 waves take every 4th ring, so each
-// wave reads LDS as a broadcast and writes one coalesced 64-element column segment per ring.
+// lhs block: a work-group owns 64 receivers (one per lane, colloc + normal in registers) and a tile of
+// rings (a few chordwise rows x some spans) whose vertices are staged in LDS; its 4 waves split the
+// spans and walk them column by column, every segment and vertex of the tile once, reading LDS as a
+// broadcast and writing one coalesced 64-element column segment per ring.
 //
-// wake partials: the wake rings are cut into tiles of RH rows x SW spans; a work-group stages one
-// tile's vertex rows and circulations in LDS, each wave takes every 4th ring of the tile for the
-// work-group's 64 receivers, and the 4 waves reduce in LDS to one partial per (tile, receiver).
+// wake partials: the wake rings are cut into tiles of rows x spans; a work-group stages one tile's vertex
+// rows and circulations in LDS, each wave walks a quarter of its spans for the work-group's 64
+// receivers, and the 4 waves reduce in LDS to one partial per (tile, receiver).
 // k_wake_reduce then sums the partials of all tiles in a fixed order (bitwise reproducible).
 #pragma once
 
@@ -40,90 +41,231 @@ struct Receivers {
     int32_t m;        // number of receivers (panels)
 };
 
-// Velocity of the ring (v0, v1, v2, v3) with image at c in the form selected by MODE:
-// 0 exact (sigma = 0), 1 exact with core, 2 FP32 rsqrt form, 3 FP64 seeded form.
+// One straight segment a -> b for the receiver and its mirror image in y = 0, in the form selected by
+// MODE: 0 exact (sigma = 0), 1 exact with core, 2 FP32 rsqrt form, 3 FP64 seeded form.  The velocity is
+// k (crx, cry, crz) + km (mrx, -cry, mrz); both images share the y part of r1 x r2.  Vertex<> holds the
+// receiver-relative terms of a vertex, so that the segments meeting there share them, and a ring of
+// a lattice shares its segments with its neighbours: per ring about 2.25 segments and 1.25 vertices
+// instead of 4 and 4, every term as in the reference (kernels.ispc:69-102, :382-415).  Contraction is
+// spelled out: a segment's value must not depend on the kernel it is compiled into (the matrices of a
+// grouped launch equal the single ones bit for bit).
 template <typename T, int MODE>
-__device__ __forceinline__ v3<T> ring_vel(const v3<T>& c, const T* v0, const T* v1, const T* v2, const T* v3_,
-                                          T sigma) {
-    if constexpr (MODE == 2) {
-        float ax = 0.f, ay = 0.f, az = 0.f;
-        fast_ring(ax, ay, az, c.x, c.y, c.z, v0, v1, v2, v3_);
-        return {ax, ay, az};
-    } else if constexpr (MODE == 3) {
-        double ax = 0.0, ay = 0.0, az = 0.0;
-        seed_ring(ax, ay, az, c.x, c.y, c.z, v0, v1, v2, v3_);
-        return {ax, ay, az};
-    } else {
-        return ring_exact<T, MODE == 1>(c, {v0[0], v0[1], v0[2]}, {v1[0], v1[1], v1[2]}, {v2[0], v2[1], v2[2]},
-                                        {v3_[0], v3_[1], v3_[2]}, sigma);
+struct SegForm {
+    struct Vertex {
+        T x, y, z, ym;  // c - v, y of the image receiver
+        T n, nm;        // MODE 0, 1: |c - v| and the image's; 2, 3: their reciprocals
+    };
+    struct Seg {
+        T k, km, crx, cry, crz, mrx, mrz;
+    };
+    static __device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+    static __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+    // whether a vertex of this n lies outside the cutoff radius
+    static __device__ __forceinline__ bool clear(T n) {
+        if constexpr (MODE <= 1)
+            return !(n < BS<T>::cut_norm);
+        else
+            return n <= T(1) / BS<T>::cut_norm;
+    }
+    static __device__ __forceinline__ Vertex vertex(const v3<T>& c, const T* v) {
+#pragma clang fp contract(off)
+        Vertex f;
+        f.x = c.x - v[0];
+        f.y = c.y - v[1];
+        f.z = c.z - v[2];
+        f.ym = -c.y - v[1];
+        const T xz = fma_(f.z, f.z, f.x * f.x);
+        const T r2 = fma_(f.y, f.y, xz), r2m = fma_(f.ym, f.ym, xz);
+        if constexpr (MODE <= 1) {
+            f.n = sqrt(r2);
+            f.nm = sqrt(r2m);
+        } else {
+            if constexpr (MODE == 2) {
+                f.n = __builtin_amdgcn_rsqf(r2);
+                f.nm = __builtin_amdgcn_rsqf(r2m);
+            } else {
+                f.n = rsqrt_seeded(r2);
+                f.nm = rsqrt_seeded(r2m);
+            }
+        }
+        return f;
+    }
+    // r0 = b - a
+    static __device__ __forceinline__ Seg segment(const Vertex& a, const Vertex& b, const v3<T>& r0, T sigma) {
+#pragma clang fp contract(off)
+        Seg s;
+        s.cry = fma_(a.z, b.x, -(a.x * b.z));
+        s.crx = fma_(a.y, b.z, -(a.z * b.y));
+        s.crz = fma_(a.x, b.y, -(a.y * b.x));
+        s.mrx = fma_(a.ym, b.z, -(a.z * b.ym));
+        s.mrz = fma_(a.x, b.ym, -(a.ym * b.x));
+        const T cry2 = s.cry * s.cry;
+        const T sq = fma_(s.crx, s.crx, fma_(s.crz, s.crz, cry2)), sqm = fma_(s.mrx, s.mrx, fma_(s.mrz, s.mrz, cry2));
+        const T d1xz = fma_(r0.z, a.z, r0.x * a.x), d2xz = fma_(r0.z, b.z, r0.x * b.x);
+        const T d1 = fma_(r0.y, a.y, d1xz), d2 = fma_(r0.y, b.y, d2xz);
+        const T d1m = fma_(r0.y, a.ym, d1xz), d2m = fma_(r0.y, b.ym, d2xz);
+        const bool ok = clear(a.n) & clear(b.n), okm = clear(a.nm) & clear(b.nm);
+        if constexpr (MODE <= 1) {
+            T core = sq, corem = sqm;
+            if constexpr (MODE == 1) {
+                const T sm = sigma * sigma * fma_(r0.z, r0.z, fma_(r0.y, r0.y, r0.x * r0.x));
+                core = sqrt(fma_(sm, sm, sq * sq));
+                corem = sqrt(fma_(sm, sm, sqm * sqm));
+            }
+            const T k = fma_(d1, b.n, -(d2 * a.n)) / (BS<T>::fourpi * core * a.n * b.n);
+            const T km = fma_(d1m, b.nm, -(d2m * a.nm)) / (BS<T>::fourpi * corem * a.nm * b.nm);
+            s.k = (ok & !(sq < BS<T>::cut_cross)) ? k : T(0);
+            s.km = (okm & !(sqm < BS<T>::cut_cross)) ? km : T(0);
+        } else {
+            T i, im;
+            if constexpr (MODE == 2) {
+                i = __builtin_amdgcn_rcpf(BS<T>::fourpi * sq);
+                im = __builtin_amdgcn_rcpf(BS<T>::fourpi * sqm);
+            } else {
+                i = rcp_seeded(BS<T>::fourpi * sq);
+                im = rcp_seeded(BS<T>::fourpi * sqm);
+            }
+            s.k = (ok & (sq >= BS<T>::cut_cross)) ? fma_(d1, a.n, -(d2 * b.n)) * i : T(0);
+            s.km = (okm & (sqm >= BS<T>::cut_cross)) ? fma_(d1m, a.nm, -(d2m * b.nm)) * im : T(0);
+        }
+        return s;
+    }
+    static __device__ __forceinline__ Seg segment(const Vertex& a, const Vertex& b, const T* va, const T* vb, T sigma) {
+        return segment(a, b, v3<T>{vb[0] - va[0], vb[1] - va[1], vb[2] - va[2]}, sigma);
+    }
+    static __device__ __forceinline__ T dot_normal(const Seg& s, const v3<T>& n) {
+#pragma clang fp contract(off)
+        const T yn = s.cry * n.y;
+        return fma_(s.k, fma_(s.crz, n.z, fma_(s.crx, n.x, yn)), s.km * fma_(s.mrz, n.z, fma_(s.mrx, n.x, -yn)));
+    }
+};
+
+constexpr int kLhsSpans = 16;  // most spans of one wave in an lhs tile
+
+// Shape of the lhs tiles of a (receiver surface, ring surface) pair: rh ring rows and spans per wave,
+// the largest that still gives about four work-groups per CU (a tile shares the segments inside it; a
+// small matrix needs the waves more).  It depends on the section alone, and a ring's value does not depend
+// on the shape.
+inline void lhs_tile_shape(int m, int ns, int nc, int& rh, int& spans) {
+    constexpr int shapes[][2] = {{4, 16}, {4, 8}, {4, 4}, {2, 4}, {2, 2}, {1, 2}, {1, 1}};
+    for (const auto& sh : shapes) {
+        rh = sh[0];
+        spans = sh[1];
+        const int64_t groups =
+            (int64_t)((m + kRecv - 1) / kRecv) * ((ns + kWaves * spans - 1) / (kWaves * spans)) * ((nc + rh - 1) / rh);
+        if (groups >= 1024) return;
     }
 }
 
-// Loads ring r's vertices (v0, v1 = +1 span, v2 = +1 span +1 chord, v3 = +1 chord) from a vertex
-// grid whose row (chordwise) stride is ns+1.
-template <typename T>
-__device__ __forceinline__ void load_ring(T* dst, const T* grid, int64_t s2, int64_t base, int32_t ns) {
-    const int64_t off[4] = {base, base + 1, base + ns + 2, base + ns + 1};
+// Adds the normal velocity of the lattice's unit rings over one wave's spans [sa, sb) of a staged tile
+// (vertex rows 0..rhe, vw columns) to out: ring (q, s) at out[s ld + q lq], or with SUM the rows' rings one
+// after another to out[s ld].  A column's old values are read before its rings are computed.
+template <typename T, int RH, int MODE, bool SUM>
+__device__ __forceinline__ void lhs_walk(const T* sv, int vw, int rhe, int sa, int sb, const v3<T>& c, const v3<T>& n,
+                                         T sigma, T* __restrict__ out, int64_t ld, int64_t lq) {
+    using S = SegForm<T, MODE>;
+    constexpr int NO = SUM ? 1 : RH;
+    typename S::Vertex prev[RH + 1];
+    T left[RH];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        dst[3 * q + 0] = grid[off[q]];
-        dst[3 * q + 1] = grid[off[q] + s2];
-        dst[3 * q + 2] = grid[off[q] + 2 * s2];
+    for (int q = 0; q <= RH; q++)
+        if (q <= rhe) prev[q] = S::vertex(c, sv + 3 * (q * vw + sa));
+#pragma unroll
+    for (int q = 0; q < RH; q++)
+        if (q < rhe)
+            left[q] = S::dot_normal(
+                S::segment(prev[q], prev[q + 1], sv + 3 * (q * vw + sa), sv + 3 * ((q + 1) * vw + sa), sigma), n);
+#pragma unroll 1
+    for (int s = sa; s < sb; s++) {
+        T* o = out + s * ld;
+        T old[NO];
+#pragma unroll
+        for (int q = 0; q < NO; q++)
+            if (q < rhe) old[q] = o[q * lq];
+        T above = T(0);  // spanwise segment of vertex row q
+        typename S::Vertex up{};  // vertex (q, s + 1)
+#pragma unroll
+        for (int q = 0; q <= RH; q++) {
+            if (q <= rhe) {
+                const T *va = sv + 3 * (q * vw + s), *vb = va + 3;
+                const typename S::Vertex cur = S::vertex(c, vb);
+                const T span = S::dot_normal(S::segment(prev[q], cur, va, vb, sigma), n);
+                if (q > 0) {
+                    const T right = S::dot_normal(S::segment(up, cur, vb - 3 * vw, vb, sigma), n);
+                    const T ring = ((above + right) - span) - left[q > 0 ? q - 1 : 0];
+                    left[q > 0 ? q - 1 : 0] = right;
+                    if constexpr (SUM)
+                        old[0] += ring;
+                    else
+                        o[(q - 1) * lq] = old[q > 0 ? q - 1 : 0] + ring;
+                }
+                above = span;
+                up = cur;
+                prev[q] = cur;
+            }
+        }
+        if constexpr (SUM) o[0] = old[0];
     }
 }
 
 // One tile of the lhs block of a (receiver surface, ring surface) pair: receivers [bx kRecv, +kRecv)
-// x rings [by TC, +TC).  lhs points at (offset_i, offset_j).  Every thread of the work-group calls it
-// (it holds a barrier); sv is the caller's LDS staging of TC rings.
-template <typename T, int TC, int MODE>  // MODE as ring_vel
-__device__ __forceinline__ void lhs_tile(T (*sv)[12], T* __restrict__ lhs, int64_t ld, const Receivers<T>& rc,
-                                         const RingSource<T>& src, T sigma, int bx, int by) {
-    const int n_rings = src.ns * src.nc;
-    const int col0 = by * TC;
-    for (int e = threadIdx.x; e < TC * 4; e += kThreads) {
-        const int r = e >> 2, q = e & 3;
-        const int lidx = col0 + r;
-        if (lidx < n_rings) {
-            const int64_t base = lidx + lidx / src.ns;  // vertex 0 of ring lidx (vlm_backend_cpu.cpp:111)
-            const int64_t off = q == 0 ? base : q == 1 ? base + 1 : q == 2 ? base + src.ns + 2 : base + src.ns + 1;
-            sv[r][3 * q + 0] = src.verts[off];
-            sv[r][3 * q + 1] = src.verts[off + src.vs2];
-            sv[r][3 * q + 2] = src.verts[off + 2 * src.vs2];
+// x rings of RH rows and kWaves * spans spans.  lhs points at (offset_i, offset_j).  Every thread of the
+// work-group calls it (it holds barriers); sv is the caller's LDS staging.
+// Bound by VALU issue (exact FP64: two IEEE divisions per segment and image pair).  Ring by ring -> shared
+// segments: 16 x 16 wing exact FP64 19.8 -> 12.9 us for a call with its fill (32 -> 256 work-groups), elliptic
+// 64 x 64 FP32 113.5 -> 79.5 us, the served batch of 32 of them 60.5 -> 52.2 ms.
+template <typename T, int RH, int MODE>  // MODE as SegForm
+__device__ __forceinline__ void lhs_tile(T* sv, T* __restrict__ lhs, int64_t ld, const Receivers<T>& rc,
+                                         const RingSource<T>& src, T sigma, int bx, int by, int spans) {
+    const int ns = src.ns, sw = kWaves * spans, tiles_span = (ns + sw - 1) / sw;
+    const int s0 = (by % tiles_span) * sw, r0 = (by / tiles_span) * RH;
+    const int swe = min(sw, ns - s0), rhe = min(RH, src.nc - r0), vw = swe + 1;
+    auto stage = [&](const T* grid, int64_t s2, int row, int rows) {  // vertex rows row .. row + rows
+        for (int e = threadIdx.x; e < (rows + 1) * vw; e += kThreads) {
+            const T* g = grid + (int64_t)(row + e / vw) * (ns + 1) + s0 + e % vw;
+            sv[3 * e + 0] = g[0];
+            sv[3 * e + 1] = g[s2];
+            sv[3 * e + 2] = g[2 * s2];
         }
-    }
+    };
+    stage(src.verts, src.vs2, r0, rhe);
     __syncthreads();
     const int lane = threadIdx.x & (kRecv - 1);
-    const int wave = threadIdx.x / kRecv;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kRecv);
     const int i = bx * kRecv + lane;
-    if (i >= rc.m) return;
-    const v3<T> c = {rc.colloc[i], rc.colloc[i + rc.cs2], rc.colloc[i + 2 * rc.cs2]};
-    const v3<T> n = {rc.normals[i], rc.normals[i + rc.ns2], rc.normals[i + 2 * rc.ns2]};
-    const int ncols = min(TC, n_rings - col0);
-    const int te0 = (src.nc - 1) * src.ns;
-    for (int r = wave; r < ncols; r += kWaves) {
-        const int lidx = col0 + r;
-        T* dst = lhs + i + (int64_t)lidx * ld;
-        T acc = *dst;
-        acc += dot(ring_vel<T, MODE>(c, sv[r], sv[r] + 3, sv[r] + 6, sv[r] + 9, sigma), n);
-        if (src.iteration > 0 && lidx >= te0) {
-            // trailing-edge column: wake rings of rows nwv-2-k, k < iteration (vlm_backend_cpu.cpp:121-139)
-            const int j = lidx - te0;
-            for (int k = 0; k < src.iteration; k++) {
-                T w[12];
-                load_ring(w, src.wake, src.ws2, (int64_t)j + (int64_t)(src.nwv - 2 - k) * (src.ns + 1), src.ns);
-                acc += dot(ring_vel<T, MODE>(c, w, w + 3, w + 6, w + 9, sigma), n);
-            }
-        }
-        *dst = acc;
+    const bool mine = i < rc.m;
+    v3<T> c{}, n{};
+    if (mine) {
+        c = {rc.colloc[i], rc.colloc[i + rc.cs2], rc.colloc[i + 2 * rc.cs2]};
+        n = {rc.normals[i], rc.normals[i + rc.ns2], rc.normals[i + 2 * rc.ns2]};
+    }
+    const int sa = wave * spans, sb = min(swe, sa + spans);
+    T* out = lhs + i + (int64_t)s0 * ld;
+    if (mine && sa < sb)
+        lhs_walk<T, RH, MODE, false>(sv, vw, rhe, sa, sb, c, n, sigma, out + (int64_t)r0 * ns * ld, ld, ns * ld);
+    if (src.iteration <= 0 || r0 + rhe < src.nc) return;
+    // trailing-edge columns: wake rings of rows nwv-2-k, k < iteration (vlm_backend_cpu.cpp:121-139)
+    for (int row = src.nwv - 1 - src.iteration; row < src.nwv - 1; row += RH) {
+        const int rows = min(RH, src.nwv - 1 - row);
+        __syncthreads();
+        stage(src.wake, src.ws2, row, rows);
+        __syncthreads();
+        if (mine && sa < sb)
+            lhs_walk<T, RH, MODE, true>(sv, vw, rows, sa, sb, c, n, sigma, out + (int64_t)(src.nc - 1) * ns * ld, ld, 0);
     }
 }
 
+template <int RH>
+constexpr int lhs_stage_values() {
+    return 3 * (RH + 1) * (kWaves * kLhsSpans + 1);
+}
+
 // lhs block of one (receiver surface, ring surface) pair, one tile per work-group.
-template <typename T, int TC, int MODE>  // MODE as ring_vel
-__global__ __launch_bounds__(kThreads) void k_lhs_block(T* __restrict__ lhs, int64_t ld, Receivers<T> rc,
-                                                        RingSource<T> src, T sigma) {
-    __shared__ T sv[TC][12];
-    lhs_tile<T, TC, MODE>(sv, lhs, ld, rc, src, sigma, blockIdx.x, blockIdx.y);
+template <typename T, int RH, int MODE>  // MODE as SegForm
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 1))) void k_lhs_block(T* __restrict__ lhs, int64_t ld, Receivers<T> rc,
+                                                        RingSource<T> src, T sigma, int spans) {
+    __shared__ T sv[lhs_stage_values<RH>()];
+    lhs_tile<T, RH, MODE>(sv, lhs, ld, rc, src, sigma, blockIdx.x, blockIdx.y, spans);
 }
 
 // One (receiver surface, ring surface) block of one influence matrix in a grouped launch: the tiles
@@ -136,7 +278,14 @@ struct LhsSection {
     Receivers<T> rc;
     RingSource<T> src;
     int32_t tiles_x, tile0;
+    int32_t rh, spans;  // tile shape (lhs_tile_shape)
 };
+
+template <typename T>
+inline int64_t lhs_tiles_y(const LhsSection<T>& s) {
+    const int sw = kWaves * s.spans;
+    return (int64_t)((s.src.ns + sw - 1) / sw) * ((s.src.nc + s.rh - 1) / s.rh);
+}
 
 // A value every lane of the wave holds alike, moved to a scalar register (the section fields the
 // grouped kernel reads from LDS would otherwise sit in vector registers and cost it occupancy).
@@ -170,6 +319,8 @@ __device__ __forceinline__ LhsSection<T> wave_uniform(const LhsSection<T>& a) {
     b.src.iteration = wave_uniform(a.src.iteration);
     b.tiles_x = wave_uniform(a.tiles_x);
     b.tile0 = wave_uniform(a.tile0);
+    b.rh = wave_uniform(a.rh);
+    b.spans = wave_uniform(a.spans);
     return b;
 }
 
@@ -182,11 +333,11 @@ __device__ __forceinline__ LhsSection<T> wave_uniform(const LhsSection<T>& a) {
 // tile runs lhs_tile, so each matrix is bitwise the per-section launches' result.
 constexpr int kGroupChunk = 64;
 
-template <typename T, int TC, int MODE>
+template <typename T, int MODE>
 __global__ __launch_bounds__(kThreads) void k_lhs_grouped(const LhsSection<T>* __restrict__ secs,
                                                           const int32_t* __restrict__ tile0,
                                                           const int32_t* __restrict__ chunk, int tiles, T sigma) {
-    __shared__ T sv[TC][12];
+    __shared__ T sv[lhs_stage_values<4>()];
     __shared__ LhsSection<T> s_sec;
     const int t = blockIdx.x;
     if (t >= tiles) return;
@@ -198,7 +349,13 @@ __global__ __launch_bounds__(kThreads) void k_lhs_grouped(const LhsSection<T>* _
     __syncthreads();
     const LhsSection<T> S = wave_uniform(s_sec);
     const int local = t - S.tile0;
-    lhs_tile<T, TC, MODE>(sv, S.lhs, S.ld, S.rc, S.src, sigma, local % S.tiles_x, local / S.tiles_x);
+    const int bx = local % S.tiles_x, by = local / S.tiles_x;
+    if (S.rh == 4)
+        lhs_tile<T, 4, MODE>(sv, S.lhs, S.ld, S.rc, S.src, sigma, bx, by, S.spans);
+    else if (S.rh == 2)
+        lhs_tile<T, 2, MODE>(sv, S.lhs, S.ld, S.rc, S.src, sigma, bx, by, S.spans);
+    else
+        lhs_tile<T, 1, MODE>(sv, S.lhs, S.ld, S.rc, S.src, sigma, bx, by, S.spans);
 }
 
 // ---- wake influence ---------------------------------------------------------------------------
@@ -245,9 +402,57 @@ __device__ __forceinline__ int find_surface(const RecvTable<T>& t, int p) {
     return s;
 }
 
-// TS: storage type of the inputs and partials, T: compute type (float for MODE 2, double for MODE 3)
-template <typename TS, typename T, int MODE>
-__global__ __launch_bounds__(kThreads) void k_wake_partials(TS* __restrict__ partial, RecvTable<TS> rt,
+// Velocity of the tile's rings with their circulations over one wave's spans [sa, sb), RH rows at a time
+// from row q0 on: every segment once with the difference of the circulations beside it (rings outside
+// the RH rows, or outside the wave's spans on their far side, add theirs where they are walked).
+template <typename T, int RH, int MODE>
+__device__ __forceinline__ void wake_walk(const T* sv, const T* sg, int vw, int swe, int rhe, int sa, int sb,
+                                          const v3<T>& c, T sigma, v3<T>& acc) {
+    using S = SegForm<T, MODE>;
+    auto add = [&](const typename S::Seg& s, T g) {
+        const T k = g * s.k, km = g * s.km;
+        acc.x += k * s.crx + km * s.mrx;
+        acc.y += (k - km) * s.cry;
+        acc.z += k * s.crz + km * s.mrz;
+    };
+    typename S::Vertex prev[RH + 1];
+#pragma unroll
+    for (int q = 0; q <= RH; q++)
+        if (q <= rhe) prev[q] = S::vertex(c, sv + 3 * (q * vw + sa));
+#pragma unroll 1
+    for (int s = sa; s <= sb; s++) {
+        // chordwise segments of vertex column s (the tile's right edge with the last span's wave)
+        if (s < sb || sb == swe) {
+#pragma unroll
+            for (int q = 0; q < RH; q++) {
+                if (q < rhe) {
+                    const T* va = sv + 3 * (q * vw + s);
+                    T g = s < swe ? -sg[q * swe + s] : T(0);
+                    if (s > 0) g += sg[q * swe + s - 1];
+                    add(S::segment(prev[q], prev[q + 1], va, va + 3 * vw, sigma), g);
+                }
+            }
+        }
+        if (s == sb) break;
+#pragma unroll
+        for (int q = 0; q <= RH; q++) {
+            if (q <= rhe) {
+                const T* va = sv + 3 * (q * vw + s);
+                const typename S::Vertex cur = S::vertex(c, va + 3);
+                T g = q < rhe ? sg[q * swe + s] : T(0);
+                if (q > 0) g -= sg[(q - 1) * swe + s];
+                add(S::segment(prev[q], cur, va, va + 3, sigma), g);
+                prev[q] = cur;
+            }
+        }
+    }
+}
+
+// TS: storage type of the inputs and partials, T: compute type (float for MODE 2).  RH: rows a wave walks
+// at a time (the launch's tiles hold more or fewer, wake_tile_shape).  Bound by VALU issue; a call of 400
+// receivers x 200 x 40 rings in exact FP64 72.3 -> 44.9 us with the shared segments.
+template <typename TS, typename T, int MODE, int RH>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MODE == 1 ? 1 : 4))) void k_wake_partials(TS* __restrict__ partial, RecvTable<TS> rt,
                                                             WakeTable<TS> wt, T sigma) {
     // LDS: vertex rows of the tile (rh+1) x (sw+1) x 3 and circulations rh x sw.  With
     // rh = floor(kTileRings / sw) and 1 <= sw <= kMaxSpanTile, (rh+1)(sw+1) <= 2 (kTileRings+1).
@@ -280,26 +485,22 @@ __global__ __launch_bounds__(kThreads) void k_wake_partials(TS* __restrict__ par
     __syncthreads();
 
     const int lane = threadIdx.x & (kRecv - 1);
-    const int wave = threadIdx.x / kRecv;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kRecv);
     const int p = blockIdx.x * kRecv + lane;
+    const int chunk = (swe + kWaves - 1) / kWaves;
+    const int sa = wave * chunk, sb = min(swe, sa + chunk);
     T part = T(0);
-    if (p < rt.total) {
+    if (p < rt.total && sa < sb) {
         const int si = find_surface(rt, p);
         const Receivers<TS>& rc = rt.r[si];
         const int li = p - rt.offset[si];
         const v3<T> c = {(T)rc.colloc[li], (T)rc.colloc[li + rc.cs2], (T)rc.colloc[li + 2 * rc.cs2]};
         const v3<T> n = {(T)rc.normals[li], (T)rc.normals[li + rc.ns2], (T)rc.normals[li + 2 * rc.ns2]};
         v3<T> acc = {T(0), T(0), T(0)};
-        for (int q = wave; q < rhe * swe; q += kWaves) {
-            const int row = q / swe, sp = q % swe;
-            const T* a = sverts + 3 * (row * vw + sp);
-            const T* d = sverts + 3 * ((row + 1) * vw + sp);
-            const T g = sgam[q];
-            const v3<T> ind = ring_vel<T, MODE>(c, a, a + 3, d + 3, d, sigma);
-            acc.x += ind.x * g;
-            acc.y += ind.y * g;
-            acc.z += ind.z * g;
-        }
+#pragma unroll 1
+        for (int q0 = 0; q0 < rhe; q0 += RH)
+            wake_walk<T, RH, MODE>(sverts + 3 * q0 * vw, sgam + q0 * swe, vw, swe, min(RH, rhe - q0), sa, sb, c, sigma,
+                                   acc);
         part = dot(acc, n);
     }
     sred[wave][lane] = part;
@@ -308,6 +509,20 @@ __global__ __launch_bounds__(kThreads) void k_wake_partials(TS* __restrict__ par
         const T s = (sred[0][lane] + sred[1][lane]) + (sred[2][lane] + sred[3][lane]);
         partial[(int64_t)tile * rt.total + p] = (TS)s;
     }
+}
+
+// k_wake_partials with the rows per walk that the launch's tiles hold (the largest of 4, 2, 1 within them).
+template <typename T, int MODE>
+inline void launch_wake_partials(dim3 grid, hipStream_t st, T* partial, const RecvTable<T>& rt, const WakeTable<T>& wt,
+                                 T sigma) {
+    int rh = 0;
+    for (int m = 0; m < wt.n; m++) rh = wt.s[m].rh > rh ? wt.s[m].rh : rh;
+    if (rh >= 4)
+        hipLaunchKernelGGL((k_wake_partials<T, T, MODE, 4>), grid, dim3(kThreads), 0, st, partial, rt, wt, sigma);
+    else if (rh >= 2)
+        hipLaunchKernelGGL((k_wake_partials<T, T, MODE, 2>), grid, dim3(kThreads), 0, st, partial, rt, wt, sigma);
+    else
+        hipLaunchKernelGGL((k_wake_partials<T, T, MODE, 1>), grid, dim3(kThreads), 0, st, partial, rt, wt, sigma);
 }
 
 // rhs[p] -= sum over tiles of partial[tile][p]: 64 receivers per work-group, 16 waves each sum
@@ -358,15 +573,16 @@ inline void launch_wake_reduce(T* rhs, int64_t rhs_stride, const T* partial, int
 }
 
 // Tile shape of one wake surface: spans per tile sw <= kMaxSpanTile, rows per tile rh with
-// rh * sw <= kTileRings, and small enough that the launch has about wake_target_groups()
-// work-groups (receiver blocks x tiles; default kTargetGroups) so every SIMD holds several waves.
-
+// rh * sw <= kTileRings, as few as give the launch about half of wake_target_groups() work-groups
+// (receiver blocks x tiles).  Half: rows of one tile share the segments between them (400 receivers x 200
+// x 40 rings take two rows and 700 work-groups; one row and 1400 work-groups measured 52 us against
+// 45 us for the whole call).
 inline void wake_tile_shape(int ns, int rows, int recv_blocks, int& sw, int& rh) {
     sw = ns < kMaxSpanTile ? ns : kMaxSpanTile;
     const int tiles_span = (ns + sw - 1) / sw;
     int rh_max = kTileRings / sw;
     if (rh_max < 1) rh_max = 1;
-    int want_row_tiles = wake_target_groups() / (recv_blocks * tiles_span);
+    int want_row_tiles = wake_target_groups() / (2 * recv_blocks * tiles_span);
     if (want_row_tiles < 1) want_row_tiles = 1;
     rh = (rows + want_row_tiles - 1) / want_row_tiles;
     if (rh < 1) rh = 1;

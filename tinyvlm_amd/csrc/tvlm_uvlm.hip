@@ -7,9 +7,8 @@
 //   k_pre    : wake shed of the trailing-edge vertex row, kinematic velocities -(dT [x;1]) at the
 //              t = 0 collocation points, rhs = -(V . n)                        (vlm.cpp:412-438)
 //   wake induction + k_wake_reduce : rhs -= wake induction                    (vlm.cpp:439)
-//              plain mode: k_wake_partials, exact FP64 Biot-Savart ring by ring;
-//              fast mode : k_wake_lattice, every wake segment once with the difference of the
-//              circulations of the two rings it borders
+//              plain mode: k_wake_partials, exact FP64 Biot-Savart, every wake segment once;
+//              fast mode : k_wake_lattice, the same sum in the FP64 seeded form
 //   solve    : plain mode: LU forward/backward substitution (getrs);
 //              fast mode : gamma = A^{-1} rhs with the FP64 inverse formed once from the LU
 //   k_post_advance (one work-group): gamma post-processing, shed of Gamma_TE into the wake,
@@ -739,7 +738,7 @@ int launch_wake(tvlm_uvlm_plan* P, int i, int& tiles) {
             hipLaunchKernelGGL((k_wake_lattice<double, 4>), grid, dim3(kThreads), 0, st, P->wpart, rt, wt, P->zs,
                                P->wzs);
     } else
-        hipLaunchKernelGGL((k_wake_partials<double, double, 0>), grid, dim3(kThreads), 0, st, P->wpart, rt, wt, 0.0);
+        launch_wake_partials<double, 0>(grid, st, P->wpart, rt, wt, 0.0);
     TVLM_LAUNCHED();
     return TVLM_OK;
 }
