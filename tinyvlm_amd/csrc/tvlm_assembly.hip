@@ -296,6 +296,21 @@ struct tvlm_lhs_group {
     std::vector<int64_t> item_tiles;  // tiles of items [0, k): item_tiles[k]
 };
 
+namespace tvlm {
+
+int lhs_group_assign_seeded(tvlm_lhs_group* G, int32_t n_items, const double* base64, float* base32, hipStream_t st) {
+    TVLM_REQUIRE(G && base64 && base32, "null argument");
+    TVLM_REQUIRE(n_items >= 0 && n_items <= G->n_items, "n_items %d of %d", n_items, G->n_items);
+    const int64_t tiles = G->item_tiles[n_items];
+    if (tiles == 0) return TVLM_OK;
+    hipLaunchKernelGGL((k_lhs_grouped<double, 3>), dim3((unsigned)tiles), dim3(kThreads), 0, st, G->secs, G->tile0,
+                       G->chunk, (int)tiles, 0.0, base64, base32);
+    TVLM_LAUNCHED();
+    return TVLM_OK;
+}
+
+}  // namespace tvlm
+
 extern "C" {
 
 int tvlm_lhs_group_create(tvlm_lhs_group** out, int32_t n_items, const tvlm_lhs_item* items, void* stream) {
@@ -357,13 +372,13 @@ int tvlm_lhs_group_assemble_f64(tvlm_lhs_group* G, int32_t n_items, int32_t seed
     const dim3 grid((unsigned)tiles);
     if (sigma != 0.0)
         hipLaunchKernelGGL((k_lhs_grouped<double, 1>), grid, dim3(tvlm::kThreads), 0, st, G->secs, G->tile0,
-                           G->chunk, (int)tiles, sigma);
+                           G->chunk, (int)tiles, sigma, (const double*)nullptr, (float*)nullptr);
     else if (seeded)
         hipLaunchKernelGGL((k_lhs_grouped<double, 3>), grid, dim3(tvlm::kThreads), 0, st, G->secs, G->tile0,
-                           G->chunk, (int)tiles, sigma);
+                           G->chunk, (int)tiles, sigma, (const double*)nullptr, (float*)nullptr);
     else
         hipLaunchKernelGGL((k_lhs_grouped<double, 0>), grid, dim3(tvlm::kThreads), 0, st, G->secs, G->tile0,
-                           G->chunk, (int)tiles, sigma);
+                           G->chunk, (int)tiles, sigma, (const double*)nullptr, (float*)nullptr);
     TVLM_LAUNCHED();
     return TVLM_OK;
 }

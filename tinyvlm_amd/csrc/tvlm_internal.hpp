@@ -88,6 +88,11 @@ int lattice_target_groups();
 int lhs_assemble_seeded_f64(const tvlm_view* lhs, int32_t n_surf, const tvlm_view* colloc, const tvlm_view* normals,
                             const tvlm_view* verts_wing, const tvlm_view* verts_wake, int32_t iteration, void* stream);
 
+// Grouped assembly in the FP64 seeded form that sets the matrices (of the group's first n_items items)
+// instead of adding to them, and stores them rounded to FP32 as well: element k past base64 at base32 + k.
+int lhs_group_assign_seeded(tvlm_lhs_group* group, int32_t n_items, const double* base64, float* base32,
+                            hipStream_t stream);
+
 // ---- small vector type ------------------------------------------------------------------------
 template <typename T>
 struct v3 {

@@ -159,10 +159,12 @@ inline void lhs_tile_shape(int m, int ns, int nc, int& rh, int& spans) {
 
 // Adds the normal velocity of the lattice's unit rings over one wave's spans [sa, sb) of a staged tile
 // (vertex rows 0..rhe, vw columns) to out: ring (q, s) at out[s ld + q lq], or with SUM the rows' rings one
-// after another to out[s ld].  A column's old values are read before its rings are computed.
+// after another to out[s ld].  A column's old values are read before its rings are computed (set: they
+// are 0, except with SUM).  out32, when not null: the same elements rounded to FP32.
 template <typename T, int RH, int MODE, bool SUM>
 __device__ __forceinline__ void lhs_walk(const T* sv, int vw, int rhe, int sa, int sb, const v3<T>& c, const v3<T>& n,
-                                         T sigma, T* __restrict__ out, int64_t ld, int64_t lq) {
+                                         T sigma, T* __restrict__ out, int64_t ld, int64_t lq, bool set,
+                                         float* __restrict__ out32) {
     using S = SegForm<T, MODE>;
     constexpr int NO = SUM ? 1 : RH;
     typename S::Vertex prev[RH + 1];
@@ -181,7 +183,7 @@ __device__ __forceinline__ void lhs_walk(const T* sv, int vw, int rhe, int sa, i
         T old[NO];
 #pragma unroll
         for (int q = 0; q < NO; q++)
-            if (q < rhe) old[q] = o[q * lq];
+            if (q < rhe) old[q] = set && !SUM ? T(0) : o[q * lq];
         T above = T(0);  // spanwise segment of vertex row q
         typename S::Vertex up{};  // vertex (q, s + 1)
 #pragma unroll
@@ -196,15 +198,21 @@ __device__ __forceinline__ void lhs_walk(const T* sv, int vw, int rhe, int sa, i
                     left[q > 0 ? q - 1 : 0] = right;
                     if constexpr (SUM)
                         old[0] += ring;
-                    else
-                        o[(q - 1) * lq] = old[q > 0 ? q - 1 : 0] + ring;
+                    else {
+                        const T v = old[q > 0 ? q - 1 : 0] + ring;
+                        o[(q - 1) * lq] = v;
+                        if (out32) out32[s * ld + (q - 1) * lq] = (float)v;
+                    }
                 }
                 above = span;
                 up = cur;
                 prev[q] = cur;
             }
         }
-        if constexpr (SUM) o[0] = old[0];
+        if constexpr (SUM) {
+            o[0] = old[0];
+            if (out32) out32[s * ld] = (float)old[0];
+        }
     }
 }
 
@@ -213,10 +221,12 @@ __device__ __forceinline__ void lhs_walk(const T* sv, int vw, int rhe, int sa, i
 // work-group calls it (it holds barriers); sv is the caller's LDS staging.
 // Bound by VALU issue (exact FP64: two IEEE divisions per segment and image pair).  Ring by ring -> shared
 // segments: 16 x 16 wing exact FP64 19.8 -> 12.9 us for a call with its fill (32 -> 256 work-groups), elliptic
-// 64 x 64 FP32 113.5 -> 79.5 us, the served batch of 32 of them 60.5 -> 52.2 ms.
+// 64 x 64 FP32 113.5 -> 79.5 us, the served batch of 32 of them 60.5 -> 52.2 ms.  With `set` the elements are
+// stored without a read, and as FP32 too: that batch 52.2 -> 47.6 ms (no fill, no conversion pass).
 template <typename T, int RH, int MODE>  // MODE as SegForm
 __device__ __forceinline__ void lhs_tile(T* sv, T* __restrict__ lhs, int64_t ld, const Receivers<T>& rc,
-                                         const RingSource<T>& src, T sigma, int bx, int by, int spans) {
+                                         const RingSource<T>& src, T sigma, int bx, int by, int spans, bool set = false,
+                                         float* lhs32 = nullptr) {
     const int ns = src.ns, sw = kWaves * spans, tiles_span = (ns + sw - 1) / sw;
     const int s0 = (by % tiles_span) * sw, r0 = (by / tiles_span) * RH;
     const int swe = min(sw, ns - s0), rhe = min(RH, src.nc - r0), vw = swe + 1;
@@ -241,8 +251,10 @@ __device__ __forceinline__ void lhs_tile(T* sv, T* __restrict__ lhs, int64_t ld,
     }
     const int sa = wave * spans, sb = min(swe, sa + spans);
     T* out = lhs + i + (int64_t)s0 * ld;
+    float* out32 = lhs32 ? lhs32 + i + (int64_t)s0 * ld : nullptr;
     if (mine && sa < sb)
-        lhs_walk<T, RH, MODE, false>(sv, vw, rhe, sa, sb, c, n, sigma, out + (int64_t)r0 * ns * ld, ld, ns * ld);
+        lhs_walk<T, RH, MODE, false>(sv, vw, rhe, sa, sb, c, n, sigma, out + (int64_t)r0 * ns * ld, ld, ns * ld, set,
+                                         out32 ? out32 + (int64_t)r0 * ns * ld : nullptr);
     if (src.iteration <= 0 || r0 + rhe < src.nc) return;
     // trailing-edge columns: wake rings of rows nwv-2-k, k < iteration (vlm_backend_cpu.cpp:121-139)
     for (int row = src.nwv - 1 - src.iteration; row < src.nwv - 1; row += RH) {
@@ -251,7 +263,8 @@ __device__ __forceinline__ void lhs_tile(T* sv, T* __restrict__ lhs, int64_t ld,
         stage(src.wake, src.ws2, row, rows);
         __syncthreads();
         if (mine && sa < sb)
-            lhs_walk<T, RH, MODE, true>(sv, vw, rows, sa, sb, c, n, sigma, out + (int64_t)(src.nc - 1) * ns * ld, ld, 0);
+            lhs_walk<T, RH, MODE, true>(sv, vw, rows, sa, sb, c, n, sigma, out + (int64_t)(src.nc - 1) * ns * ld, ld, 0,
+                                        set, out32 ? out32 + (int64_t)(src.nc - 1) * ns * ld : nullptr);
     }
 }
 
@@ -336,7 +349,8 @@ constexpr int kGroupChunk = 64;
 template <typename T, int MODE>
 __global__ __launch_bounds__(kThreads) void k_lhs_grouped(const LhsSection<T>* __restrict__ secs,
                                                           const int32_t* __restrict__ tile0,
-                                                          const int32_t* __restrict__ chunk, int tiles, T sigma) {
+                                                          const int32_t* __restrict__ chunk, int tiles, T sigma,
+                                                          const T* base = nullptr, float* base32 = nullptr) {
     __shared__ T sv[lhs_stage_values<4>()];
     __shared__ LhsSection<T> s_sec;
     const int t = blockIdx.x;
@@ -350,12 +364,13 @@ __global__ __launch_bounds__(kThreads) void k_lhs_grouped(const LhsSection<T>* _
     const LhsSection<T> S = wave_uniform(s_sec);
     const int local = t - S.tile0;
     const int bx = local % S.tiles_x, by = local / S.tiles_x;
+    float* l32 = base32 ? base32 + (S.lhs - base) : nullptr;  // with base32 the matrices are set, not added to
     if (S.rh == 4)
-        lhs_tile<T, 4, MODE>(sv, S.lhs, S.ld, S.rc, S.src, sigma, bx, by, S.spans);
+        lhs_tile<T, 4, MODE>(sv, S.lhs, S.ld, S.rc, S.src, sigma, bx, by, S.spans, base32 != nullptr, l32);
     else if (S.rh == 2)
-        lhs_tile<T, 2, MODE>(sv, S.lhs, S.ld, S.rc, S.src, sigma, bx, by, S.spans);
+        lhs_tile<T, 2, MODE>(sv, S.lhs, S.ld, S.rc, S.src, sigma, bx, by, S.spans, base32 != nullptr, l32);
     else
-        lhs_tile<T, 1, MODE>(sv, S.lhs, S.ld, S.rc, S.src, sigma, bx, by, S.spans);
+        lhs_tile<T, 1, MODE>(sv, S.lhs, S.ld, S.rc, S.src, sigma, bx, by, S.spans, base32 != nullptr, l32);
 }
 
 // ---- wake influence ---------------------------------------------------------------------------

@@ -8,8 +8,8 @@
 // circulation differences, steady forces and per-surface CL/CM.
 //   mode 0 (plain FP64): exact FP64 assembly, FP64 LU and substitution, one request after another;
 //                        this is the reference's arithmetic, operation for operation.
-//   mode 1 (served)    : every request's FP64 influence matrix in the seeded form, copied to FP32,
-//                        one batched FP32 LU for all requests, then FP64 iterative refinement
+//   mode 1 (served)    : every request's FP64 influence matrix in the seeded form, stored rounded to
+//                        FP32 as well, one batched FP32 LU for all requests, then FP64 iterative refinement
 //                        x += A32^{-1} (b - A64 x) (kRefine + 1 corrections, residual in FP64 against
 //                        the FP64 matrix), so the answer carries the FP64 matrix's accuracy.  The
 //                        returned x of every request is checked: ||b - A64 x||_inf <= sqrt(N) eps
@@ -49,7 +49,8 @@ struct tvlm_vlm_plan {
     double *verts[kMaxS] = {}, *wake[kMaxS] = {};                // per request b: + b * vsz / wsz
     double *colloc[kMaxS] = {}, *normals[kMaxS] = {}, *areas[kMaxS] = {};
     double *vel[kMaxS] = {}, *forces[kMaxS] = {}, *gdelta[kMaxS] = {};
-    double *lhs = nullptr, *rhs = nullptr, *x = nullptr, *res = nullptr, *tr = nullptr, *coef = nullptr;
+    double *lhs = nullptr, *rhs = nullptr, *x = nullptr, *res = nullptr, *coef = nullptr;
+    double* par = nullptr;  // per request: 16 n_surf transform values, then kPar values (tvlm_vlm_solve_n)
     float *lhs32 = nullptr, *r32 = nullptr;
     int32_t *ipiv = nullptr, *info = nullptr;
     double *rowabs = nullptr, *berr = nullptr;  // served mode: row sums of |A64|, backward error per request
@@ -57,9 +58,7 @@ struct tvlm_vlm_plan {
     std::vector<int32_t> st_status, st_corr;     // per request of the last solve (tvlm_vlm_refinement)
     std::vector<double> st_berr;
     bool checked = false;                        // the last solve's requests were checked (and rescued)
-    double* tr_host = nullptr;  // pinned: transforms of all requests and surfaces
-    std::vector<double> alpha, beta, ref;  // per request; ref: CM reference point in the moved frame
-    double u_inf = 1.0, rho = 1.0;
+    double* par_host = nullptr;  // pinned copy of par
     bool solved = false;
     tvlm_lhs_group* group = nullptr;  // served mode: every request's influence matrix, one grouped launch
 
@@ -73,6 +72,145 @@ struct tvlm_vlm_plan {
 
 namespace tvlm {
 namespace {
+
+constexpr int kPar = 12;  // alpha, freestream (3), lift axis (3), CM reference point (3), dynamic pressure
+
+struct VSurf {
+    const double* init;
+    double *verts, *wake, *colloc, *normals, *areas, *vel, *forces, *gdelta;
+    int64_t vsz, wsz, psz;  // elements per request: vertices, wake, panels
+    int32_t ns, nc, off;
+};
+
+struct VTab {
+    int32_t n, N, items;  // items: vertices and panels of all surfaces
+    const double* par;
+    double *rhs, *coef;
+    const double* x;
+    VSurf s[kMaxS];
+};
+
+// Geometry and rhs of requests b0 + blockIdx.y (vlm.cpp:97-124): a thread per vertex (the wing moved by
+// the request's transform; its trailing edge before and after is the wake's one ring row) or per
+// panel (metrics at alpha, freestream velocity, rhs = -(V . n)).
+// Bound by the launches, so one for all requests: with a dozen small launches per request before and nine
+// after its solve, 32 requests of 256 panels took 2.33 ms, with this kernel and k_vlm_post 0.77 ms.
+__global__ __launch_bounds__(256) void k_vlm_geom(VTab t, int b0) {
+    const int b = b0 + blockIdx.y;
+    int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= t.items) return;
+    int m = 0;
+    for (; m + 1 < t.n; m++) {
+        const int here = (t.s[m].ns + 1) * (t.s[m].nc + 1) + t.s[m].ns * t.s[m].nc;
+        if (e < here) break;
+        e -= here;
+    }
+    const VSurf& S = t.s[m];
+    const double* par = t.par + (int64_t)b * (16 * t.n + kPar);
+    const double* M = par + 16 * m;
+    par += 16 * t.n;
+    const int ns = S.ns, nc = S.nc, vs1 = ns + 1, nv = vs1 * (nc + 1), np = ns * nc;
+    auto moved = [&](int v, int r) {
+        const double x[4] = {S.init[v], S.init[v + nv], S.init[v + 2 * nv], S.init[v + 3 * nv]};
+        return displace_row(M, 1, 4, r, x);
+    };
+    if (e < nv) {
+        double* V = S.verts + b * S.vsz;
+        double* W = S.wake + b * S.wsz;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const double y = moved(e, r);
+            V[e + r * nv] = y;
+            if (e / vs1 == nc) {
+                W[e % vs1 + r * 2 * vs1] = y;
+                W[vs1 + e % vs1 + r * 2 * vs1] = S.init[e + r * nv];
+            }
+        }
+        return;
+    }
+    const int p = e - nv, i = p % ns, j = p / ns;
+    auto vertex = [&](int v) -> v3<double> { return {moved(v, 0), moved(v, 1), moved(v, 2)}; };
+    const int v0 = i + j * vs1;
+    v3<double> c, n;
+    double area;
+    panel_metrics(par[0], vertex(v0), vertex(v0 + 1), vertex(v0 + 1 + vs1), vertex(v0 + vs1), c, n, area);
+    const double fx = par[1], fy = par[2], fz = par[3];
+    const int64_t o = b * S.psz;
+    double *C = S.colloc + 3 * o, *Nn = S.normals + 3 * o, *U = S.vel + 3 * o;
+    C[p] = c.x;
+    C[p + np] = c.y;
+    C[p + 2 * np] = c.z;
+    Nn[p] = n.x;
+    Nn[p + np] = n.y;
+    Nn[p + 2 * np] = n.z;
+    U[p] = fx;
+    U[p + np] = fy;
+    U[p + 2 * np] = fz;
+    S.areas[o + p] = area;
+    t.rhs[(int64_t)b * t.N + S.off + p] = -(fx * n.x + fy * n.y + fz * n.z);
+}
+
+constexpr int kVPostThreads = 1024;
+
+// Circulation differences, steady forces and the coefficient sums of request b0 + blockIdx.x, one
+// work-group (vlm.cpp:126-151): coef[(b n + m) * 8 + {0: area, 1: mac, 2: cl, 3..5: cm}], area and MAC
+// only as such (CL and CM are formed from the surfaces' sums on the host).
+__global__ __launch_bounds__(kVPostThreads) void k_vlm_post(VTab t, int b0) {
+    __shared__ double red[kVPostThreads / 64][6];
+    const int b = b0 + blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const double* par = t.par + (int64_t)b * (16 * t.n + kPar) + 16 * t.n;
+    const v3<double> U = {par[1], par[2], par[3]}, la = {par[4], par[5], par[6]}, ref = {par[7], par[8], par[9]};
+    for (int m = 0; m < t.n; m++) {
+        const VSurf& S = t.s[m];
+        const int ns = S.ns, nc = S.nc, vs1 = ns + 1, nv = vs1 * (nc + 1), np = ns * nc;
+        const int64_t o = b * S.psz;
+        const double* g = t.x + (int64_t)b * t.N + S.off;
+        const double* V = S.verts + b * S.vsz;
+        auto vertex = [&](int v) -> v3<double> { return {V[v], V[v + nv], V[v + 2 * nv]}; };
+        double v[6] = {};
+        for (int p = threadIdx.x; p < np; p += kVPostThreads) {
+            const int i = p % ns, j = p / ns, va = i + j * vs1;
+            const v3<double> a = vertex(va), e = vertex(va + 1);
+            const double area = S.areas[o + p];
+            const double gd = p >= ns ? g[p] - g[p - ns] : g[p];
+            const v3<double> F = gd * cross(U, e - a);  // rho = 1 as in the reference (vlm_backend_cpu.cpp:282)
+            S.gdelta[o + p] = gd;
+            double* f = S.forces + 3 * o + p;
+            f[0] = F.x;
+            f[np] = F.y;
+            f[2 * np] = F.z;
+            const v3<double> lever = 0.5 * (a + e) - ref, mo = cross(lever, F);
+            v[0] += area;
+            v[2] += dot(F, la);
+            v[3] += mo.x;
+            v[4] += mo.y;
+            v[5] += mo.z;
+        }
+        for (int i = threadIdx.x; i < ns; i += kVPostThreads) {
+            const v3<double> l0 = vertex(i), l1 = vertex(i + 1);
+            const v3<double> d0 = l0 - vertex(i + nc * vs1), d1 = l1 - vertex(i + 1 + nc * vs1), d3 = l1 - l0;
+            const double c0 = sqrt(dot(d0, d0)), c1 = sqrt(dot(d1, d1));
+            v[1] += 0.5 * (c0 * c0 + c1 * c1) * sqrt(dot(d3, d3));
+        }
+#pragma unroll
+        for (int k = 0; k < 6; k++)
+#pragma unroll
+            for (int h = 32; h > 0; h >>= 1) v[k] += __shfl_xor(v[k], h, 64);
+        __syncthreads();  // the previous surface's sums are read
+        if (lane == 0)
+            for (int k = 0; k < 6; k++) red[wave][k] = v[k];
+        __syncthreads();
+        if (threadIdx.x < 6) {
+            const int k = threadIdx.x;
+            double sum = 0.0, area = 0.0;
+            for (int w = 0; w < kVPostThreads / 64; w++) {
+                sum += red[w][k];
+                area += red[w][0];
+            }
+            t.coef[((int64_t)b * t.n + m) * 8 + k] = k == 0 ? sum : k == 1 ? sum / area : sum / par[10];
+        }
+    }
+}
 
 // r = rhs - A x per request (FP64).  A work-group takes 64 rows (one per lane) and its 8 waves
 // split the columns (wave w: columns w, w + 8, ...), so each wave reads 64 consecutive rows of a
@@ -177,13 +315,6 @@ __global__ void k_add_f32(double* __restrict__ x, const float* __restrict__ d, i
         x[i] += (double)d[i];
 }
 
-// gamma_delta(i, j) = gamma(i, j) - gamma(i, j-1), gamma_delta(i, 0) = gamma(i, 0) (vlm.cpp:126-139)
-__global__ void k_gamma_delta(const double* __restrict__ g, double* __restrict__ gd, int ns, int nc) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= ns * nc) return;
-    gd[p] = p >= ns ? g[p] - g[p - ns] : g[p];
-}
-
 int grid_for(int64_t n) { return (int)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096); }
 
 void views(tvlm_vlm_plan* P, int b, int m, tvlm_view& v, tvlm_view& w, tvlm_view& c, tvlm_view& nn, tvlm_view& a,
@@ -199,73 +330,50 @@ void views(tvlm_vlm_plan* P, int b, int m, tvlm_view& v, tvlm_view& w, tvlm_view
     gd = {P->gdelta[m] + b * P->psz[m], {ns, nc, 1}, {1, ns, ns * nc}};
 }
 
-// geometry, influence matrix (matrix = false: zeroed only; the caller assembles it) and rhs of
-// request b (vlm.cpp:97-124)
-int assemble(tvlm_vlm_plan* P, int b, bool seeded, bool matrix = true) {
-    hipStream_t st = P->stream;
-    const int n = P->n_surf;
-    std::vector<tvlm_view> V(n), W(n), C(n), Nn(n), A(n), VEL(n), F(n), GD(n), TR(n), INIT(n);
-    for (int m = 0; m < n; m++) {
-        views(P, b, m, V[m], W[m], C[m], Nn[m], A[m], VEL[m], F[m], GD[m]);
-        const int64_t ns = P->ns[m], nc = P->nc[m];
-        INIT[m] = {P->init[m], {ns + 1, nc + 1, 4}, {1, ns + 1, (ns + 1) * (nc + 1)}};
-        TR[m] = {P->tr + ((int64_t)b * n + m) * 16, {4, 4, 1}, {1, 4, 16}};
-        TVLM_HIP(hipMemcpyAsync(V[m].ptr, P->init[m], sizeof(double) * P->vsz[m], hipMemcpyDeviceToDevice, st));
+VTab table(const tvlm_vlm_plan* P) {
+    VTab t{};
+    t.n = P->n_surf;
+    t.N = P->N;
+    t.par = P->par;
+    t.rhs = P->rhs;
+    t.coef = P->coef;
+    t.x = P->x;
+    for (int m = 0; m < t.n; m++) {
+        t.s[m] = {P->init[m], P->verts[m], P->wake[m], P->colloc[m], P->normals[m], P->areas[m], P->vel[m],
+                  P->forces[m], P->gdelta[m], P->vsz[m], P->wsz[m], P->psz[m], (int32_t)P->ns[m], (int32_t)P->nc[m],
+                  (int32_t)P->off[m]};
+        t.items += (int32_t)(P->vsz[m] / 4 + P->psz[m]);
     }
-    TVLM_TRY(tvlm_wake_shed_f64(n, V.data(), W.data(), 0, st));
-    TVLM_TRY(tvlm_displace_wing_f64(n, TR.data(), V.data(), INIT.data(), st));
-    TVLM_TRY(tvlm_wake_shed_f64(n, V.data(), W.data(), 1, st));
-    TVLM_TRY(tvlm_mesh_metrics_f64(P->alpha[b], n, V.data(), C.data(), Nn.data(), A.data(), st));
-    const int64_t NN = (int64_t)P->N * P->N;
-    double* lhs = P->lhs + (P->mode == 1 ? b * NN : 0);
-    double* rhs = P->rhs + (int64_t)b * P->N;
-    TVLM_TRY(tvlm_fill_f64(0, lhs, 1, 0.0, NN, st));
-    TVLM_TRY(tvlm_fill_f64(0, rhs, 1, 0.0, P->N, st));
-    tvlm_view L = {lhs, {P->N, P->N, 1}, {1, P->N, NN}};
-    if (matrix && seeded)
-        TVLM_TRY(lhs_assemble_seeded_f64(&L, n, C.data(), Nn.data(), V.data(), W.data(), 1, st));
-    else if (matrix)
-        TVLM_TRY(tvlm_lhs_assemble_f64(&L, n, C.data(), Nn.data(), V.data(), W.data(), 1, 0.0, st));
-    const double a = P->alpha[b], be = P->beta[b], u = P->u_inf;
-    const double fs[3] = {u * std::cos(a) * std::cos(be), -u * std::cos(a) * std::sin(be), u * std::sin(a)};
-    for (int m = 0; m < n; m++)
-        for (int k = 0; k < 3; k++)
-            TVLM_TRY(tvlm_fill_f64(0, static_cast<double*>(VEL[m].ptr) + k * P->psz[m], 1, fs[k], P->psz[m], st));
-    tvlm_view R = {rhs, {P->N, 1, 1}, {1, P->N, P->N}};
-    TVLM_TRY(tvlm_rhs_assemble_velocities_f64(&R, n, Nn.data(), VEL.data(), st));
+    return t;
+}
+
+// geometry and rhs of requests [b0, b0 + count)
+int geometry(tvlm_vlm_plan* P, int b0, int count) {
+    const VTab t = table(P);
+    hipLaunchKernelGGL(k_vlm_geom, dim3((t.items + 255) / 256, count), dim3(256), 0, P->stream, t, b0);
+    TVLM_LAUNCHED();
     return TVLM_OK;
 }
 
-// circulation differences, forces and per-surface coefficients of request b (vlm.cpp:126-151);
-// coef[(b n_surf + m) * 8 + {0: area, 1: mac, 2: cl, 3..5: cm}]
-int post(tvlm_vlm_plan* P, int b) {
+// circulation differences, forces and coefficients of requests [b0, b0 + count)
+int post(tvlm_vlm_plan* P, int b0, int count) {
+    hipLaunchKernelGGL(k_vlm_post, dim3(count), dim3(kVPostThreads), 0, P->stream, table(P), b0);
+    TVLM_LAUNCHED();
+    return TVLM_OK;
+}
+
+// influence matrix of request b, whose geometry stands (seeded: the served form)
+int matrix(tvlm_vlm_plan* P, int b, bool seeded) {
     hipStream_t st = P->stream;
     const int n = P->n_surf;
-    const double a = P->alpha[b], be = P->beta[b], u = P->u_inf;
-    const double fs[3] = {u * std::cos(a) * std::cos(be), -u * std::cos(a) * std::sin(be), u * std::sin(a)};
-    // lift axis normalize(fs x y) (vlm/src/vlm_utils.cpp:13-15)
-    double la[3] = {-fs[2], 0.0, fs[0]};
-    const double ln = std::sqrt(la[0] * la[0] + la[2] * la[2]);
-    la[0] /= ln;
-    la[2] /= ln;
-    const double* ref = P->ref.data() + 3 * b;
-    for (int m = 0; m < n; m++) {
-        tvlm_view V, W, C, Nn, A, VEL, F, GD;
-        views(P, b, m, V, W, C, Nn, A, VEL, F, GD);
-        const double* g = P->x + (int64_t)b * P->N + P->off[m];
-        hipLaunchKernelGGL(k_gamma_delta, dim3(grid_for(P->psz[m])), dim3(256), 0, st, g,
-                           static_cast<double*>(GD.ptr), (int)P->ns[m], (int)P->nc[m]);
-        TVLM_LAUNCHED();
-        TVLM_TRY(tvlm_forces_steady_f64(&V, &GD, &VEL, &F, st));
-        double* cf = P->coef + ((int64_t)b * n + m) * 8;
-        tvlm_view A2 = {A.ptr, {P->ns[m], P->nc[m], 1}, {1, P->ns[m], P->psz[m]}};
-        TVLM_TRY(tvlm_sum_f64(&A2, 2, cf + 0, st));
-        TVLM_TRY(tvlm_mesh_mac_f64(&V, &A2, cf + 1, st));
-        // area and MAC enter only the normalisation: CL and CM are formed on the host from these sums
-        TVLM_TRY(tvlm_coeff_cl_f64(&F, la, fs, P->rho, 1.0, cf + 2, st));
-        TVLM_TRY(tvlm_coeff_cm_f64(&F, &V, ref, fs, P->rho, 1.0, 1.0, cf + 3, st));
-    }
-    return TVLM_OK;
+    std::vector<tvlm_view> V(n), W(n), C(n), Nn(n), A(n), VEL(n), F(n), GD(n);
+    for (int m = 0; m < n; m++) views(P, b, m, V[m], W[m], C[m], Nn[m], A[m], VEL[m], F[m], GD[m]);
+    const int64_t NN = (int64_t)P->N * P->N;
+    double* lhs = P->lhs + (P->mode == 1 ? b * NN : 0);
+    TVLM_TRY(tvlm_fill_f64(0, lhs, 1, 0.0, NN, st));
+    tvlm_view L = {lhs, {P->N, P->N, 1}, {1, P->N, NN}};
+    if (seeded) return lhs_assemble_seeded_f64(&L, n, C.data(), Nn.data(), V.data(), W.data(), 1, st);
+    return tvlm_lhs_assemble_f64(&L, n, C.data(), Nn.data(), V.data(), W.data(), 1, 0.0, st);
 }
 
 // Served mode, after the solve: reads the per-request test results; for every request that failed,
@@ -339,7 +447,7 @@ int rescue(tvlm_vlm_plan* P) {
             TVLM_HIP(hipStreamSynchronize(st));
             if (i64 == kGetrfStalled) {
                 // its factors are invalid and the matrix is gone: assemble it again, one-group panels
-                TVLM_TRY(assemble(P, b, true));
+                TVLM_TRY(matrix(P, b, true));
                 TVLM_TRY(getrf_single_group_f64(&L64, ipiv, inf, st));
                 TVLM_HIP(hipMemcpyAsync(&i64, inf, sizeof(int32_t), hipMemcpyDeviceToHost, st));
                 TVLM_HIP(hipStreamSynchronize(st));
@@ -354,7 +462,7 @@ int rescue(tvlm_vlm_plan* P) {
         }
         P->st_status[b] = status;
         P->st_corr[b] = corr;
-        TVLM_TRY(post(P, b));
+        TVLM_TRY(post(P, b, 1));
     }
     return TVLM_OK;
 }
@@ -398,7 +506,7 @@ int tvlm_vlm_create(tvlm_vlm_plan** plan, int32_t n_surf, const int64_t* ns, con
     auto fail = [&](int rc) {
         (void)tvlm_lhs_group_destroy(P->group);
         for (void* p : P->allocs) (void)hipFree(p);
-        if (P->tr_host) (void)hipHostFree(P->tr_host);
+        if (P->par_host) (void)hipHostFree(P->par_host);
         if (P->done) (void)hipEventDestroy(P->done);
         delete P;
         return rc;
@@ -426,23 +534,17 @@ int tvlm_vlm_create(tvlm_vlm_plan** plan, int32_t n_surf, const int64_t* ns, con
     if (rc == TVLM_OK && mode == 1) rc = P->alloc((void**)&P->conv, sizeof(int32_t) * batch);
     if (rc == TVLM_OK) rc = P->alloc((void**)&P->rhs, sizeof(double) * N * batch);
     if (rc == TVLM_OK) rc = P->alloc((void**)&P->x, sizeof(double) * N * batch);
-    if (rc == TVLM_OK) rc = P->alloc((void**)&P->tr, sizeof(double) * 16 * n_surf * batch);
+    if (rc == TVLM_OK) rc = P->alloc((void**)&P->par, sizeof(double) * (16 * n_surf + kPar) * batch);
     if (rc == TVLM_OK) rc = P->alloc((void**)&P->coef, sizeof(double) * 8 * n_surf * batch);
     if (rc == TVLM_OK) rc = P->alloc((void**)&P->ipiv, sizeof(int32_t) * N * nb);
     if (rc == TVLM_OK) rc = P->alloc((void**)&P->info, sizeof(int32_t) * batch);
     if (rc == TVLM_OK) {
-        hipError_t e = hipHostMalloc((void**)&P->tr_host, sizeof(double) * 16 * n_surf * batch, hipHostMallocDefault);
+        hipError_t e = hipHostMalloc((void**)&P->par_host, sizeof(double) * (16 * n_surf + kPar) * batch,
+                                     hipHostMallocDefault);
         if (e != hipSuccess) {
             set_error("hipHostMalloc failed: %s", hipGetErrorString(e));
             rc = TVLM_ERR_NOMEM;
         }
-    }
-    if (rc == TVLM_OK) {
-        // the wake rows' w coordinate is 1 and stays so (vlm.cpp:94)
-        for (int m = 0; m < n_surf && rc == TVLM_OK; m++)
-            for (int b = 0; b < batch && rc == TVLM_OK; b++)
-                rc = tvlm_fill_f64(0, P->wake[m] + b * P->wsz[m] + 3 * (P->ns[m] + 1) * 2, 1, 1.0, (P->ns[m] + 1) * 2,
-                                   stream);
     }
     if (rc == TVLM_OK && hipEventCreateWithFlags(&P->done, hipEventDisableTiming) != hipSuccess) {
         set_error("hipEventCreateWithFlags failed");
@@ -468,9 +570,6 @@ int tvlm_vlm_create(tvlm_vlm_plan** plan, int32_t n_surf, const int64_t* ns, con
         rc = tvlm_lhs_group_create(&P->group, batch, items.data(), stream);
     }
     if (rc != TVLM_OK) return fail(rc);
-    P->alpha.assign(batch, 0.0);
-    P->beta.assign(batch, 0.0);
-    P->ref.assign(3 * batch, 0.0);
     *plan = P;
     return TVLM_OK;
 }
@@ -487,44 +586,43 @@ int tvlm_vlm_solve_n(tvlm_vlm_plan* P, int32_t n_active, const double* alpha, co
     TVLM_REQUIRE(n_active >= 1 && n_active <= P->batch, "n_active %d out of range 1..%d", n_active, P->batch);
     const int n = P->n_surf, B = n_active;
     P->active = B;
-    P->u_inf = u_inf;
-    P->rho = rho;
     const double c0[3] = {cm_ref ? cm_ref[0] : 0.25, cm_ref ? cm_ref[1] : 0.0, cm_ref ? cm_ref[2] : 0.0};
-    TVLM_HIP(hipEventSynchronize(P->done));  // the pinned transform buffer may still be read
+    TVLM_HIP(hipEventSynchronize(P->done));  // the pinned parameters may still be read
     for (int b = 0; b < B; b++) {
-        P->alpha[b] = alpha[b];
-        P->beta[b] = beta ? beta[b] : 0.0;
+        const double a = alpha[b], be = beta ? beta[b] : 0.0, u = u_inf;
+        double* T = P->par_host + (int64_t)b * (16 * n + kPar);
         // translation by -100 u (cos a, 0, sin a): 100-chord wake row (vlm.cpp:104-108)
-        const double tx = -100.0 * u_inf * std::cos(alpha[b]), tz = -100.0 * u_inf * std::sin(alpha[b]);
-        for (int m = 0; m < n; m++) {
-            double* T = P->tr_host + ((int64_t)b * n + m) * 16;
+        const double tx = -100.0 * u * std::cos(a), tz = -100.0 * u * std::sin(a);
+        for (int m = 0; m < n; m++, T += 16) {
             for (int k = 0; k < 16; k++) T[k] = (k % 5 == 0) ? 1.0 : 0.0;
             T[12] = tx;
             T[14] = tz;
         }
-        P->ref[3 * b + 0] = c0[0] + tx;
-        P->ref[3 * b + 1] = c0[1];
-        P->ref[3 * b + 2] = c0[2] + tz;
+        const double fs[3] = {u * std::cos(a) * std::cos(be), -u * std::cos(a) * std::sin(be), u * std::sin(a)};
+        // lift axis normalize(fs x y) (vlm/src/vlm_utils.cpp:13-15)
+        const double ln = std::sqrt(fs[2] * fs[2] + fs[0] * fs[0]);
+        const double v[kPar] = {a,          fs[0], fs[1],      fs[2],           -fs[2] / ln, 0.0,
+                                fs[0] / ln, c0[0] + tx, c0[1], c0[2] + tz,
+                                0.5 * rho * (fs[0] * fs[0] + fs[1] * fs[1] + fs[2] * fs[2]), 0.0};
+        std::copy(v, v + kPar, T);
     }
     hipStream_t st = P->stream;
-    TVLM_HIP(hipMemcpyAsync(P->tr, P->tr_host, sizeof(double) * 16 * n * B, hipMemcpyHostToDevice, st));
+    TVLM_HIP(hipMemcpyAsync(P->par, P->par_host, sizeof(double) * (16 * n + kPar) * B, hipMemcpyHostToDevice, st));
+    TVLM_TRY(geometry(P, 0, B));
     const int64_t N = P->N, NN = N * N;
     if (P->mode == 0) {
         tvlm_view L = {P->lhs, {N, N, 1}, {1, N, NN}};
         for (int b = 0; b < B; b++) {
-            TVLM_TRY(assemble(P, b, false));
+            TVLM_TRY(matrix(P, b, false));
             TVLM_TRY(tvlm_getrf_f64(&L, P->ipiv, P->info + b, st));
             TVLM_HIP(hipMemcpyAsync(P->x + b * N, P->rhs + b * N, sizeof(double) * N, hipMemcpyDeviceToDevice, st));
             tvlm_view X = {P->x + b * N, {N, 1, 1}, {1, N, N}};
             TVLM_TRY(tvlm_getrs_f64(&L, P->ipiv, &X, st));
-            TVLM_TRY(post(P, b));
         }
+        TVLM_TRY(post(P, 0, B));
     } else {
-        // geometry and rhs request by request, then every request's matrix in one grouped launch
-        for (int b = 0; b < B; b++) TVLM_TRY(assemble(P, b, true, false));
-        TVLM_TRY(tvlm_lhs_group_assemble_f64(P->group, B, 1, 0.0, st));
-        hipLaunchKernelGGL(k_to_f32, dim3(4096), dim3(256), 0, st, P->lhs, P->lhs32, NN * B);
-        TVLM_LAUNCHED();
+        // every request's matrix and its FP32 copy in one grouped launch
+        TVLM_TRY(lhs_group_assign_seeded(P->group, B, P->lhs, P->lhs32, st));
         tvlm_view L32 = {P->lhs32, {N, N, B}, {1, N, NN}};
         TVLM_TRY(tvlm_getrf_f32(&L32, P->ipiv, P->info, st));
         tvlm_view R32 = {P->r32, {N, 1, B}, {1, N, N}};
@@ -557,7 +655,7 @@ int tvlm_vlm_solve_n(tvlm_vlm_plan* P, int32_t n_active, const double* alpha, co
         hipLaunchKernelGGL(k_refine_check, dim3(B), dim3(256), 0, st, P->res, P->x, P->rowabs, P->info, (int)N,
                            P->berr, P->conv);
         TVLM_LAUNCHED();
-        for (int b = 0; b < B; b++) TVLM_TRY(post(P, b));
+        TVLM_TRY(post(P, 0, B));
     }
     TVLM_HIP(hipEventRecord(P->done, st));
     P->solved = true;
@@ -651,7 +749,7 @@ int tvlm_vlm_destroy(tvlm_vlm_plan* P) {
     (void)tvlm_lhs_group_destroy(P->group);
     for (void* p : P->allocs) (void)hipFree(p);
     (void)hipEventDestroy(P->done);
-    if (P->tr_host) (void)hipHostFree(P->tr_host);
+    if (P->par_host) (void)hipHostFree(P->par_host);
     delete P;
     return TVLM_OK;
 }
