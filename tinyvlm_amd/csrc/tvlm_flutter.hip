@@ -37,7 +37,7 @@ namespace {
 constexpr int kFlMaxIter = 50;                                 // iterations stop once it > 50 (uvlm_2dof.cpp:637, :795)
 constexpr double kFlEps = (double)1.19209e-07f;                // EPS_f (vlm_types.hpp:24)
 constexpr double kPiF = (double)3.141593f;                     // PI_f (vlm_types.hpp:21)
-constexpr int kFlChunk = 8;                                    // airspeeds per k_fl_gemm work-group
+constexpr int kFlTile = 16;                                    // rows and airspeeds per k_fl_gemm work-group
 constexpr int kFlGemmCols = 512;                               // columns per k_fl_gemm work-group
 constexpr int kFlPostThreads = 1024;
 
@@ -291,37 +291,56 @@ __global__ __launch_bounds__(64 * kRedWaves) void k_fl_reduce(FlConst c, FlBufs 
     if (wave == 0 && p < c.N) d.rhs[b * d.sp + p] = d.rhs_vel[b * d.sp + p] - red[0][lane];
 }
 
-// gpart[b][cb][row] = A^{-1}(row, columns of block cb) rhs_b: 64 rows per work-group (one per lane),
-// its 4 waves split the block's columns, kFlChunk airspeeds (blockIdx.z) per work-group so that each
-// element of A^{-1} is read once per chunk.
+// gpart[b][cb][row] = A^{-1}(row, columns of block cb) rhs_b for kFlTile rows and kFlTile airspeeds
+// (blockIdx.z) on the FP64 matrix cores (16x16x4), the work-group's 4 waves splitting the block's columns.
+// A lane's operands are A^{-1}(row lane & 15, .) and airspeed lane & 15's rhs, at columns col + 4 (lane >> 4)
+// + k for instruction k of 4, so that a lane reads 32 consecutive bytes of rhs.  Rows past N and airspeeds
+// past B repeat the last one and are not stored; columns past the block count as 0.
+// Bound by the read of A^{-1} and its latency: 16-row tiles give 4 times the work-groups of 64-row ones and one
+// read of A^{-1} per 16 airspeeds.  2000 panels, 16 airspeeds: 136 us a launch with one row per lane and 8
+// airspeeds per work-group on the vector unit, 8.3 us so.  An airspeed's sums do not depend on the others.
 __global__ __launch_bounds__(256) void k_fl_gemm(FlConst c, FlBufs d, const double* __restrict__ Ainv,
                                                  double* __restrict__ gpart, int cbs) {
-    __shared__ double red[4][kFlChunk][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    typedef double vd4 __attribute__((ext_vector_type(4)));
+    __shared__ double red[4][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, m = lane & 15, h = lane >> 4;
     const int N = c.N;
-    const int row = blockIdx.x * 64 + lane;
-    const int c0 = blockIdx.y * cbs, c1 = min(N, c0 + cbs);
-    const int b0 = blockIdx.z * kFlChunk;
-    const int nb = min(kFlChunk, c.B - b0);
-    double acc[kFlChunk];
+    const int r0 = blockIdx.x * kFlTile, b0 = blockIdx.z * kFlTile;
+    const int span = cbs / 4;  // a multiple of 16
+    const int c0 = blockIdx.y * cbs + wave * span, c1 = min(N, c0 + span);
+    const double* ap = Ainv + min(r0 + m, N - 1);
+    const double* xp = d.rhs + min(b0 + m, c.B - 1) * d.sp;
+    vd4 acc = {0.0, 0.0, 0.0, 0.0};
+    int col = c0 + 4 * h;
+#pragma unroll 2
+    for (int e = c0; e + 16 <= c1; e += 16, col += 16) {
+        double p[4], q[4];
 #pragma unroll
-    for (int k = 0; k < kFlChunk; k++) acc[k] = 0.0;
-    if (row < N) {
-        for (int col = c0 + wave; col < c1; col += 4) {
-            const double a = Ainv[row + (int64_t)col * N];
+        for (int k = 0; k < 4; k++) {
+            p[k] = ap[(int64_t)(col + k) * N];
+            q[k] = xp[col + k];
+        }
 #pragma unroll
-            for (int k = 0; k < kFlChunk; k++)
-                if (k < nb) acc[k] += a * d.rhs[(b0 + k) * d.sp + col];
+        for (int k = 0; k < 4; k++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(p[k], q[k], acc, 0, 0, 0);
+    }
+    if (c0 < c1 && (c1 - c0) % 16) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const bool in = col + k < c1;
+            const double p = in ? ap[(int64_t)(col + k) * N] : 0.0;
+            const double q = in ? xp[col + k] : 0.0;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(p, q, acc, 0, 0, 0);
         }
     }
+    // result register r: row h + 4 r of the tile, airspeed m
 #pragma unroll
-    for (int k = 0; k < kFlChunk; k++) red[wave][k][lane] = acc[k];
+    for (int r = 0; r < 4; r++) red[wave][r][lane] = acc[r];
     __syncthreads();
-    if (wave == 0 && row < N) {
-        const int ncb = gridDim.y;
-        for (int k = 0; k < nb; k++)
-            gpart[((int64_t)(b0 + k) * ncb + blockIdx.y) * N + row] =
-                (red[0][k][lane] + red[1][k][lane]) + (red[2][k][lane] + red[3][k][lane]);
+    const int b = b0 + (threadIdx.x >> 4), row = threadIdx.x & 15;  // stores: rows along the lanes
+    if (b < c.B && r0 + row < N) {
+        const int r = row >> 2, l = (row & 3) * 16 + (threadIdx.x >> 4);
+        gpart[((int64_t)b * gridDim.y + blockIdx.y) * N + r0 + row] =
+            (red[0][r][l] + red[1][r][l]) + (red[2][r][l] + red[3][r][l]);
     }
 }
 
@@ -552,8 +571,8 @@ int fl_iteration(tvlm_flutter_plan* P, int step) {
     hipLaunchKernelGGL(k_fl_reduce, dim3((c.N + 63) / 64, c.B), dim3(64 * kRedWaves), 0, st, c, P->d, P->st,
                        P->partial, P->spart, tiles);
     TVLM_LAUNCHED();
-    hipLaunchKernelGGL(k_fl_gemm, dim3((c.N + 63) / 64, P->ncb, (c.B + kFlChunk - 1) / kFlChunk), dim3(256), 0, st, c,
-                       P->d, P->ainv, P->gpart, P->cbs);
+    hipLaunchKernelGGL(k_fl_gemm, dim3((c.N + kFlTile - 1) / kFlTile, P->ncb, (c.B + kFlTile - 1) / kFlTile), dim3(256), 0,
+                       st, c, P->d, P->ainv, P->gpart, P->cbs);
     TVLM_LAUNCHED();
     hipLaunchKernelGGL(k_fl_post, dim3(c.B), dim3(kFlPostThreads), 0, st, c, P->d, P->air, P->st, P->gpart, P->ncb,
                        step);
