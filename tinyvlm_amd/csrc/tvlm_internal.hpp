@@ -74,6 +74,14 @@ int noalloc_scratch_setup();
 // work-groups): the recovery path after a cooperative panel's bounded wait gave up
 int getrf_single_group_f64(const tvlm_view* a, int32_t* ipiv, int32_t* info, void* stream);
 int getrf_single_group_f32(const tvlm_view* a, int32_t* ipiv, int32_t* info, void* stream);
+
+// getrs of several right-hand sides one after another on the same factors: what it derives from them first
+// (block inverses, composed interchanges) is made once, in `prep` of getrs_prep_bytes_f32 bytes (0 where n is
+// past the sizes that use it; prep is then null), for as long as the factors stand.
+size_t getrs_prep_bytes_f32(int64_t n, int batch);
+int getrs_prepare_f32(const tvlm_view* a, const int32_t* ipiv, void* prep, hipStream_t stream);
+int getrs_prepared_f32(const tvlm_view* a, const int32_t* ipiv, void* prep, const tvlm_view* x, hipStream_t stream);
+
 constexpr int32_t kGetrfStalled = -999;  // info of a matrix whose cooperative panel gave up waiting
 
 // Work-group targets of the wake-induction launches, library-wide (tvlm_set_tile_targets): the

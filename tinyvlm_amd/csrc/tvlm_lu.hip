@@ -17,12 +17,12 @@
 //   3. k_update     : A22 -= L21 U12 on the matrix cores (double-buffered 16-deep k-slices).
 // Panels taller than the cooperative groups hold (and taller than 8192 rows) use the
 // column-by-column k_panel + k_laswp + k_trsm instead.
-// getrs (n <= 16384): the interchanges are composed per block of 64 pivots and the 64 x 64
-// diagonal blocks of L and U inverted (k_solve_prep), then one work-group per right-hand side
-// applies the interchanges and both blocked substitutions with the column in LDS
-// (k_solve_blocked); from n = 1024 with few right-hand sides, the interchanges are applied alone
-// (k_solve_perm) and each 64-row block step runs on all trailing row blocks at once
-// (k_trsv_step); larger n uses block-row kernels (k_diag_solve / k_off_update).
+// getrs (n <= 16384): the interchanges are composed (k_solve_prep per block of 64 pivots, k_solve_compose
+// over the blocks) and the 64 x 64 diagonal blocks of L and U inverted (k_solve_prep); then up to n = 256 one
+// work-group per right-hand side does the rest (k_solve_small), above that the interchanges are applied
+// (k_solve_perm) and each 256-row step of a substitution runs on all trailing row blocks at once
+// (k_trsv_step), or, with many right-hand sides, 64-row steps multiply all of them on the matrix cores
+// (k_inv_apply, k_update); larger n uses block-row kernels (k_diag_solve / k_off_update).
 #include <atomic>
 #include <map>
 #include <utility>
@@ -1491,6 +1491,7 @@ struct UpdCfg<double> {
 };
 
 constexpr int kUpdDK = 16;  // k-slice depth
+constexpr int64_t kUpdMaxLd = (int64_t)1 << 26;  // leading dimensions whose 16 columns fit 32-bit offsets
 
 // The FP32 128 x 64 tile is held to 6 waves per SIMD (its accumulators then sit in 80 vector registers
 // beside the operands instead of 32 accumulation registers: 5 -> 6 waves; measured ~1 % on getrf).
@@ -2217,28 +2218,27 @@ int getrf(const tvlm_view* av, int32_t* ipiv, int32_t* info, void* stream, bool 
     return TVLM_OK;
 }
 
-// ---- blocked getrs: interchange lists + diagonal-block inverses + one work-group per rhs -------
-//
-// k_solve_prep, y = 0: composes the interchanges of pivot block b (64 positions) into (dst, src)
-//   pairs (one wave); y = 1 / 2: inverts the 64 x 64 diagonal block b of L (unit lower) / U (upper),
-//   one column per lane, each row's dot product split over 4 waves.
-// k_solve_blocked: the rhs column lives in LDS; the interchange lists are applied block after
-//   block; then x_b = Linv_b (x_b - L_{b,<b} x_{<b}) for b ascending and x_b = Uinv_b (x_b -
-//   U_{b,>b} x_{>b}) for b descending, each off-diagonal product split over 16 thread groups
-//   reading 64 consecutive rows per column, partial sums reduced in LDS.
+// ---- blocked getrs ----------------------------------------------------------------------------
 constexpr int kSB = 64;            // solve block
+constexpr int kSW = 4 * kSB;       // rows of a substitution step
 constexpr int kSolveMaxN = 16384;  // rhs column in LDS
 constexpr int kSolvePairs = 1 + 2 * 2 * kSB;
 
+// y = 0: composes the interchanges of pivot block b (64 positions) into (dst, src) pairs (one wave);
+// y = 1 / 2: inverts the 64 x 64 diagonal block b of L (unit lower) / U (upper): each wave one 16 x 16
+// diagonal tile by substitution, a column per lane; then tile pairs and the two 32-row halves are merged by
+// [A 0; B C]^-1 = [A^-1 0; -C^-1 B A^-1, C^-1] (U: its mirror image) on the matrix cores.  Bound by the chain of
+// dependent steps: row by row over all 64 with the sums split over the waves it took 46 us, 32 times 8 blocks;
+// 14 us so.
 template <typename T>
 __global__ __launch_bounds__(256) void k_solve_prep(const T* __restrict__ a, int64_t lda, int n,
                                                     const int32_t* __restrict__ ipiv, int32_t* __restrict__ pairs,
                                                     T* __restrict__ inv, int64_t sa) {
+    using M = Mf16<T>;
     __shared__ int s_p[kSB];
     __shared__ int s_pd[2 * kSB], s_ps[2 * kSB];
     __shared__ T s_a[kSB][kSB + 1];
     __shared__ T s_x[kSB][kSB + 1];  // the inverse, row by row
-    __shared__ T s_red[4][kSB];
     const int nb_ = (n + kSB - 1) / kSB;  // batch: one matrix per blockIdx.z
     a += (int64_t)blockIdx.z * sa;
     ipiv += (int64_t)blockIdx.z * n;
@@ -2264,34 +2264,70 @@ __global__ __launch_bounds__(256) void k_solve_prep(const T* __restrict__ a, int
     for (int e = t; e < kSB * kSB; e += 256) {
         const int r = e % kSB, c = e / kSB;
         s_a[r][c] = (r < rb && c < rb) ? a[(r0 + r) + (int64_t)(r0 + c) * lda] : (r == c ? T(1) : T(0));
+        s_x[r][c] = T(0);
     }
     __syncthreads();
-    // Column j of the inverse belongs to lane j; row i of it is formed from the rows already done,
-    // the dot product over them split over the 4 waves (wave g takes p = g, g + 4, ...) and summed
-    // in a fixed order.  Unit lower: X_ij = delta_ij - sum_{j <= p < i} L_ip X_pj, rows ascending;
-    // upper: X_ij = (delta_ij - sum_{i < p <= j} U_ip X_pj) / U_ii, rows descending.
-    const int j = lane;
-    for (int k = 0; k < kSB; k++) {
-        const int i = lower ? k : kSB - 1 - k;
-        T part = T(0);
+    const int m = lane & 15;
+    {
+        T v[16];
+        const int o = 16 * g;
         if (lower) {
-            for (int p = j + ((g - j) % 4 + 4) % 4; p < i; p += 4) part += s_a[i][p] * s_x[p][j];
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                T sum = T(0);
+#pragma unroll
+                for (int p = 0; p < i; p++) sum += s_a[o + i][o + p] * v[p];
+                v[i] = i < m ? T(0) : (i == m ? T(1) : -sum);
+            }
         } else {
-            for (int p = i + 1 + g; p <= j; p += 4) part += s_a[i][p] * s_x[p][j];
+#pragma unroll
+            for (int i = 15; i >= 0; i--) {
+                T sum = T(0);
+#pragma unroll
+                for (int p = i + 1; p < 16; p++) sum += s_a[o + i][o + p] * v[p];
+                v[i] = i > m ? T(0) : ((i == m ? T(1) : T(0)) - sum) / s_a[o + i][o + i];
+            }
         }
-        s_red[g][j] = part;
-        __syncthreads();
-        if (g == 0) {
-            const T sum = (s_red[0][j] + s_red[1][j]) + (s_red[2][j] + s_red[3][j]);
-            T v;
-            if (lower)
-                v = i < j ? T(0) : (i == j ? T(1) : -sum);
-            else
-                v = i > j ? T(0) : ((i == j ? T(1) : T(0)) - sum) / s_a[i][i];
-            s_x[i][j] = v;
-        }
-        __syncthreads();
+        if (lane < 16)
+#pragma unroll
+            for (int i = 0; i < 16; i++) s_x[o + i][o + m] = v[i];
     }
+    __syncthreads();
+    typedef typename M::vacc vacc;
+    // c + P(tile pi, pk of s) Q, Q a 16 x 16 tile in the second operand's layout
+    auto mul = [&](const T(*P)[kSB + 1], int pi, int pk, const vacc& q, vacc c) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) c = M::mfma(P[16 * pi + m][16 * pk + M::k(lane, r)], q[r], c);
+        return c;
+    };
+    auto tile = [&](int ki, int kj) {
+        vacc q;
+#pragma unroll
+        for (int r = 0; r < 4; r++) q[r] = s_x[16 * ki + M::k(lane, r)][16 * kj + m];
+        return q;
+    };
+    auto put = [&](int ki, int kj, const vacc& q) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) s_x[16 * ki + M::k(lane, r)][16 * kj + m] = -q[r];
+    };
+    const vacc zero = {T(0), T(0), T(0), T(0)};
+    if (g < 2) {  // i: the tile row to form, k: the tile row it draws on
+        const int i = lower ? 2 * g + 1 : 2 * g, k = lower ? 2 * g : 2 * g + 1;
+        put(i, k, mul(s_x, i, i, mul(s_a, i, k, tile(k, k), zero), zero));
+    }
+    __syncthreads();
+    {
+        const int i0 = lower ? 2 : 0, q0 = lower ? 0 : 2;  // first tile row to form, first it draws on
+        const int i = i0 + (g >> 1), col = q0 + (g & 1);
+        const vacc x0 = tile(q0, col), x1 = tile(q0 + 1, col);
+        const vacc t0 = mul(s_a, i0, q0 + 1, x1, mul(s_a, i0, q0, x0, zero));
+        const vacc t1 = mul(s_a, i0 + 1, q0 + 1, x1, mul(s_a, i0 + 1, q0, x0, zero));
+        vacc y = zero;
+        if (lower ? true : i == i0) y = mul(s_x, i, i0, t0, y);
+        if (lower ? i > i0 : true) y = mul(s_x, i, i0 + 1, t1, y);
+        put(i, col, y);
+    }
+    __syncthreads();
     T* out = inv + ((int64_t)(lower ? 0 : 1) * ((n + kSB - 1) / kSB) + b) * kSB * kSB;
     for (int e = t; e < kSB * kSB; e += 256) {
         const int r = e % kSB, c = e / kSB;
@@ -2299,180 +2335,343 @@ __global__ __launch_bounds__(256) void k_solve_prep(const T* __restrict__ a, int
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(1024) void k_solve_blocked(const T* __restrict__ a, int64_t lda, int n,
-                                                        const int32_t* __restrict__ pairs, const T* __restrict__ inv,
-                                                        T* __restrict__ x, int64_t ldx, int64_t sa, int64_t sx) {
-    __shared__ T xs[kSolveMaxN];
-    __shared__ T red[16][kSB];
-    __shared__ T yb[kSB];
-    const int t = threadIdx.x, r = t & 63, g = t >> 6;
-    const int nblk = (n + kSB - 1) / kSB;
-    a += (int64_t)blockIdx.z * sa;  // batch: one matrix per blockIdx.z
-    pairs += (int64_t)blockIdx.z * nblk * kSolvePairs;
-    inv += (int64_t)blockIdx.z * 2 * nblk * kSB * kSB;
-    x += (int64_t)blockIdx.z * sx;
-    T* xc = x + (int64_t)blockIdx.x * ldx;
-    for (int i = t; i < n; i += 1024) xs[i] = xc[i];
-    __syncthreads();
-    for (int b = 0; b < nblk; b++) {  // P b: interchange lists in pivot order
-        const int32_t* pl = pairs + (int64_t)b * kSolvePairs;
-        const int np = pl[0];
-        T v = T(0);
-        if (t < np) v = xs[pl[2 + 2 * t]];
-        __syncthreads();
-        if (t < np) xs[pl[1 + 2 * t]] = v;
-        __syncthreads();
-    }
-    const T* linv = inv;
-    const T* uinv = inv + (int64_t)nblk * kSB * kSB;
-    // L y = P b
-    for (int b = 0; b < nblk; b++) {
-        const int r0 = b * kSB, rb = min(kSB, n - r0);
-        T acc = T(0);
-        if (r < rb)
-            for (int j = g; j < r0; j += 16) acc += a[(r0 + r) + (int64_t)j * lda] * xs[j];
-        red[g][r] = acc;
-        __syncthreads();
-        if (t < kSB) {
-            T y = t < rb ? xs[r0 + t] : T(0);
-#pragma unroll
-            for (int q = 0; q < 16; q++) y -= red[q][t];
-            yb[t] = y;
-        }
-        __syncthreads();
-        T s = T(0);
-        const T* lb = linv + (int64_t)b * kSB * kSB;
-#pragma unroll
-        for (int p = 4 * g; p < 4 * g + 4; p++) s += lb[r + p * kSB] * yb[p];
-        red[g][r] = s;
-        __syncthreads();
-        if (t < rb) {
-            T v = T(0);
-#pragma unroll
-            for (int q = 0; q < 16; q++) v += red[q][t];
-            xs[r0 + t] = v;
-        }
-        __syncthreads();
-    }
-    // U x = y
-    for (int b = nblk - 1; b >= 0; b--) {
-        const int r0 = b * kSB, rb = min(kSB, n - r0);
-        T acc = T(0);
-        if (r < rb)
-            for (int j = r0 + kSB + g; j < n; j += 16) acc += a[(r0 + r) + (int64_t)j * lda] * xs[j];
-        red[g][r] = acc;
-        __syncthreads();
-        if (t < kSB) {
-            T y = t < rb ? xs[r0 + t] : T(0);
-#pragma unroll
-            for (int q = 0; q < 16; q++) y -= red[q][t];
-            yb[t] = y;
-        }
-        __syncthreads();
-        T s = T(0);
-        const T* ub = uinv + (int64_t)b * kSB * kSB;
-#pragma unroll
-        for (int p = 4 * g; p < 4 * g + 4; p++) s += ub[r + p * kSB] * yb[p];
-        red[g][r] = s;
-        __syncthreads();
-        if (t < rb) {
-            T v = T(0);
-#pragma unroll
-            for (int q = 0; q < 16; q++) v += red[q][t];
-            xs[r0 + t] = v;
-        }
-        __syncthreads();
-    }
-    for (int i = t; i < n; i += 1024) xc[i] = xs[i];
-}
-
-// Multi-work-group form for large n and few right-hand sides (one work-group streaming the whole
-// factor per right-hand side is bound by what one CU can read).  k_solve_perm applies the
-// interchange lists with the column in LDS (one work-group per rhs); then one k_trsv_step launch per
-// 64-row block and triangle.  Forward step b: work-group j takes row block r = b + 1 + j and
-// subtracts L_{r,b} x_b (x_b final from the previous launch); the group of r = b + 1 then finishes
-// x_r = Linv_r (its updated value).  Backward step b: row block r = b - 1 - j, U_{r,b} x_b, and the
-// group of r = b - 1 finishes x_r = Uinv_r (...).  The first launch of each triangle (b = -1 forward,
-// b = nblk backward) only finishes its first block.  Each off-diagonal block is read once per rhs:
-// 64 consecutive rows per column by each wave, 4 waves splitting the 64 columns.
-constexpr int kTrsvMinN = 1024;     // below this, one work-group per rhs is as fast
-constexpr int kTrsvMaxRhs = 256;    // rhs x matrices; more right-hand sides fill the device anyway
-
-template <typename T>
-__global__ __launch_bounds__(1024) void k_solve_perm(int n, const int32_t* __restrict__ pairs, T* __restrict__ x,
-                                                     int64_t ldx, int64_t sx) {
-    __shared__ T xs[kSolveMaxN];
+// perm[i]: the row of the right-hand side that all interchanges bring to row i (one work-group per matrix;
+// a block's list is in flight while the one before it is applied).  Pivots that a panel which gave up waiting
+// never wrote are skipped: perm stays within the matrix.
+__global__ __launch_bounds__(256) void k_solve_compose(int n, const int32_t* __restrict__ pairs,
+                                                       int32_t* __restrict__ perm) {
+    __shared__ int32_t s_i[kSolveMaxN];
     const int t = threadIdx.x;
     const int nblk = (n + kSB - 1) / kSB;
-    pairs += (int64_t)blockIdx.z * nblk * kSolvePairs;
-    T* xc = x + (int64_t)blockIdx.z * sx + (int64_t)blockIdx.x * ldx;
-    for (int i = t; i < n; i += 1024) xs[i] = xc[i];
+    pairs += (int64_t)blockIdx.x * nblk * kSolvePairs;
+    perm += (int64_t)blockIdx.x * n;
+    for (int i = t; i < n; i += 256) s_i[i] = i;
+    auto load = [&](int b, int& np, int& dst, int& src) {  // at most 2 kSB = 128 pairs, all initialised ones read
+        const int32_t* pl = pairs + (int64_t)b * kSolvePairs;
+        np = pl[0];
+        const int e = t < 2 * kSB ? t : 0;
+        dst = pl[1 + 2 * e];
+        src = pl[2 + 2 * e];
+    };
+    int np, dst, src;
+    load(0, np, dst, src);
     __syncthreads();
     for (int b = 0; b < nblk; b++) {
-        const int32_t* pl = pairs + (int64_t)b * kSolvePairs;
-        const int np = pl[0];
-        T v = T(0);
-        if (t < np) v = xs[pl[2 + 2 * t]];
+        int np1 = 0, dst1 = 0, src1 = 0;
+        if (b + 1 < nblk) load(b + 1, np1, dst1, src1);
+        int v = 0;
+        const bool mine = t < np && (unsigned)src < (unsigned)n && (unsigned)dst < (unsigned)n;
+        if (mine) v = s_i[src];
         __syncthreads();
-        if (t < np) xs[pl[1 + 2 * t]] = v;
+        if (mine) s_i[dst] = v;
         __syncthreads();
+        np = np1, dst = dst1, src = src1;
     }
-    for (int i = t; i < n; i += 1024) xc[i] = xs[i];
+    for (int i = t; i < n; i += 256) perm[i] = s_i[i];
 }
 
+// The triangular tiles of kSW rows that finish them: thread (r, g) = (t & 63, t >> 6) holds columns 4 g .. 4 g + 3
+// of row r, of the four diagonal blocks' inverses and of the off-diagonal tiles between them.
 template <typename T, bool LOWER>
-__global__ __launch_bounds__(256) void k_trsv_step(const T* __restrict__ a, int64_t lda, int n,
-                                                   const T* __restrict__ inv, T* __restrict__ x, int64_t ldx,
-                                                   int64_t sa, int64_t sx, int b) {
-    __shared__ T xb[kSB];
-    __shared__ T red[4][kSB];
+struct SolveTiles {
+    T iv[4][4], off[6][4];
+    static __device__ __forceinline__ constexpr int at(int q, int s) {  // index of tile (q, s), s before q
+        return LOWER ? q * (q - 1) / 2 + s : (3 - q) * (2 - q) / 2 + (3 - s);
+    }
+    // a: the matrix at the step's first row and column, nr rows left from there (past them the last row or
+    // column, or the first inverse, is read, and not used); inv: its blocks' inverses
+    __device__ __forceinline__ void load(const T* __restrict__ a, int64_t lda, int nr, const T* __restrict__ inv, int r,
+                                         int g) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+#pragma unroll
+            for (int p = 0; p < 4; p++)
+                iv[q][p] = (inv + (q * kSB < nr ? q : 0) * kSB * kSB + (4 * g + p) * kSB)[(unsigned)r];
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+                if (LOWER ? s < q : s > q) {
+                    const unsigned row = min(q * kSB + r, nr - 1);
+#pragma unroll
+                    for (int p = 0; p < 4; p++) off[at(q, s)][p] = (a + (int64_t)min(s * kSB + 4 * g + p, nr - 1) * lda)[row];
+                }
+        }
+    }
+    // Substitution in the step's rows: x = its right-hand side (LDS), replaced by the solution; acc[q]: what
+    // this thread's columns subtract from row q kSB + r already.  Rows past nr hold 0 and stay so.
+    __device__ __forceinline__ void solve(T* x, T (*red)[kSB], T* yb, T acc[4], int nr, int t) const {
+        const int r = t & 63, g = __builtin_amdgcn_readfirstlane(t >> 6);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int q = LOWER ? e : 3 - e;
+            if (q * kSB >= nr) continue;  // uniform over the work-group
+            red[g][r] = acc[q];
+            __syncthreads();
+            if (t < kSB) {
+                T y = x[q * kSB + t];
+#pragma unroll
+                for (int k = 0; k < 16; k++) y -= red[k][t];
+                yb[t] = q * kSB + t < nr ? y : T(0);
+            }
+            __syncthreads();
+            T s = T(0);
+#pragma unroll
+            for (int p = 0; p < 4; p++) s += iv[q][p] * yb[4 * g + p];
+            red[g][r] = s;
+            __syncthreads();
+            if (t < kSB) {
+                T v = T(0);
+#pragma unroll
+                for (int k = 0; k < 16; k++) v += red[k][t];
+                x[q * kSB + t] = q * kSB + t < nr ? v : T(0);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < 4; w++)
+                if (LOWER ? w > q : w < q)
+#pragma unroll
+                    for (int p = 0; p < 4; p++)
+                        if (q * kSB + 4 * g + p < nr) acc[w] += off[at(w, q)][p] * x[q * kSB + 4 * g + p];
+        }
+    }
+};
+
+// n <= kSW: one work-group per right-hand side, its column in LDS.
+// The whole chain is latency (8 dependent 64-row steps): the tiles are in registers before it starts.  256 rows,
+// 32 FP32 matrices: 11 us; a walk over 64-row steps that each read their own tiles took 21 us.
+template <typename T>
+__global__ __launch_bounds__(1024) void k_solve_small(const T* __restrict__ a, int64_t lda, int n,
+                                                      const int32_t* __restrict__ perm, const T* __restrict__ inv,
+                                                      T* __restrict__ x, int64_t ldx, int64_t sa, int64_t sx) {
+    __shared__ T xs[kSW];
+    __shared__ T red[16][kSB];
     __shared__ T yb[kSB];
-    const int t = threadIdx.x, rl = t & 63, g = t >> 6;
+    const int t = threadIdx.x, r = t & 63, g = __builtin_amdgcn_readfirstlane(t >> 6);
     const int nblk = (n + kSB - 1) / kSB;
+    a += (int64_t)blockIdx.z * sa;  // batch: one matrix per blockIdx.z
+    inv += (int64_t)blockIdx.z * 2 * nblk * kSB * kSB;
+    T* xc = x + (int64_t)blockIdx.z * sx + (int64_t)blockIdx.x * ldx;
+    SolveTiles<T, true> lo;
+    SolveTiles<T, false> up;
+    lo.load(a, lda, n, inv, r, g);
+    if (sizeof(T) == 4) up.load(a, lda, n, inv + (int64_t)nblk * kSB * kSB, r, g);
+    if (t < kSW) xs[t] = t < n ? xc[perm[(int64_t)blockIdx.z * n + t]] : T(0);
+    __syncthreads();
+    {
+        T acc[4] = {T(0), T(0), T(0), T(0)};
+        lo.solve(xs, red, yb, acc, n, t);
+    }
+    if (sizeof(T) == 8) up.load(a, lda, n, inv + (int64_t)nblk * kSB * kSB, r, g);
+    T acc[4] = {T(0), T(0), T(0), T(0)};
+    up.solve(xs, red, yb, acc, n, t);
+    if (t < n) xc[t] = xs[t];
+}
+
+// x = P x, one work-group per right-hand side
+template <typename T>
+__global__ __launch_bounds__(1024) void k_solve_perm(int n, const int32_t* __restrict__ perm, T* __restrict__ x,
+                                                     int64_t ldx, int64_t sx) {
+    __shared__ T xs[kSolveMaxN];
+    perm += (int64_t)blockIdx.z * n;
+    T* xc = x + (int64_t)blockIdx.z * sx + (int64_t)blockIdx.x * ldx;
+    for (int i = threadIdx.x; i < n; i += 1024) xs[i] = xc[i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += 1024) xc[i] = xs[perm[i]];
+}
+
+// Substitution step after the rows of step b (kSW rows, x_b final from the previous launch): work-group 0
+// subtracts their part from the next kSW rows in order and finishes these (SolveTiles); work-group j > 0
+// subtracts it from the j-th 64-row block beyond.  The first launch of a triangle (b = -1 forward, the number
+// of steps backward) only finishes its first rows.  Each off-diagonal tile is read once per right-hand side, 64
+// consecutive rows per column by each wave, 16 waves splitting the columns.
+// Bound by the chain of launches and, in work-group 0, of its four 64-row solves: all its tiles but the
+// inverse's products are read before the chain starts, and 256 rows per launch instead of 64 take a quarter of the
+// launches.  Both substitutions of one FP64 right-hand side at n = 4096: 1.04 -> 0.60 ms; FP32 at n = 16384,
+// 2 matrices: 5.3 -> 1.9 ms.
+template <typename T, bool LOWER>
+__global__ __launch_bounds__(1024) void k_trsv_step(const T* __restrict__ a, int64_t lda, int n,
+                                                    const T* __restrict__ inv, T* __restrict__ x, int64_t ldx,
+                                                    int64_t sa, int64_t sx, int b) {
+    __shared__ T xb[kSW];
+    __shared__ T xn[kSW];
+    __shared__ T red[16][kSB];
+    __shared__ T yb[kSB];
+    const int t = threadIdx.x, r = t & 63, g = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nblk = (n + kSB - 1) / kSB, nst = (n + kSW - 1) / kSW;
     a += (int64_t)blockIdx.z * sa;
     inv += (int64_t)blockIdx.z * 2 * nblk * kSB * kSB + (LOWER ? 0 : (int64_t)nblk * kSB * kSB);
     T* xc = x + (int64_t)blockIdx.z * sx + (int64_t)blockIdx.y * ldx;
-    const int j = blockIdx.x;
-    const int r = LOWER ? b + 1 + j : b - 1 - j;  // this group's row block
-    const int r0 = r * kSB, c0 = b * kSB;
-    const bool has_b = LOWER ? b >= 0 : b < nblk;
-    T y = T(0);
-    if (t < kSB) y = r0 + t < n ? xc[r0 + t] : T(0);
-    if (has_b) {
-        if (t < kSB) xb[t] = c0 + t < n ? xc[c0 + t] : T(0);
+    const int c0 = b * kSW;
+    const bool has_b = LOWER ? b >= 0 : b < nst;
+    const int cols = has_b ? min(kSW, n - c0) : 0;
+    // sum over this thread's 16 columns of step b in row `row` (past the matrix: its last row or column is read, and
+    // not used)
+    auto part = [&](int row) {
+        const unsigned at = min(row, n - 1);
+        T m[16];
+#pragma unroll
+        for (int c = 0; c < 16; c++) m[c] = (a + (int64_t)min(c0 + 16 * g + c, n - 1) * lda)[at];
+        T s = T(0);
+#pragma unroll
+        for (int c = 0; c < 16; c++) s += 16 * g + c < cols ? m[c] * xb[16 * g + c] : T(0);
+        return s;
+    };
+    if (has_b && t < kSW) xb[t] = t < cols ? xc[c0 + t] : T(0);
+    if (blockIdx.x > 0) {
+        const int j = blockIdx.x - 1;
+        const int r0 = LOWER ? (b + 2) * kSW + j * kSB : (b - 1) * kSW - (j + 1) * kSB;
+        const T y = t < kSB && r0 + t < n ? xc[r0 + t] : T(0);
         __syncthreads();
-        T acc = T(0);
-        if (r0 + rl < n) {
-            const T* ab = a + (r0 + rl) + (int64_t)c0 * lda;
-#pragma unroll 4
-            for (int c = 16 * g; c < 16 * g + 16; c++)
-                if (c0 + c < n) acc += ab[(int64_t)c * lda] * xb[c];
+        red[g][r] = part(r0 + r);
+        __syncthreads();
+        if (t < kSB && r0 + t < n) {
+            T s = y;
+#pragma unroll
+            for (int k = 0; k < 16; k++) s -= red[k][t];
+            xc[r0 + t] = s;
         }
-        red[g][rl] = acc;
-        __syncthreads();
-        if (t < kSB) y -= red[0][t] + red[1][t] + red[2][t] + red[3][t];
-    }
-    if (j != 0) {  // a later block: store the partial update
-        if (t < kSB && r0 + t < n) xc[r0 + t] = y;
         return;
     }
-    // the next block in order: finish it with its diagonal-block inverse
-    if (t < kSB) yb[t] = y;
+    const int w = LOWER ? b + 1 : b - 1, r0 = w * kSW, nr = n - r0;
+    SolveTiles<T, LOWER> tiles;
+    if (sizeof(T) == 4) tiles.load(a + r0 + (int64_t)r0 * lda, lda, nr, inv + (int64_t)w * 4 * kSB * kSB, r, g);
+    if (t < kSW) xn[t] = t < nr ? xc[r0 + t] : T(0);
     __syncthreads();
-    const T* ib = inv + (int64_t)r * kSB * kSB;
-    T s = T(0);
+    T acc[4] = {T(0), T(0), T(0), T(0)};
+    if (has_b)
 #pragma unroll
-    for (int p = 16 * g; p < 16 * g + 16; p++) s += ib[rl + p * kSB] * yb[p];
-    red[g][rl] = s;
-    __syncthreads();
-    if (t < kSB && r0 + t < n) xc[r0 + t] = red[0][t] + red[1][t] + red[2][t] + red[3][t];
+        for (int q = 0; q < 4; q++) {
+            acc[q] = part(r0 + q * kSB + r);
+            __builtin_amdgcn_sched_barrier(0);  // 16 loads in flight beside the tiles: 128 registers hold no more
+        }
+    if (sizeof(T) == 8) tiles.load(a + r0 + (int64_t)r0 * lda, lda, nr, inv + (int64_t)w * 4 * kSB * kSB, r, g);
+    tiles.solve(xn, red, yb, acc, nr, t);
+    if (t < min(kSW, nr)) xc[r0 + t] = xn[t];
 }
 
-// shape[2] > 1 solves a batch: matrix b at A.ptr + b A.stride[2] with pivots ipiv + b n, its
-// right-hand sides at X.ptr + b X.stride[2].
+// X_b = inv X_b for the 64 rows of a diagonal block (rb of them in the matrix) and all right-hand sides, a wave
+// per 16 of them, on the matrix cores
 template <typename T>
-int getrs(const tvlm_view* av, const int32_t* ipiv, const tvlm_view* xv, void* stream) {
+__global__ __launch_bounds__(256) void k_inv_apply(const T* __restrict__ inv, T* __restrict__ x, int64_t ldx, int rb,
+                                                   int nrhs) {
+    using M = Mf16<T>;
+    typedef typename M::vacc vacc;
+    const int lane = threadIdx.x & 63, m = lane & 15;
+    const int j = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16 + m;
+    T* xc = x + (int64_t)min(j, nrhs - 1) * ldx;
+    T q[4][4];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int row = 16 * k + M::k(lane, r);
+            q[k][r] = row < rb ? xc[row] : T(0);
+        }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        vacc y = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) y = M::mfma(inv[16 * i + m + (16 * k + M::k(lane, r)) * kSB], q[k][r], y);
+        if (j < nrhs)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int row = 16 * i + M::k(lane, r);
+                if (row < rb) xc[row] = y[r];
+            }
+    }
+}
+
+// Right-hand sides times rows from which the substitutions run as products over all right-hand sides.  Below,
+// a step per 256 rows and right-hand side is faster; 256 rhs of 2000 FP64 rows take 1.16 ms so (products:
+// 1.3), 512 2.06 ms (1.39), 64 of 8192 rows 6.1 ms (5.7), 1024 of 600 rows 0.49 ms (0.42).
+constexpr int64_t kManyRhs = 512 * 1024;
+
+// What getrs makes of the factors before it sees a right-hand side: inverses of the diagonal blocks, the
+// composed interchanges, and the lists they come from.
+template <typename T>
+struct SolvePrep {
+    T* inv;
+    int32_t *perm, *pairs;
+    static bool covers(int64_t n) { return n <= kSolveMaxN; }
+    static size_t bytes(int n, int batch) {
+        const size_t nblk = (n + kSB - 1) / kSB;
+        return (sizeof(T) * 2 * nblk * kSB * kSB + sizeof(int32_t) * (n + nblk * kSolvePairs)) * batch;
+    }
+    void place(void* ws, int n, int batch) {
+        const size_t nblk = (n + kSB - 1) / kSB;
+        inv = static_cast<T*>(ws);
+        perm = reinterpret_cast<int32_t*>(inv + 2 * nblk * kSB * kSB * batch);
+        pairs = perm + (size_t)n * batch;
+    }
+    int make(const T* a, int64_t lda, int n, int64_t sa, int batch, const int32_t* ipiv, hipStream_t st) const {
+        const int nblk = (n + kSB - 1) / kSB;
+        hipLaunchKernelGGL(k_solve_prep<T>, dim3(nblk, 3, batch), dim3(256), 0, st, a, lda, n, ipiv, pairs, inv, sa);
+        TVLM_LAUNCHED();
+        hipLaunchKernelGGL(k_solve_compose, dim3(batch), dim3(256), 0, st, n, pairs, perm);
+        TVLM_LAUNCHED();
+        return TVLM_OK;
+    }
+    int solve(const T* a, int64_t lda, int n, int64_t sa, int batch, T* x, int64_t ldx, int64_t sx, int nrhs,
+              hipStream_t st) const {
+        if (n <= kSW) {
+            hipLaunchKernelGGL(k_solve_small<T>, dim3(nrhs, 1, batch), dim3(1024), 0, st, a, lda, n, perm, inv, x, ldx,
+                               sa, sx);
+            TVLM_LAUNCHED();
+            return TVLM_OK;
+        }
+        hipLaunchKernelGGL(k_solve_perm<T>, dim3(nrhs, 1, batch), dim3(1024), 0, st, n, perm, x, ldx, sx);
+        TVLM_LAUNCHED();
+        const int nblk = (n + kSB - 1) / kSB, nst = (n + kSW - 1) / kSW;
+        if ((int64_t)nrhs * n >= kManyRhs && lda < kUpdMaxLd && ldx < kUpdMaxLd) {
+            for (int z = 0; z < batch; z++) {
+                const T* az = a + (int64_t)z * sa;
+                const T* iz = inv + (int64_t)z * 2 * nblk * kSB * kSB;
+                T* xz = x + (int64_t)z * sx;
+                auto finish = [&](int b, int tri) {
+                    hipLaunchKernelGGL(k_inv_apply<T>, dim3((nrhs + 63) / 64), dim3(256), 0, st,
+                                       iz + ((int64_t)tri * nblk + b) * kSB * kSB, xz + b * kSB, ldx,
+                                       n - b * kSB < kSB ? n - b * kSB : kSB, nrhs);
+                };
+                for (int b = 0; b < nblk; b++) {
+                    const int c0 = b * kSB, r0 = c0 + kSB;
+                    finish(b, 0);
+                    TVLM_LAUNCHED();
+                    launch_update<T>(xz + r0, ldx, az + r0 + (int64_t)c0 * lda, lda, xz + c0, ldx, n - r0, nrhs, kSB, 0, 1,
+                                     st);
+                    TVLM_LAUNCHED();
+                }
+                for (int b = nblk - 1; b >= 0; b--) {
+                    const int c0 = b * kSB;
+                    finish(b, 1);
+                    TVLM_LAUNCHED();
+                    launch_update<T>(xz, ldx, az + (int64_t)c0 * lda, lda, xz + c0, ldx, c0, nrhs,
+                                     n - c0 < kSB ? n - c0 : kSB, 0, 1, st);
+                    TVLM_LAUNCHED();
+                }
+            }
+            return TVLM_OK;
+        }
+        for (int b = -1; b < nst - 1; b++) {
+            const int beyond = b < 0 ? 0 : nblk - 4 * (b + 2);
+            hipLaunchKernelGGL((k_trsv_step<T, true>), dim3(1 + (beyond > 0 ? beyond : 0), nrhs, batch), dim3(1024), 0, st,
+                               a, lda, n, inv, x, ldx, sa, sx, b);
+            TVLM_LAUNCHED();
+        }
+        for (int b = nst; b > 0; b--) {
+            const int beyond = b == nst ? 0 : 4 * (b - 1);
+            hipLaunchKernelGGL((k_trsv_step<T, false>), dim3(1 + beyond, nrhs, batch), dim3(1024), 0, st, a, lda, n, inv, x,
+                               ldx, sa, sx, b);
+            TVLM_LAUNCHED();
+        }
+        return TVLM_OK;
+    }
+};
+
+// shape[2] > 1 solves a batch: matrix b at A.ptr + b A.stride[2] with pivots ipiv + b n, its
+// right-hand sides at X.ptr + b X.stride[2].  prepared: the batch's SolvePrep, made from these factors.
+template <typename T>
+int getrs(const tvlm_view* av, const int32_t* ipiv, const tvlm_view* xv, void* stream, void* prepared = nullptr) {
     TVLM_REQUIRE(av && xv && av->ptr && xv->ptr && ipiv, "null argument");
     TVLM_REQUIRE(av->stride[0] == 1 && xv->stride[0] == 1, "column-major operands required");
     const int n = (int)av->shape[0];
@@ -2488,36 +2687,13 @@ int getrs(const tvlm_view* av, const int32_t* ipiv, const tvlm_view* xv, void* s
     hipStream_t st = as_stream(stream);
     const T* a = static_cast<const T*>(av->ptr);
     T* x = static_cast<T*>(xv->ptr);
-    if (n <= kSolveMaxN && (int64_t)n * sizeof(T) <= 128 * 1024) {
-        const int nblk = (n + kSB - 1) / kSB;
-        void* ws = nullptr;
-        const size_t inv_bytes = sizeof(T) * 2 * (size_t)nblk * kSB * kSB * batch;
-        TVLM_TRY(device_workspace(inv_bytes + sizeof(int32_t) * (size_t)nblk * kSolvePairs * batch, &ws, kWsSolveInv, st));
-        T* inv = static_cast<T*>(ws);
-        int32_t* pairs = reinterpret_cast<int32_t*>(static_cast<char*>(ws) + inv_bytes);
-        hipLaunchKernelGGL(k_solve_prep<T>, dim3(nblk, 3, batch), dim3(256), 0, st, a, lda, n, ipiv, pairs, inv, sa);
-        TVLM_LAUNCHED();
-        if (n < kTrsvMinN || (int64_t)nrhs * batch > kTrsvMaxRhs) {
-            hipLaunchKernelGGL(k_solve_blocked<T>, dim3(nrhs, 1, batch), dim3(1024), 0, st, a, lda, n, pairs, inv, x,
-                               ldx, sa, sx);
-            TVLM_LAUNCHED();
-            return TVLM_OK;
-        }
-        hipLaunchKernelGGL(k_solve_perm<T>, dim3(nrhs, 1, batch), dim3(1024), 0, st, n, pairs, x, ldx, sx);
-        TVLM_LAUNCHED();
-        for (int b = -1; b < nblk - 1; b++) {
-            const int groups = b < 0 ? 1 : nblk - 1 - b;
-            hipLaunchKernelGGL((k_trsv_step<T, true>), dim3(groups, nrhs, batch), dim3(256), 0, st, a, lda, n, inv, x,
-                               ldx, sa, sx, b);
-            TVLM_LAUNCHED();
-        }
-        for (int b = nblk; b > 0; b--) {
-            const int groups = b == nblk ? 1 : b;
-            hipLaunchKernelGGL((k_trsv_step<T, false>), dim3(groups, nrhs, batch), dim3(256), 0, st, a, lda, n, inv, x,
-                               ldx, sa, sx, b);
-            TVLM_LAUNCHED();
-        }
-        return TVLM_OK;
+    if (SolvePrep<T>::covers(n)) {
+        SolvePrep<T> P;
+        void* ws = prepared;
+        if (!ws) TVLM_TRY(device_workspace(SolvePrep<T>::bytes(n, batch), &ws, kWsSolveInv, st));
+        P.place(ws, n, batch);
+        if (!prepared) TVLM_TRY(P.make(a, lda, n, sa, batch, ipiv, st));
+        return P.solve(a, lda, n, sa, batch, x, ldx, sx, nrhs, st);
     }
     for (int z = 0; z < batch; z++) {
         const T* az = a + (int64_t)z * sa;
@@ -2577,6 +2753,20 @@ int getrf_single_group_f64(const tvlm_view* a, int32_t* ipiv, int32_t* info, voi
 }
 int getrf_single_group_f32(const tvlm_view* a, int32_t* ipiv, int32_t* info, void* stream) {
     return getrf<float>(a, ipiv, info, stream, false);
+}
+
+size_t getrs_prep_bytes_f32(int64_t n, int batch) {
+    return SolvePrep<float>::covers(n) ? SolvePrep<float>::bytes((int)n, batch) : 0;
+}
+int getrs_prepare_f32(const tvlm_view* a, const int32_t* ipiv, void* prep, hipStream_t st) {
+    if (!prep) return TVLM_OK;
+    SolvePrep<float> P;
+    P.place(prep, (int)a->shape[0], (int)a->shape[2]);
+    return P.make(static_cast<const float*>(a->ptr), a->stride[1], (int)a->shape[0], a->stride[2], (int)a->shape[2], ipiv,
+                  st);
+}
+int getrs_prepared_f32(const tvlm_view* a, const int32_t* ipiv, void* prep, const tvlm_view* x, hipStream_t st) {
+    return getrs<float>(a, ipiv, x, st, prep);
 }
 
 }  // namespace tvlm

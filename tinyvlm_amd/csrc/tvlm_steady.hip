@@ -53,6 +53,7 @@ struct tvlm_vlm_plan {
     double* par = nullptr;  // per request: 16 n_surf transform values, then kPar values (tvlm_vlm_solve_n)
     float *lhs32 = nullptr, *r32 = nullptr;
     int32_t *ipiv = nullptr, *info = nullptr;
+    void* prep = nullptr;  // served mode: what getrs derives from the factors, once for all corrections
     double *rowabs = nullptr, *berr = nullptr;  // served mode: row sums of |A64|, backward error per request
     int32_t* conv = nullptr;                     // served mode: 1 = the request's x passed the test
     std::vector<int32_t> st_status, st_corr;     // per request of the last solve (tvlm_vlm_refinement)
@@ -526,7 +527,11 @@ int tvlm_vlm_create(tvlm_vlm_plan** plan, int32_t n_surf, const int64_t* ns, con
         if (rc == TVLM_OK) rc = tvlm_copy(0, P->init[m], 1, 1, verts_init[m], 1, sizeof(double), P->vsz[m], stream);
     }
     if (rc == TVLM_OK) rc = P->alloc((void**)&P->lhs, sizeof(double) * NN * nb);
-    if (rc == TVLM_OK && mode == 1) rc = P->alloc((void**)&P->lhs32, sizeof(float) * NN * nb);
+    if (rc == TVLM_OK && mode == 1) {  // prep stands behind lhs32 (an allocation of its own takes 0.1 ms)
+        const size_t prep = getrs_prep_bytes_f32(N, batch), at = (sizeof(float) * NN * nb + 255) / 256 * 256;
+        rc = P->alloc((void**)&P->lhs32, at + prep);
+        if (rc == TVLM_OK && prep) P->prep = reinterpret_cast<char*>(P->lhs32) + at;
+    }
     if (rc == TVLM_OK && mode == 1) rc = P->alloc((void**)&P->r32, sizeof(float) * N * batch);
     if (rc == TVLM_OK && mode == 1) rc = P->alloc((void**)&P->res, sizeof(double) * N * batch);
     if (rc == TVLM_OK && mode == 1) rc = P->alloc((void**)&P->rowabs, sizeof(double) * N * batch);
@@ -625,6 +630,7 @@ int tvlm_vlm_solve_n(tvlm_vlm_plan* P, int32_t n_active, const double* alpha, co
         TVLM_TRY(lhs_group_assign_seeded(P->group, B, P->lhs, P->lhs32, st));
         tvlm_view L32 = {P->lhs32, {N, N, B}, {1, N, NN}};
         TVLM_TRY(tvlm_getrf_f32(&L32, P->ipiv, P->info, st));
+        TVLM_TRY(getrs_prepare_f32(&L32, P->ipiv, P->prep, st));
         tvlm_view R32 = {P->r32, {N, 1, B}, {1, N, N}};
         // x = 0, r = b; then kRefine + 1 corrections x += A32^{-1} r, r = b - A64 x
         TVLM_TRY(tvlm_fill_f64(0, P->x, 1, 0.0, N * B, st));
@@ -643,7 +649,7 @@ int tvlm_vlm_solve_n(tvlm_vlm_plan* P, int32_t n_active, const double* alpha, co
                 hipLaunchKernelGGL(k_to_f32, dim3(grid_for(N * B)), dim3(256), 0, st, P->res, P->r32, N * B);
             }
             TVLM_LAUNCHED();
-            TVLM_TRY(tvlm_getrs_f32(&L32, P->ipiv, &R32, st));
+            TVLM_TRY(getrs_prepared_f32(&L32, P->ipiv, P->prep, &R32, st));
             hipLaunchKernelGGL(k_add_f32, dim3(grid_for(N * B)), dim3(256), 0, st, P->x, P->r32, N * B);
             TVLM_LAUNCHED();
         }
