@@ -23,7 +23,8 @@ Structure
   with copies of its first motion, whose results are dropped.
 - admission: whenever a lane is free, the queue (steady: per mesh; unsteady: per mesh) whose oldest
   waiting request arrived first is served: for steady requests an idle plan of that mesh (or a new
-  one) takes up to its cap of that mesh's waiting requests, in arrival order.  Requests that arrive
+  one, if the mesh has none or at least two of its requests wait) takes up to its cap of that mesh's
+  waiting requests, in arrival order.  Requests that arrive
   while others are on the device are admitted as soon as a lane and a plan (memory) are free,
   whatever else is running.
 
@@ -525,6 +526,11 @@ class Server:
                     if kind == "unsteady":
                         slot = self._uslot_for(mesh, free_lanes[0], now, self.usims(len(waiting[k])))
                     else:
+                        # A lone request waits for its mesh's running plan: a further plan takes milliseconds
+                        # to create, during which nothing else is admitted, about as long as the running
+                        # solve (72 requests on 4 lanes, 0.6 ms apart: mean latency 9.1 -> 7.4 ms).
+                        if len(waiting[k]) < 2 and self.slots[mesh] and all(s.busy for s in self.slots[mesh]):
+                            continue
                         slot = self._slot_for(mesh, free_lanes[0], now)
                     if slot is not None:
                         chosen = (k, slot)
