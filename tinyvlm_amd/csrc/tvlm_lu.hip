@@ -1987,13 +1987,14 @@ int defer_gather(T* a, int64_t lda, int n, int batch, int64_t sb, const int32_t*
     return TVLM_OK;
 }
 
-// Factorisations whose tall panels are cooperative (all panels NB wide), taken two panels at a
-// time so that the trailing matrix is read and written once per pair: panel A at kp, its
-// interchanges and U12 (k_swap_trsm, mode 0); panel B's columns updated by panel A, panel B; panel
-// B's interchanges on both sides (mode 1); the rows of panel B right of it updated by panel A (one
-// NB-row GEMM); panel B's U12 (mode 2); one rank-2NB update of the trailing matrix.  The same
-// products as one panel at a time, summed in a different order.
-constexpr int kPairMinRows = 6144;  // trailing matrices at least this tall are updated once per pair
+// Factorisations whose tall panels are cooperative (all panels NB wide), taken kGroupPanels panels at a
+// time so that the trailing matrix is read and written once per group.  For each panel of a group: its
+// columns updated by the group's earlier panels, the panel, its interchanges on both sides (mode 1; the
+// group's first: and U12, mode 0), its rows right of it updated by the group's earlier panels, its U12
+// (mode 2); then one update of the trailing matrix by the whole group.  The same products as one panel
+// at a time, summed in a different order.
+constexpr int kGroupPanels = 4;
+constexpr int kGroupMinRows = 3072;  // trailing matrices at least this tall are updated once per group
 
 // ---- the factorisation plan -------------------------------------------------------------------
 // Which path a getrf call takes and, for the cooperative path, every panel's form and exchange
@@ -2090,28 +2091,29 @@ int getrf_coop_pairs(T* a, int64_t lda, int n, int batch, int64_t sb, int32_t* i
     };
     auto at = [&](int r, int c) { return a + r + (int64_t)c * lda; };
     for (int kp = 0; kp < n;) {
-        const int kbA = n - kp < NB ? n - kp : NB, jA = kp + kbA;
-        TVLM_TRY(panel(kp, kbA));
-        TVLM_TRY(swap_trsm(kp, kbA, 0, kp));
-        if (jA >= n) break;
-        if (n - jA < kPairMinRows) {  // the trailing matrix stays in the last-level cache: one panel at a time
-            launch_update<T>(at(jA, jA), lda, at(jA, kp), lda, at(kp, jA), lda, n - jA, n - jA, kbA, sb, batch, st);
-            TVLM_LAUNCHED();
-            kp = jA;
-            continue;
+        // a trailing matrix below kGroupMinRows stays in the last-level cache: one panel at a time
+        const int last = kp + NB < n && n - kp - NB >= kGroupMinRows ? kp + kGroupPanels * NB : kp + NB;
+        int c = kp;
+        while (c < last && c < n) {
+            const int kb = n - c < NB ? n - c : NB, j1 = c + kb, r = c - kp;  // r: rank of the group's panels so far
+            if (r) {
+                launch_update<T>(at(c, c), lda, at(c, kp), lda, at(kp, c), lda, n - c, kb, r, sb, batch, st);
+                TVLM_LAUNCHED();
+            }
+            TVLM_TRY(panel(c, kb));
+            TVLM_TRY(swap_trsm(c, kb, r ? 1 : 0, kp));
+            if (r && j1 < n) {
+                launch_update<T>(at(c, j1), lda, at(c, kp), lda, at(kp, j1), lda, kb, n - j1, r, sb, batch, st);
+                TVLM_LAUNCHED();
+                TVLM_TRY(swap_trsm(c, kb, 2, c));
+            }
+            c = j1;
         }
-        const int kbB = n - jA < NB ? n - jA : NB, jB = jA + kbB;
-        launch_update<T>(at(jA, jA), lda, at(jA, kp), lda, at(kp, jA), lda, n - jA, kbB, kbA, sb, batch, st);
-        TVLM_LAUNCHED();
-        TVLM_TRY(panel(jA, kbB));
-        TVLM_TRY(swap_trsm(jA, kbB, 1, kp));
-        if (jB >= n) break;
-        launch_update<T>(at(jA, jB), lda, at(jA, kp), lda, at(kp, jB), lda, kbB, n - jB, kbA, sb, batch, st);
-        TVLM_LAUNCHED();
-        TVLM_TRY(swap_trsm(jA, kbB, 2, jA));
-        launch_update<T>(at(jB, jB), lda, at(jB, kp), lda, at(kp, jB), lda, n - jB, n - jB, kbA + kbB, sb, batch, st);
-        TVLM_LAUNCHED();
-        kp = jB;
+        if (c < n) {
+            launch_update<T>(at(c, c), lda, at(c, kp), lda, at(kp, c), lda, n - c, n - c, c - kp, sb, batch, st);
+            TVLM_LAUNCHED();
+        }
+        kp = c;
     }
     TVLM_TRY(defer_gather<T>(a, lda, n, batch, sb, gtab, st));
     hipLaunchKernelGGL(k_coop_fail_info, dim3((batch + 255) / 256), dim3(256), 0, st, fail, info, batch);
@@ -2583,8 +2585,9 @@ __global__ __launch_bounds__(256) void k_inv_apply(const T* __restrict__ inv, T*
 }
 
 // Right-hand sides times rows from which the substitutions run as products over all right-hand sides.  Below,
-// a step per 256 rows and right-hand side is faster; 256 rhs of 2000 FP64 rows take 1.16 ms so (products:
-// 1.3), 512 2.06 ms (1.39), 64 of 8192 rows 6.1 ms (5.7), 1024 of 600 rows 0.49 ms (0.42).
+// a step per 256 rows and right-hand side is faster or equal.  At the line, steps and products: 128 rhs of 4096
+// FP64 rows 2.80 and 2.64 ms (FP32 1.69 and 1.95), 64 of 8192 rows 6.1 and 5.7 ms (3.86 and 3.89), 1024 of 600 rows
+// 0.49 and 0.42 ms (0.31 and 0.33); at twice that, 256 of 4096 rows, 4.9 and 2.7 ms (3.0 and 2.0).
 constexpr int64_t kManyRhs = 512 * 1024;
 
 // What getrs makes of the factors before it sees a right-hand side: inverses of the diagonal blocks, the
