@@ -4,7 +4,7 @@ tunables here).
 Two knobs set how the wake induction is tiled into work-groups:
 - the lattice work-group target of a fast-mode UVLM plan (tvlm_uvlm_set_lattice_target; library
   default 1024): above it a launch takes 2 or 4 wake rows per tile, below it the spans are split;
-- the ring-by-ring form's target (tvlm_set_tile_targets, default 2048) for
+- the Backend form's target (tvlm_set_tile_targets, default 2048) for
   Backend::rhs_assemble_wake_influence and the plain UVLM loop.
 
 The tuner times each candidate on the caller's own workload (whole simulations replayed from the
@@ -125,7 +125,7 @@ def set_targets(wake_groups: int = 0, lattice_groups: int = 0):
 def tune_wake_influence(rhs, gamma_wake, colloc, normals, verts_wake, lifting, iteration,
                         candidates=WAKE_CANDIDATES, cache: Cache | None = None, reps: int = 5,
                         force: bool = False) -> dict:
-    """Picks the library-wide target of the ring-by-ring wake induction for this call's shape (the
+    """Picks the library-wide target of the Backend wake induction for this call's shape (the
     receivers, wake surfaces and rows of `iteration`) by timing Backend::rhs_assemble_wake_influence
     between HIP events; rhs is restored after timing.  Sets the target (keeping the lattice one)."""
     import torch

@@ -85,7 +85,7 @@ int getrs_prepared_f32(const tvlm_view* a, const int32_t* ipiv, void* prep, cons
 constexpr int32_t kGetrfStalled = -999;  // info of a matrix whose cooperative panel gave up waiting
 
 // Work-group targets of the wake-induction launches, library-wide (tvlm_set_tile_targets): the
-// ring-by-ring form's tile shape (wake_tile_shape) and new UVLM plans' lattice launches.
+// Backend form's tile shape (wake_tile_shape) and new UVLM plans' lattice launches.
 constexpr int kTargetGroups = 2048;     // default of wake_target_groups()
 constexpr int kLatTargetGroups = 1024;  // default of lattice_target_groups()
 int wake_target_groups();
