@@ -80,10 +80,10 @@ COPY_PROBE_BYTES = 1 << 30
 # y-free terms and the 1/(4 pi) factor moved out of the segment loop (the traffic passes precede
 # those changes, which moved no memory access).
 WAKE_COUNTERS = {
-    "exact": {"traffic_bytes": 3008144, "algorithmic_bytes": 349384, "executed_flops_per_pair": 237.9},
-    "far": {"traffic_bytes": 2465922, "algorithmic_bytes": 188327, "executed_flops_per_pair": 284.9},
-    "far_sims64": {"traffic_bytes": 121996697, "algorithmic_bytes": 12052939, "executed_flops_per_pair": 226.0},
-    "exact_sims64": {"traffic_bytes": 174869909, "algorithmic_bytes": 22360576, "executed_flops_per_pair": 222.7},
+    "exact": {"traffic_bytes": 3008144, "algorithmic_bytes": 349384, "executed_flops_per_pair": 218.8},
+    "far": {"traffic_bytes": 2465922, "algorithmic_bytes": 188327, "executed_flops_per_pair": 263.8},
+    "far_sims64": {"traffic_bytes": 121996697, "algorithmic_bytes": 12052939, "executed_flops_per_pair": 207.7},
+    "exact_sims64": {"traffic_bytes": 174869909, "algorithmic_bytes": 22360576, "executed_flops_per_pair": 204.4},
 }
 NS, NC, HALF_SPAN, CHORD = 40, 10, 2.0, 1.0
 T_STEPS = 501  # UVLM::run loops t_steps-1 times -> 500 time steps
