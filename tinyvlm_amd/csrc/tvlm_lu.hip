@@ -286,8 +286,11 @@ __device__ int wave_compose_swaps(int first, int cnt, const int* piv, int* pd, i
 //
 // Every work-group factors the candidates for itself (a 64-step chain in registers and LDS: one
 // launch and no exchange) and then takes its share of the other rows, 16 per wave and step on the
-// matrix cores: with Y = L21^T, 16 columns of the panel at a time, Y_b = Uinv_bb^T (A_b^T - sum_{c<b}
-// U_cb^T Y_c) (Uinv_bb: inverse of the 16 x 16 diagonal block).  The MFMA output layout is the
+// matrix cores: with Y = L21^T, 16 columns of the panel at a time, R_b = A_b^T - sum_{c<b} U_cb^T Y_c and
+// Y_b = Uinv_bb^T R_b (Uinv_bb: inverse of the 16 x 16 diagonal block), then corrected once, Y_b += Uinv_bb^T
+// (R_b - U_bb^T Y_b).  Without the correction the error of Y_b grows with the condition of U_bb (1e8: 1e-11 of the
+// matrix in FP64), while its multipliers stay below 1; with it the factors are as accurate as column by column
+// up to spec_condition_limit, past which the round fails.  The MFMA output layout is the
 // second operand's layout, so the blocks chain without moving between lanes.  What bounds it is the
 // candidates' chain, 64 dependent pivot steps.  Per 4096-row FP64 panel of one matrix, round 1 takes 21 us
 // (loads 2.3, chain 12.8, inverses and staging 2.8, rows 2.9; FP32 17 us) and a later round 52 us (its
@@ -500,6 +503,21 @@ struct SpecChain {
     }
 };
 
+// Row ln of |X| |U| summed (X = U^{-1}, a row of each per lane, in every row of 16 lanes): what an explicit
+// inverse multiplies the rounding of the product by.
+template <typename T, int... J>
+__device__ __forceinline__ T spec_condition(const T (&x)[16], const T (&u)[16], int ln, std::integer_sequence<int, J...>) {
+    T rows = T(0), sum = T(0);
+#pragma unroll
+    for (int i = 0; i < 16; i++) rows += i >= ln ? (T)fabs(u[i]) : T(0);
+    ((sum += (T)fabs(x[J]) * row_value<J>(rows)), ...);
+    return sum;
+}
+// Largest such sum of a panel that may stand: the correction below leaves (eps cond)^2 of it, which is below
+// eps up to here.  Wings stay far below (elliptic 12 x 100: 350, 64 x 64: 35).
+__device__ __forceinline__ double spec_condition_limit(double) { return 0x1p22; }
+__device__ __forceinline__ float spec_condition_limit(float) { return 0x1p9f; }
+
 // R rows per lane: 64 R candidates.  Grid (x: shares of the rows, z: matrices), 256 threads.
 template <typename T, int R>
 __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t lda, int n, int k0, int kb,
@@ -528,7 +546,7 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
     __shared__ int s_row[64 * R];    // candidate -> row (relative to k0), -1: none
     __shared__ int s_pos[64 * R];    // candidate -> final row (candidates that became no pivot)
     __shared__ uint32_t s_cmap[R == 2 ? kSpecMaxRows / 32 : 1];  // rows that are candidates below the diagonal block
-    __shared__ int s_bad;
+    __shared__ int s_bad, s_ill;
     // candidates: the diagonal rows, from round 2 on also rows of the earlier rounds' keys
     int crow = -1;  // row of candidate 64 + lane
     if constexpr (R == 2) {
@@ -560,7 +578,7 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
     if (t < 64) {
         s_row[lane] = lane < kb ? lane : -1;
         if constexpr (R == 2) s_row[64 + lane] = crow;
-        if (lane == 0) s_bad = 0;
+        if (lane == 0) s_bad = s_ill = 0;
     }
     __syncthreads();
     if constexpr (R == 2)
@@ -831,8 +849,14 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
         if (lane < 16)
 #pragma unroll
             for (int i = 0; i < 16; i++) sInv[g][ln][i] = s[i];
+        const T cond = spec_condition(s, rt, ln, std::make_integer_sequence<int, 16>{});
+        if (__ballot(!(cond <= spec_condition_limit(T(0)))) != 0ull && lane == 0) s_ill = 1;
     }
     __syncthreads();
+    if (s_ill != 0) {  // the rows' multipliers would not be accurate
+        if (t == 0) *fail = 1;
+        return;
+    }
     // the other rows, 16 per wave and step
     const T one = T(1), strict = R == 2 ? T(1) - T(64) * (sizeof(T) == 8 ? (T)2.2e-16 : (T)1.2e-7f) : T(1);
     bool failed = false;
@@ -849,6 +873,14 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
                 for (int r = 0; r < 4; r++)
                     y[b] = M::mfma(sU[16 * c + M::k(lane, r)][16 * b + ln], y[c][r], y[b]);
             typename M::vacc s = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+            for (int r = 0; r < 4; r++) s = M::mfma(sInv[b][M::k(lane, r)][ln], y[b][r], s);
+            // s += Uinv_bb^T (y_b - U_bb^T s)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int k = M::k(lane, r);
+                y[b] = M::mfma(k <= ln ? sU[16 * b + k][16 * b + ln] : T(0), s[r], y[b]);
+            }
 #pragma unroll
             for (int r = 0; r < 4; r++) s = M::mfma(sInv[b][M::k(lane, r)][ln], y[b][r], s);
             y[b] = s;
