@@ -50,3 +50,24 @@ def test_nearly_dependent_columns(n, batch, npdt, gap):
     for A, lu, piv, inf in zip(As, lus, pivs, info):
         assert inf == 0 and np.array_equal(piv, np.arange(n))
         assert _worst(A.astype(np.float64), lu, np.finfo(npdt).eps) <= n
+
+
+@pytest.mark.parametrize("npdt", [np.float64, np.float32])
+@pytest.mark.parametrize("row", [0, 20, 100])
+def test_pivot_larger_by_an_ulp(row, npdt):
+    """A row whose entry exceeds the diagonal's by one ulp is the pivot, also where their quotient rounds to 1
+    (row 0: an exact tie instead, which the first row wins)."""
+    print(f"[case] pivot by an ulp row={row} {npdt.__name__}", flush=True)
+    n = 130
+    rng = np.random.default_rng(row)
+    d = rng.uniform(1.0, 2.0, 4096).astype(npdt)
+    d = d[np.nextafter(d, npdt(3)) * (npdt(1) / d) <= 1][:8]
+    assert len(d) == 8
+    As = []
+    for v in d:
+        A = (rng.standard_normal((n, n)) / n + 4.0 * np.eye(n)).astype(npdt)
+        A[0, 0], A[row if row else 100, 0] = v, -(np.nextafter(v, npdt(3)) if row else v)
+        As.append(A)
+    _, pivs, info = _factor(As, npdt)
+    assert np.all(info == 0)
+    assert np.array_equal(pivs[:, 0], np.full(8, row))

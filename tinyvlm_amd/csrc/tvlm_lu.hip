@@ -268,14 +268,16 @@ __device__ int wave_compose_swaps(int first, int cnt, const int* piv, int* pd, i
 // Partial pivoting has one exchange over all rows per column; on the influence matrices of wings
 // nearly every pivot lies in the panel's diagonal block.  k_panel_spec factors a small set of
 // candidate rows on its own, eliminates all other rows against the resulting U11 and checks that
-// none of them would have been a pivot: every multiplier |l| <= 1.  When that holds everywhere, the
-// candidates' pivots are the ones partial pivoting over all rows picks (on a tie the first row, which
-// is the diagonal block's), so nothing had to be exchanged.  Three rounds:
+// none of them would have been a pivot: every multiplier |l| < 1.  When that holds everywhere, the
+// candidates' pivots are the ones partial pivoting over all rows picks, so nothing had to be exchanged.
+// Three rounds:
 //   round 1 (R = 1): candidates = the panel's kb diagonal rows, no interchange among them;
 //   rounds 2, 3 (R = 2): only for matrices whose earlier rounds failed: plus up to 64 rows that broke
 //                    the check in them, column by column the worst first (keys).
-// A column whose pivot is zero or not finite, a tie among candidates, an |l| above 1 (within rounding
-// of 1 in rounds 2 and 3, where a tie is not settled by the row order) or a NaN fails the round.
+// A column whose pivot is zero or not finite, a tie among candidates, an |l| above 1 or within its own rounding
+// of 1 (a row larger than the pivot by an ulp can have |l| = 1; a tie is not settled by the row order) or a
+// NaN fails the round.  Wings keep clear of that line (largest |l| 0.9992 over elliptic, swept and rectangular
+// ones of 256 to 4096 panels).
 // The rounds write their result to sp.w and leave the matrix as it is: the next round copies the
 // result of one that stood, the panel kernel launched after them (k_panel_coop / k_panel_reg) copies
 // round 3's, or factors the panel itself where all failed.  A matrix whose panels failed kSpecFails
@@ -757,16 +759,18 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
             }
         }
     }
-    // every multiplier of the candidates (columns before a row's own pivot) is at most 1
+    // every multiplier of the candidates (columns before a row's own pivot) is below 1 (rounds 2 and 3, which
+    // searched the pivot among them: at most 1)
+    constexpr T strict = T(1) - T(64) * (sizeof(T) == 8 ? (T)2.2e-16 : (T)1.2e-7f);
 #pragma unroll
     for (int q = 0; q < R; q++)
 #pragma unroll
         for (int k = 0; k < KC; k++) {
             const int c = KC * g + k;
             const bool mult = (R == 1 ? step[q] > c : act[q] || step[q] > c) && c < kb;
-            over1 = over1 || (mult && !(fabs(x[q][k]) <= T(1)));
+            over1 = over1 || (mult && !(fabs(x[q][k]) <= (R == 1 ? strict : T(1))));
         }
-    // round 1 goes on to the other rows after an |l| above 1 among the candidates (they are all
+    // round 1 goes on to the other rows after such an |l| among the candidates (they are all
     // candidates again, the keys of the others are wanted)
     if (R == 1 && __ballot(over1) != 0ull && lane == 0) *fail = 1;
     bad = bad || (R == 2 && over1);
@@ -858,7 +862,6 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
         return;
     }
     // the other rows, 16 per wave and step
-    const T one = T(1), strict = R == 2 ? T(1) - T(64) * (sizeof(T) == 8 ? (T)2.2e-16 : (T)1.2e-7f) : T(1);
     bool failed = false;
     for (int tile = 4 * share + g; tile < tiles; tile += 4 * shares) {
         if (tile >= 4 * shares) load_rows(tile);  // the first tile is here already
@@ -890,7 +893,7 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
         for (int b = 0; b < 4; b++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                over = over || !((T)fabs(y[b][r]) <= (R == 2 ? strict : one));
+                over = over || !((T)fabs(y[b][r]) <= strict);
                 if (use) w[row + (int64_t)(16 * b + M::k(lane, r)) * sp.ldw] = y[b][r];
             }
         over = over && use;
@@ -902,7 +905,7 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
 #pragma unroll
                     for (int r = 0; r < 4; r++) {
                         const T v = use ? (T)fabs(y[b][r]) : T(0);
-                        const float f = v <= (R == 2 ? strict : one) ? 0.0f : (v < T(3e38) ? (float)v : 3.4e38f);
+                        const float f = v <= strict ? 0.0f : (v < T(3e38) ? (float)v : 3.4e38f);
                         float top = fmaxf(f, row_rotated<8>(f));
                         top = fmaxf(top, row_rotated<4>(top));
                         top = fmaxf(top, row_rotated<2>(top));
