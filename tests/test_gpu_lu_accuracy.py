@@ -71,3 +71,26 @@ def test_pivot_larger_by_an_ulp(row, npdt):
     _, pivs, info = _factor(As, npdt)
     assert np.all(info == 0)
     assert np.array_equal(pivs[:, 0], np.full(8, row))
+
+
+@pytest.mark.parametrize("npdt", [np.float64, np.float32])
+@pytest.mark.parametrize("n,batch", [(70, 1), (192, 1), (192, 8), (1200, 1)])
+def test_growing_inverse_of_l(n, batch, npdt):
+    """U12 for panels whose L11 has diagonal blocks of large inverse (-0.97 below the diagonal): rows and columns
+    of the first panel's U12, where every sum has at most 16 terms and one correction as many again."""
+    print(f"[case] growing inverse n={n} batch={batch} {npdt.__name__}", flush=True)
+    rng = np.random.default_rng(n)
+    As = []
+    for b in range(batch):
+        L = np.eye(n)
+        for k in range(0, 64, 16):
+            L[k:k + 16, k:k + 16] -= 0.97 * np.tril(np.ones((16, 16)), -1)
+        U = np.eye(n)
+        U[:64, 64:] = rng.uniform(-1.0, 1.0, (64, n - 64))
+        As.append((L @ U).astype(npdt))
+    lus, pivs, info = _factor(As, npdt)
+    for A, lu, piv, inf in zip(As, lus, pivs, info):
+        assert inf == 0 and np.array_equal(piv, np.arange(n))
+        L, U = np.tril(lu, -1) + np.eye(n), np.triu(lu)
+        err = np.abs(A - L @ U)[:64, 64:] / (np.abs(L) @ np.abs(U))[:64, 64:]
+        assert np.max(err) <= 4 * 16 * np.finfo(npdt).eps

@@ -1377,7 +1377,9 @@ __global__ __launch_bounds__(NT) void k_panel_coop(T* __restrict__ a, int64_t ld
 // U12 = L11^{-1} A12 (L11 unit lower).  A wave takes 16 columns, which no other wave touches: every
 // value it needs is read before any is written, so the waves meet only once, for L11.  U12 is formed
 // on the matrix cores, 16 rows at a time: Z_b = Linv_bb (A_b - sum_{c<b} L_bc Z_c), Linv_bb the
-// inverse of L11's 16 x 16 diagonal block (each work-group inverts the four, a wave each); the MFMA
+// inverse of L11's 16 x 16 diagonal block (each work-group inverts the four, a wave each), corrected once
+// with its residual (multipliers of up to 1 allow entries of 2^14 in that inverse; without the correction
+// |A12 - L11 U12| reached 1400 eps |L11| |U12|, with it as little as by substitution); the MFMA
 // output layout is the second operand's, so the blocks chain in registers, and the block's rows are
 // read through the interchanges and written once.
 // Bound by the latency of the scattered column reads: 15.4 us per launch (mean over a factorisation of
@@ -1478,6 +1480,12 @@ __global__ __launch_bounds__(256) void k_swap_trsm(T* __restrict__ a, int64_t ld
 #pragma unroll
             for (int r = 0; r < 4; r++) x[b] = M::mfma(s_l[16 * b + ln][16 * c + M::k(lane, r)], x[c][r], x[b]);
         typename M::vacc s = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+        for (int r = 0; r < 4; r++) s = M::mfma(s_inv[b][ln][M::k(lane, r)], x[b][r], s);
+        // s += inv (x_b - L_bb s), the unit diagonal's part first
+        x[b] -= s;
+#pragma unroll
+        for (int r = 0; r < 4; r++) x[b] = M::mfma(s_l[16 * b + ln][16 * b + M::k(lane, r)], s[r], x[b]);
 #pragma unroll
         for (int r = 0; r < 4; r++) s = M::mfma(s_inv[b][ln][M::k(lane, r)], x[b][r], s);
         x[b] = s;
