@@ -94,3 +94,50 @@ def test_growing_inverse_of_l(n, batch, npdt):
         L, U = np.tril(lu, -1) + np.eye(n), np.triu(lu)
         err = np.abs(A - L @ U)[:64, 64:] / (np.abs(L) @ np.abs(U))[:64, 64:]
         assert np.max(err) <= 4 * 16 * np.finfo(npdt).eps
+
+
+@pytest.mark.parametrize("npdt", [np.float64, np.float32])
+@pytest.mark.parametrize("n,batch", [(32, 3), (33, 3), (40, 300), (49, 300), (65, 2), (128, 2), (129, 2), (193, 1), (257, 9)])
+def test_no_dominant_diagonal(n, batch, npdt):
+    """Matrices whose pivots lie anywhere, at the sizes where the rounds of a panel begin, take all rows as
+    candidates, or give up: LAPACK's pivots (FP64; FP32 sums may order near ties otherwise) and factors."""
+    import scipy.linalg as sl
+
+    print(f"[case] no dominant diagonal n={n} batch={batch} {npdt.__name__}", flush=True)
+    rng = np.random.default_rng(n)
+    As = [rng.standard_normal((n, n)).astype(npdt) for _ in range(batch)]
+    lus, pivs, info = _factor(As, npdt)
+    for b in range(0, batch, max(1, batch // 7)):
+        A, lu, piv = As[b].astype(np.float64), lus[b], pivs[b]
+        assert info[b] == 0
+        if npdt == np.float64:
+            assert np.array_equal(piv, sl.lu_factor(A)[1])
+        assert np.max(np.abs(np.tril(lu, -1))) <= 1 + 4 * np.finfo(npdt).eps
+        for k in range(n):
+            A[[k, piv[k]]] = A[[piv[k], k]]
+        assert _worst(A, lu, np.finfo(npdt).eps) <= n
+
+
+def test_scratch_of_a_large_batch_of_small_matrices():
+    """65535 FP32 matrices of 16 x 16 (67 MB): what the factorisation keeps is its interchange lists (2056 bytes a
+    matrix, with a quarter more than asked for), not room for panels that these matrices do not have."""
+    import torch
+
+    from tinyvlm_amd import capi as H
+    from tinyvlm_amd.serve import stream_create, stream_destroy
+
+    H.init(0)
+    n, batch = 16, 65535
+    print(f"[case] scratch n={n} batch={batch}", flush=True)
+    a = torch.randn(batch, n, n, device="cuda").permute(2, 1, 0)
+    ipiv = torch.zeros(n * batch, dtype=torch.int32, device="cuda")
+    info = torch.full((batch,), -1, dtype=torch.int32, device="cuda")
+    st = stream_create()  # a stream without any scratch yet
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    H.getrf(a, ipiv, info, stream=st)
+    torch.cuda.synchronize()
+    used = before - torch.cuda.mem_get_info()[0]
+    stream_destroy(st)
+    assert info.cpu().abs().max() == 0
+    assert used <= 1.5 * 2056 * batch

@@ -273,7 +273,9 @@ __device__ int wave_compose_swaps(int first, int cnt, const int* piv, int* pd, i
 // Three rounds:
 //   round 1 (R = 1): candidates = the panel's kb diagonal rows, no interchange among them;
 //   rounds 2, 3 (R = 2): only for matrices whose earlier rounds failed: plus up to 64 rows that broke
-//                    the check in them, column by column the worst first (keys).
+//                    the check in them, column by column the worst first (keys); not tried where round 1
+//                    was broken in more than half of the columns.  A panel with at most 64 other rows has all of
+//                    them as candidates of round 2, and no round 3.
 // A column whose pivot is zero or not finite, a tie among candidates, an |l| above 1 or within its own rounding
 // of 1 (a row larger than the pivot by an ulp can have |l| = 1; a tie is not settled by the row order) or a
 // NaN fails the round.  Wings keep clear of that line (largest |l| 0.9992 over elliptic, swept and rectangular
@@ -281,7 +283,7 @@ __device__ int wave_compose_swaps(int first, int cnt, const int* piv, int* pd, i
 // The rounds write their result to sp.w and leave the matrix as it is: the next round copies the
 // result of one that stood, the panel kernel launched after them (k_panel_coop / k_panel_reg) copies
 // round 3's, or factors the panel itself where all failed.  A matrix whose panels failed kSpecFails
-// times in a row skips the rounds from then on.
+// times in a row skips the rounds from then on, up to the panels whose rows are all candidates.
 // On the influence matrices of rectangular and 25-degree swept wings every panel stands in round 1;
 // on the elliptic ones (pivots at the tip panels, up to 1538 rows below the diagonal) up to half in
 // round 1, most others in round 2 and, at 64 x 64, a quarter in round 3.
@@ -329,6 +331,17 @@ constexpr int kSpecFails = 2;  // failed panels in a row after which a matrix sk
 // elliptic 64 x 64 wing need round 3, with these 17.
 constexpr int kSpecSlots = 16;
 constexpr int kSpecRounds = 3;
+// Columns with such a row past which rounds 2 and 3 are not tried: their candidates cannot hold all the pivots (a
+// wing breaks at most 8, a matrix without a dominant diagonal nearly all; two failed rounds of 256 rows and
+// more took 100 us).
+constexpr int kSpecMaxBroken = NB / 2;
+// Panels of at most this many rows have no rounds: k_panel_reg takes 1.6 us a column, a round's chain the same
+// whatever the width.  With more matrices than CUs k_panel_reg, of which a CU holds several, gains: 1000 FP32
+// matrices without a dominant diagonal, 40 x 40: 93 us without rounds, 130 with; 64 x 64 in FP64: 312 and 247.
+template <typename T>
+constexpr int spec_min_rows(int64_t batch) {
+    return batch <= 256 ? 32 : sizeof(T) == 8 ? 48 : 64;
+}
 constexpr int kSpecMaxRows = 32768;  // rows of a panel (the cooperative panels hold no more)
 
 // Buffers of one panel's speculative rounds (device); sets are zeroed once per factorisation.
@@ -337,9 +350,12 @@ struct SpecBufs {
     bool on = false;
     T* w = nullptr;                      // results: matrix z at w + z ldw NB, {rows, NB} column-major
     int64_t ldw = 0;
-    // this panel's [kSpecRounds - 1][batch][kSpecSlots][NB]: largest |l| > 1, with its row
+    // this panel's [kSpecRounds - 1][batch][kSpecSlots][NB]: largest |l| > 1, with its row (null for a panel
+    // whose other rows are all candidates of round 2)
     unsigned long long* keys = nullptr;
-    int32_t* fail = nullptr;    // this panel's [kSpecRounds][batch]: the round failed
+    int rounds = kSpecRounds;   // rounds of this panel
+    int32_t* fail = nullptr;    // this panel's [kSpecRounds][batch]: 1 where the round failed, 2 in round 1
+                                // where its blocks' condition failed it (then no row was checked)
     int32_t* ostate = nullptr;  // [batch]: failed panels in a row
     int batch = 1;
 };
@@ -355,7 +371,7 @@ __device__ __forceinline__ int spec_stood(const SpecBufs<T>& sp, int z, int roun
 // Whether one of the rounds stood for matrix z (the failure count is kept by the one `keeper` thread).
 template <typename T>
 __device__ __forceinline__ bool spec_settled(const SpecBufs<T>& sp, int z, bool keeper) {
-    const bool ok = spec_stood(sp, z, kSpecRounds) != 0;
+    const bool ok = spec_stood(sp, z, sp.rounds) != 0;
     if (keeper) {
         if (ok)
             sp.ostate[z] = 0;
@@ -365,15 +381,22 @@ __device__ __forceinline__ bool spec_settled(const SpecBufs<T>& sp, int z, bool 
     return ok;
 }
 
-// Copies a round's result into the panel; thread id of count.
+// Copies a round's result into the panel; thread id of count (whole waves, 64 rows x 8 columns each at a time).
 template <typename T>
 __device__ __forceinline__ void spec_commit(const SpecBufs<T>& sp, int z, T* a, int64_t lda, int n, int k0, int kb,
                                             int id, int count) {
     const T* w = sp.w + (int64_t)z * sp.ldw * NB;
     const int m = n - k0;
-    for (int r = id; r < m; r += count)
-#pragma unroll 8
-        for (int j = 0; j < kb; j++) a[(k0 + r) + (int64_t)(k0 + j) * lda] = w[r + (int64_t)j * sp.ldw];
+    for (int e = id >> 6; e < (m + 63) / 64 * (NB / 8); e += count >> 6) {
+        const int r = e / (NB / 8) * 64 + (id & 63), j0 = e % (NB / 8) * 8;
+        T v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (r < m && j0 + j < kb) v[j] = w[r + (int64_t)(j0 + j) * sp.ldw];
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (r < m && j0 + j < kb) a[(k0 + r) + (int64_t)(k0 + j0 + j) * lda] = v[j];
+    }
 }
 
 __device__ __forceinline__ double lane_value(double v, int l) {
@@ -536,7 +559,7 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
         if (stood != 0) return;
     }
     int32_t* fail = sp.fail + (round - 1) * sp.batch + z;
-    if (sp.ostate[z] >= kSpecFails) {
+    if (sp.keys && sp.ostate[z] >= kSpecFails) {
         if (blockIdx.x == 0 && t == 0) *fail = 1;
         return;
     }
@@ -553,10 +576,11 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
     int crow = -1;  // row of candidate 64 + lane
     if constexpr (R == 2) {
         for (int e = t; e < (m + 31) / 32; e += 256) s_cmap[e] = 0u;
-        // round by round, lane = column: its worst row first, then its other rows; entry e of the list
-        // sits in lane e
+        // all other rows where they are that few; else round by round, lane = column: its worst row first, then its
+        // other rows; entry e of the list sits in lane e
         int count = 0;
-        for (int rd = 0; rd < round - 1; rd++) {
+        if (!sp.keys && kb + lane < m) crow = kb + lane;
+        for (int rd = 0; sp.keys && rd < round - 1; rd++) {
             const unsigned long long* keys = sp.keys + ((int64_t)(rd * sp.batch + z) * kSpecSlots) * NB + lane;
             unsigned long long key[kSpecSlots + 1];
             key[0] = 0ull;
@@ -564,6 +588,11 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
             for (int s = 1; s <= kSpecSlots; s++) key[s] = keys[(s - 1) * NB];
 #pragma unroll
             for (int s = 1; s <= kSpecSlots; s++) key[0] = key[s] > key[0] ? key[s] : key[0];
+            // alike in every wave: the columns that round 1 found a row for (none where no row was checked)
+            if (rd == 0 && (sp.fail[z] == 2 || __popcll(__ballot(key[0] != 0ull)) > kSpecMaxBroken)) {
+                if (blockIdx.x == 0 && t == 0) *fail = 1;
+                return;
+            }
 #pragma unroll
             for (int s = 0; s <= kSpecSlots; s++) {
                 const int row = key[s] != 0ull ? (int)~(uint32_t)key[s] : -1;
@@ -772,7 +801,7 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
         }
     // round 1 goes on to the other rows after such an |l| among the candidates (they are all
     // candidates again, the keys of the others are wanted)
-    if (R == 1 && __ballot(over1) != 0ull && lane == 0) *fail = 1;
+    if (R == 1 && blockIdx.x == 0 && __ballot(over1) != 0ull && lane == 0) atomicMax(fail, 1);
     bad = bad || (R == 2 && over1);
     if (__ballot(bad) != 0ull && lane == 0) s_bad = 1;
     // the diagonal block in pivot order (identity beyond kb), U negated for the products below
@@ -839,7 +868,7 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
             if (lane == 0) out[0] = ni + __popcll(mo);
         }
     }
-    if (m <= kb || share < 0) return;
+    if (m <= kb || share < 0 || (R == 2 && !sp.keys)) return;
     // inverse of U's diagonal block g, a row per lane (in every row of 16 lanes)
     {
         T rt[16], s[16];
@@ -858,7 +887,7 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
     }
     __syncthreads();
     if (s_ill != 0) {  // the rows' multipliers would not be accurate
-        if (t == 0) *fail = 1;
+        if (t == 0) atomicMax(fail, 2);
         return;
     }
     // the other rows, 16 per wave and step
@@ -899,7 +928,7 @@ __global__ __launch_bounds__(256) void k_panel_spec(T* __restrict__ a, int64_t l
         over = over && use;
         if (__ballot(over) != 0ull) {
             failed = true;
-            if (round < kSpecRounds) {  // per column the row of the largest |l| among the wave's 16
+            if (sp.keys && round < kSpecRounds) {  // per column the row of the largest |l| among the wave's 16
 #pragma unroll
                 for (int b = 0; b < 4; b++)
 #pragma unroll
@@ -933,7 +962,7 @@ __global__ __launch_bounds__(NT) void k_panel_reg(T* __restrict__ a, int64_t lda
     // after a speculative panel: nothing to do where one of its earlier rounds stood; where the last did,
     // the launch's work-groups copy its result; work-group 0 factors the panel where all failed
     if (sp.on && spec_settled(sp, blockIdx.z, blockIdx.x == 0 && threadIdx.x == 0)) {
-        if (spec_stood(sp, blockIdx.z, kSpecRounds - 1) == 0)
+        if (spec_stood(sp, blockIdx.z, sp.rounds - 1) == 0)
             spec_commit(sp, blockIdx.z, a, lda, n, k0, kb, blockIdx.x * NT + threadIdx.x, gridDim.x * NT);
         return;
     }
@@ -1231,7 +1260,7 @@ __global__ __launch_bounds__(NT) void k_panel_coop(T* __restrict__ a, int64_t ld
     constexpr int NW = NT / 64, MG = kCoopMaxGroups;
     const int z = blockIdx.z, g = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
     if (sp.on && spec_settled(sp, z, g == 0 && t == 0)) {
-        if (spec_stood(sp, z, kSpecRounds - 1) == 0)
+        if (spec_stood(sp, z, sp.rounds - 1) == 0)
             spec_commit(sp, z, a + (int64_t)z * sb, lda, n, k0, kb, g * NT + t, G * NT);
         return;
     }
@@ -1690,14 +1719,20 @@ struct SpecWork {
     SpecBufs<T> panel(int kp) const {
         SpecBufs<T> b = base;
         const int64_t s = kp / NB, batch = base.batch;
-        b.keys += s * (kSpecRounds - 1) * batch * kSpecSlots * NB;
+        if (base.ldw - kp <= spec_min_rows<T>(batch)) b.on = false;
+        if ((size_t)s < keyed(base.ldw))
+            b.keys += s * (kSpecRounds - 1) * batch * kSpecSlots * NB;
+        else
+            b.keys = nullptr, b.rounds = 2;
         b.fail += s * kSpecRounds * batch;
         return b;
     }
+    // panels with more rows below their first NB than round 2 has candidates
+    static size_t keyed(int64_t n) { return n > 2 * NB ? (size_t)(n - 2 * NB + NB - 1) / NB : 0; }
     // bytes of the flags, the failure counts and the keys (zeroed before the first panel), and in all
     static size_t zeroed(int n, int batch) {
         const size_t panels = (size_t)(n + NB - 1) / NB;
-        return (sizeof(unsigned long long) * panels * (kSpecRounds - 1) * kSpecSlots * NB +
+        return (sizeof(unsigned long long) * keyed(n) * (kSpecRounds - 1) * kSpecSlots * NB +
                 sizeof(int32_t) * (kSpecRounds * panels + 1)) * batch;
     }
     static size_t bytes(int n, int batch) {
@@ -1708,7 +1743,7 @@ struct SpecWork {
         const size_t panels = (size_t)(n + NB - 1) / NB;
         base.on = true;
         base.keys = static_cast<unsigned long long*>(ws);
-        base.fail = reinterpret_cast<int32_t*>(base.keys + panels * (kSpecRounds - 1) * batch * kSpecSlots * NB);
+        base.fail = reinterpret_cast<int32_t*>(base.keys + keyed(n) * (kSpecRounds - 1) * batch * kSpecSlots * NB);
         base.ostate = base.fail + kSpecRounds * panels * batch;
         base.w = reinterpret_cast<T*>(static_cast<char*>(ws) + (zeroed(n, batch) + 255) / 256 * 256);
         base.ldw = n;
@@ -1729,7 +1764,7 @@ int panel_spec(T* a, int64_t lda, int n, int kp, int kb, int32_t* ipiv, int32_t*
     const dim3 grid(shares + 1, 1, batch);  // one more for the candidates' result
     hipLaunchKernelGGL((k_panel_spec<T, 1>), grid, dim3(256), 0, st, a, lda, n, kp, kb, ipiv, perm, sb, sp, 1);
     TVLM_LAUNCHED();
-    for (int round = 2; round <= kSpecRounds; round++) {
+    for (int round = 2; round <= sp.rounds; round++) {
         hipLaunchKernelGGL((k_panel_spec<T, 2>), grid, dim3(256), 0, st, a, lda, n, kp, kb, ipiv, perm, sb, sp, round);
         TVLM_LAUNCHED();
     }
@@ -1741,10 +1776,8 @@ template <typename T>
 int panel_fast(T* a, int64_t lda, int n, int kp, int kb, int32_t* ipiv, int32_t* info, int32_t* perm, hipStream_t st,
                int batch, int64_t sb, const SpecWork<T>& spec) {
     SpecBufs<T> sp;
-    if (spec.base.on) {
-        sp = spec.panel(kp);
-        TVLM_TRY(panel_spec<T>(a, lda, n, kp, kb, ipiv, perm, st, batch, sb, sp));
-    }
+    if (spec.base.on) sp = spec.panel(kp);
+    if (sp.on) TVLM_TRY(panel_spec<T>(a, lda, n, kp, kb, ipiv, perm, st, batch, sb, sp));
     return panel_one_group<T>(a, lda, n, kp, kb, ipiv, info, perm, st, batch, sb, sp);
 }
 
@@ -2114,10 +2147,8 @@ int getrf_coop_pairs(T* a, int64_t lda, int n, int batch, int64_t sb, int32_t* i
         TVLM_REQUIRE(p.ctr_set >= 0 && p.ctr_set < plan.ctr_sets, "cooperative panel %d: counter set %d of %d", s,
                      p.ctr_set, plan.ctr_sets);
         SpecBufs<T> sp;
-        if (spec.base.on) {
-            sp = spec.panel(kp);
-            TVLM_TRY(panel_spec<T>(a, lda, n, kp, kb, ipiv, perm, st, batch, sb, sp));
-        }
+        if (spec.base.on) sp = spec.panel(kp);
+        if (sp.on) TVLM_TRY(panel_spec<T>(a, lda, n, kp, kb, ipiv, perm, st, batch, sb, sp));
         return panel_coop<T>(a, lda, n, kp, kb, p.groups, ipiv, info, perm, st, batch, sb,
                              ctr + (size_t)p.ctr_set * batch * kCoopCtr, cval, crow, xrow, fail, sp);
     };
@@ -2184,13 +2215,23 @@ int getrf(const tvlm_view* av, int32_t* ipiv, int32_t* info, void* stream, bool 
     TVLM_TRY(device_workspace(sizeof(int32_t) * kPermInts * 2 * (size_t)batch, &ws, kWsLuPerm, st));
     int32_t* perm = static_cast<int32_t*>(ws);
     const GetrfPlan plan = getrf_plan<T>(n, batch, allow_coop);
+    void* cws = nullptr;
+    if (plan.path == kPathCoopPairs) TVLM_TRY(device_workspace(plan.coop_bytes(sizeof(T)), &cws, kWsLuCoop, st));
     // Speculative panels wherever a panel kernel of at most kFastPanelRows rows or a cooperative one
     // follows them.  With a spin limit set (a diagnostic), cooperative factorisations go without, so that
     // the waits it bounds are run.
     SpecWork<T> spec;
-    if (n > 0 && n <= kSpecMaxRows && (plan.path == kPathCoopPairs ? g_coop_spin_limit.load() == kCoopSpinLimit : n <= kFastPanelRows)) {
-        void* sws = nullptr;
-        TVLM_TRY(device_workspace(SpecWork<T>::bytes(n, batch), &sws, kWsLuSpec, st));
+    // Without room for their buffers the panels go without as well.
+    void* sws = nullptr;
+    if (n > spec_min_rows<T>(batch) && n <= kSpecMaxRows &&
+        (plan.path == kPathCoopPairs ? g_coop_spin_limit.load() == kCoopSpinLimit : n <= kFastPanelRows)) {
+        const int rc = device_workspace(SpecWork<T>::bytes(n, batch), &sws, kWsLuSpec, st);
+        if (rc == TVLM_ERR_NOMEM)
+            (void)hipGetLastError();
+        else
+            TVLM_TRY(rc);
+    }
+    if (sws) {
         spec.place(sws, n, batch);
         const int64_t words = (int64_t)(SpecWork<T>::zeroed(n, batch) / sizeof(int32_t));
         hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st,
@@ -2203,8 +2244,6 @@ int getrf(const tvlm_view* av, int32_t* ipiv, int32_t* info, void* stream, bool 
         // the attempt counter and the failure word (all zeroed here, once for the whole
         // factorisation), the candidates, the published rows and U11, and the deferred
         // interchanges' gather lists.
-        void* cws = nullptr;
-        TVLM_TRY(device_workspace(plan.coop_bytes(sizeof(T)), &cws, kWsLuCoop, st));
         int32_t* ctr = static_cast<int32_t*>(cws);
         int32_t* crow = ctr + plan.nctr;
         T* cval = reinterpret_cast<T*>((reinterpret_cast<uintptr_t>(crow + plan.ncand) + 255) & ~(uintptr_t)255);
