@@ -90,3 +90,50 @@ def test_trailing_update_rejects_bad_arguments():
     assert lib.tvlm_lu_update(ctypes.c_int32(4), None, ctypes.c_int64(1), None, ctypes.c_int64(1), None,
                               ctypes.c_int64(1), ctypes.c_int64(0), ctypes.c_int64(0), ctypes.c_int64(0),
                               ctypes.c_int32(1), ctypes.c_int64(0), None) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+def test_update_with_a_large_leading_dimension(prec):
+    """A leading dimension of 1.6e8 (15 of them pass 2^31): columns of B that far apart, in an allocation that ends
+    with the last one; dot products of 16 terms, the bound above."""
+    import torch
+
+    from tinyvlm_amd import capi as H
+
+    H.init(0)
+    m, n, k, ld = 70, 16, 16, 160_000_000
+    print(f"[case] lu update {prec} ldb={ld}", flush=True)
+    dt, eb = (torch.float32, 4) if prec == "f32" else (torch.float64, 8)
+    buf = torch.empty(ld * (n - 1) + k, dtype=dt, device="cuda")
+    B = buf.as_strided((k, n), (1, ld))
+    B.copy_(torch.randn(k, n, dtype=dt, device="cuda"))
+    A = torch.randn(k, m, dtype=dt, device="cuda").t()
+    C = torch.randn(n, m, dtype=dt, device="cuda").t()
+    C0 = C.to(torch.float64, copy=True)
+    H.check(H.lib().tvlm_lu_update(ctypes.c_int32(eb), ctypes.c_void_p(C.data_ptr()), ctypes.c_int64(m),
+                                   ctypes.c_void_p(A.data_ptr()), ctypes.c_int64(m), ctypes.c_void_p(buf.data_ptr()),
+                                   ctypes.c_int64(ld), ctypes.c_int64(m), ctypes.c_int64(n), ctypes.c_int64(k),
+                                   ctypes.c_int32(1), ctypes.c_int64(0), H.stream_ptr()))
+    Bd = B.double().contiguous()
+    err = (C.double() - (C0 - A.double() @ Bd)).abs()
+    bound = (k + 2) * float(torch.finfo(dt).eps) * (A.double().abs() @ Bd.abs() + C0.abs())
+    assert bool((err <= bound).all())
+
+
+def test_leading_dimensions_past_the_updates_offsets_are_refused():
+    """Arguments are checked before anything is queued: matrices with a trailing update and a leading dimension of
+    2^28 or more give an error (no device is touched)."""
+    from tinyvlm_amd import capi as H
+
+    lib = H.lib()
+    fake = ctypes.c_void_p(4096)
+    v = H.View()
+    v.ptr, v.shape[:], v.stride[:] = 4096, (65, 65, 1), (1, 1 << 28, 65 << 28)
+    for f in (lib.tvlm_getrf_f32, lib.tvlm_getrf_f64):
+        assert f(ctypes.byref(v), fake, fake, None) == 1
+        assert b"out of range" in lib.tvlm_last_error()
+    i64, one = ctypes.c_int64, ctypes.c_int32(1)
+    for lds in ((1 << 28, 64, 64), (64, 1 << 28, 64), (64, 64, 1 << 28)):
+        assert lib.tvlm_lu_update(ctypes.c_int32(4), fake, i64(lds[0]), fake, i64(lds[1]), fake, i64(lds[2]), i64(64),
+                                  i64(64), i64(64), one, i64(0), None) == 1

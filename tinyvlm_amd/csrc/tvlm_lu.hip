@@ -1563,7 +1563,8 @@ struct UpdCfg<double> {
 };
 
 constexpr int kUpdDK = 16;  // k-slice depth
-constexpr int64_t kUpdMaxLd = (int64_t)1 << 26;  // leading dimensions whose 16 columns fit 32-bit offsets
+// Leading dimensions below this keep k_update's per-lane offsets (at most 15 of them and 15) in 32 bits, unsigned.
+constexpr int64_t kUpdMaxLd = (int64_t)1 << 28;
 
 // The FP32 128 x 64 tile is held to 6 waves per SIMD (its accumulators then sit in 80 vector registers
 // beside the operands instead of 32 accumulation registers: 5 -> 6 waves; measured ~1 % on getrf).
@@ -1579,7 +1580,7 @@ void k_update(T* __restrict__ C, int64_t ldc, const T* __restrict__ A, int64_t l
     __shared__ T sa[2][DK][TI];
     __shared__ T sb[2][TJ][DK + 1];
     const int i0 = blockIdx.x * TI, j0 = blockIdx.y * TJ;
-    // uniform tile bases: every per-lane offset below fits 32 bits (< 4 ld + TI)
+    // uniform tile bases: every per-lane offset below fits 32 bits (kUpdMaxLd)
     C += (int64_t)blockIdx.z * sbatch + i0 + (int64_t)j0 * ldc;
     A += (int64_t)blockIdx.z * sbatch + i0;
     B += (int64_t)blockIdx.z * sbatch + (int64_t)j0 * ldb;
@@ -1591,7 +1592,7 @@ void k_update(T* __restrict__ C, int64_t ldc, const T* __restrict__ A, int64_t l
     const int li = l % BM, lg = l / BM;
     const int ta_i = t % TI, ta_k = t / TI;  // A staging: rows along the threads
     const int tb_k = t % DK, tb_j = t / DK;  // B staging: k along the threads
-    const int offA = ta_i + ta_k * (int)lda, offB = tb_k + tb_j * (int)ldb;
+    const unsigned offA = ta_i + ta_k * (unsigned)lda, offB = tb_k + tb_j * (unsigned)ldb;
     const int nsl = (kb + DK - 1) / DK;
     T ra[NA], rb[NBq];
     auto load = [&](int s) {
@@ -1639,7 +1640,7 @@ void k_update(T* __restrict__ C, int64_t ldc, const T* __restrict__ A, int64_t l
                 for (int bj = 0; bj < NBJ; bj++) acc[bi][bj] = G::mfma(b[bj], a[bi], acc[bi][bj]);
         }
     }
-    const int offC = li + G::drow(l, 0) * (int)ldc;
+    const unsigned offC = li + G::drow(l, 0) * (unsigned)ldc;
 #pragma unroll
     for (int bi = 0; bi < NBI; bi++) {
         const int i = wi + bi * BM + li;
@@ -2205,6 +2206,7 @@ int getrf(const tvlm_view* av, int32_t* ipiv, int32_t* info, void* stream, bool 
     const int batch = (int)av->shape[2];
     const int64_t lda = av->stride[1], sb = av->stride[2];
     TVLM_REQUIRE(lda >= n || n == 0, "lda < n");
+    TVLM_REQUIRE(n <= NB || lda < kUpdMaxLd, "lda %lld out of range for a trailing update", (long long)lda);
     TVLM_REQUIRE(batch >= 1 && batch <= 65535, "batch %d out of range", batch);
     TVLM_REQUIRE(batch == 1 || sb >= lda * n, "matrices of the batch overlap (stride[2] < stride[1] * n)");
     hipStream_t st = as_stream(stream);
@@ -2882,8 +2884,8 @@ int tvlm_lu_update(int32_t elem_bytes, void* c, int64_t ldc, const void* a, int6
     TVLM_REQUIRE(elem_bytes == 4 || elem_bytes == 8, "elem_bytes must be 4 or 8");
     TVLM_REQUIRE(m >= 0 && n >= 0 && k >= 0 && m < (1 << 30) && n < (1 << 30) && k < (1 << 30), "m/n/k out of range");
     TVLM_REQUIRE(batch >= 1 && batch <= 65535 && (batch == 1 || stride >= 0), "batch %d / stride out of range", batch);
-    TVLM_REQUIRE(ldc >= (m > 1 ? m : 1) && lda >= (m > 1 ? m : 1) && ldb >= (k > 1 ? k : 1) && ldc < (1 << 28) &&
-                     lda < (1 << 28) && ldb < (1 << 28),
+    TVLM_REQUIRE(ldc >= (m > 1 ? m : 1) && lda >= (m > 1 ? m : 1) && ldb >= (k > 1 ? k : 1) &&
+                     ldc < tvlm::kUpdMaxLd && lda < tvlm::kUpdMaxLd && ldb < tvlm::kUpdMaxLd,
                  "leading dimensions out of range");
     if (m == 0 || n == 0 || k == 0) return TVLM_OK;
     TVLM_REQUIRE(c && a && b, "null matrix");
