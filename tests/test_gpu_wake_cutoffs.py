@@ -47,3 +47,34 @@ def test_lattice_near_cutoffs(rows, ns, bad):
         return
     assert np.all(np.isfinite(out[1]))
     assert np.max(np.abs(out[0] - out[1])) <= 2e-12 * np.max(np.abs(out[0]))
+
+
+@pytest.mark.parametrize("chord", [1.0, 0.05, 0.02, 0.005])
+@pytest.mark.parametrize("rows,ns,nc", [(1, 5, 3), (7, 40, 10), (30, 65, 4)])
+def test_small_wing_at_the_cutoffs(rows, ns, nc, chord):
+    """A wing right in front of its wake, down to chords at which the absolute cutoffs meet most of its
+    segments: tiles walked without the cutoffs, twice, and with them from the start."""
+    import torch
+
+    from tinyvlm_amd import capi as H
+
+    H.init(0)
+    print(f"[case] lattice columns chord={chord} rows={rows} ns={ns} nc={nc}", flush=True)
+    rng = np.random.default_rng(ns)
+    d = chord / nc
+    ys = np.linspace(0.0, 2.0 * chord, ns + 1)
+    w = np.zeros((ns + 1, rows + 1, 4))
+    w[:, :, 0], w[:, :, 1], w[:, :, 3] = chord + d * np.arange(rows + 1)[None, :], ys[:, None], 1.0
+    w[:, :, 2] = 0.1 * chord * np.sin(np.arange(rows + 1))[None, :]
+    g = rng.standard_normal((ns, rows))
+    c = np.zeros((ns, nc, 3))
+    c[:, :, 0], c[:, :, 1] = d * (np.arange(nc) + 0.75)[None, :], 0.5 * (ys[1:] + ys[:-1])[:, None]
+    n = np.zeros((ns, nc, 3)) + [0.1, 0.05, 1.0]
+    t = lambda x: [H.to_device(x, torch.float64)]  # noqa: E731
+    out = []
+    for f in (H.rhs_assemble_wake_influence, H.rhs_assemble_wake_influence_lattice):
+        rhs = torch.zeros(ns * nc, dtype=torch.float64, device="cuda")
+        f(rhs, t(g), t(c), t(n), t(w), [True], rows)
+        out.append(rhs.cpu().numpy())
+    assert np.all(np.isfinite(out[1]))
+    assert np.max(np.abs(out[0] - out[1])) <= 2e-12 * np.max(np.abs(out[0]))

@@ -219,6 +219,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                                                       double* __restrict__ partial, int64_t spart, int step, int rows,
                                                       int sw, int tiles_span) {
     __shared__ LatTile<RH> tile_s;
+    if (threadIdx.x == 0) tile_s.small = 0;
     double *const sverts = tile_s.verts, *const sgam = tile_s.gam;
     __shared__ double sred[kWaves][kRecv];
     const int b = blockIdx.z;

@@ -628,46 +628,6 @@ __device__ __forceinline__ LatVertex lat_vertex(double cx, double cy, double cz,
     return f;
 }
 
-// Segment a->b of strength g for the receiver and for its image in y = 0, without the 1/(4 pi) factor
-// (lattice_chunk applies it once to its sum).  The two evaluations share every term without a y
-// component: r0 = b - a (taken as (c - a) - (c - b), whose y part is the same for the image), the y
-// component of r1 x r2 and its square, and the x and z parts of r0.r1 and r0.r2.
-__device__ __forceinline__ void lat_pair(double& ax, double& ay, double& az, const LatVertex& a, const LatVertex& b,
-                                         double g) {
-    const double r0x = a.x - b.x, r0y = a.y - b.y, r0z = a.z - b.z;
-    const double cry = a.z * b.x - a.x * b.z;
-    const double cry2 = cry * cry;
-    const double d1xz = r0x * a.x + r0z * a.z;
-    const double d2xz = r0x * b.x + r0z * b.z;
-    constexpr double cut = BS<double>::cut_cross;
-    // |r| < RCUT  <=>  1/|r| > 1/RCUT
-    constexpr double rimax = 1.0 / BS<double>::cut_norm;
-    {
-        const double crx = a.y * b.z - a.z * b.y;
-        const double crz = a.x * b.y - a.y * b.x;
-        const double sq = crx * crx + crz * crz + cry2;
-        const double d1 = d1xz + r0y * a.y, d2 = d2xz + r0y * b.y;
-        const bool ok = (sq >= cut) & (a.ri <= rimax) & (b.ri <= rimax);
-        const double t = (d1 * a.ri - d2 * b.ri) * rcp_seeded(sq) * g;
-        const double coeff = ok ? t : 0.0;
-        ax += coeff * crx;
-        ay += coeff * cry;
-        az += coeff * crz;
-    }
-    {
-        const double crx = a.ym * b.z - a.z * b.ym;
-        const double crz = a.x * b.ym - a.ym * b.x;
-        const double sq = crx * crx + crz * crz + cry2;
-        const double d1 = d1xz + r0y * a.ym, d2 = d2xz + r0y * b.ym;
-        const bool ok = (sq >= cut) & (a.rim <= rimax) & (b.rim <= rimax);
-        const double t = (d1 * a.rim - d2 * b.rim) * rcp_seeded(sq) * g;
-        const double coeff = ok ? t : 0.0;
-        ax += coeff * crx;
-        ay -= coeff * cry;
-        az += coeff * crz;
-    }
-}
-
 constexpr int kLatChunkMax = 16;  // spans per wave
 
 // A segment a -> b of a staged tile: b - a, and the difference of the circulations beside it.
@@ -683,10 +643,13 @@ struct LatTile {
     double gam[RH * kSpans];                    // circulations rhe x swe
     LatSegment span[(RH + 1) * kSpans];         // vertex row q, from vertex column s to s + 1: q * swe + s
     LatSegment chord[RH * (kSpans + 1)];        // vertex column s, from vertex row q to q + 1: q * vw + s
+    int small;                                  // not 0: some ring is so small that its segments meet the cutoffs
 };
 
 // The segments of a tile whose vertices and circulations are staged (between two barriers).  Rings
-// outside the tile count 0 in the differences: their own tile adds them.
+// outside the tile count 0 in the differences: their own tile adds them.  A receiver in line with a ring's
+// middle has |r1 x r2| of half the ring's area with its chordwise edges, wherever along the line it stands: rings
+// whose half is below the cutoff, within a tenth, set t.small (0 before).
 template <int RH>
 __device__ __forceinline__ void lattice_segments(LatTile<RH>& t, int swe, int rhe) {
     const int vw = swe + 1;
@@ -704,11 +667,55 @@ __device__ __forceinline__ void lattice_segments(LatTile<RH>& t, int swe, int rh
         double g = 0.0;
         if (s < swe) g -= t.gam[q * swe + s];
         if (s > 0) g += t.gam[q * swe + s - 1];
-        t.chord[e] = {w[0] - v[0], w[1] - v[1], w[2] - v[2], g};
+        const double x = w[0] - v[0], y = w[1] - v[1], z = w[2] - v[2];
+        t.chord[e] = {x, y, z, g};
+        if (s < swe) {
+            const double sx = v[3] - v[0], sy = v[4] - v[1], sz = v[5] - v[2];
+            const double nx = y * sz - z * sy, ny = z * sx - x * sz, nz = x * sy - y * sx;
+            if (nx * nx + ny * ny + nz * nz < 4.4 * BS<double>::cut_cross) t.small = 1;
+        }
     }
 }
 
 __device__ __forceinline__ uint32_t hi_word(double v) { return (uint32_t)__double2hiint(v); }
+
+// A staged segment a->b for the receiver and for its image in y = 0, without the 1/(4 pi) factor (lattice_chunk
+// applies it once to its sum).  The two share every term without a y component: the y component of r1 x r2
+// and its square, and the x and z parts of r0.r1 and r0.r2.
+__device__ __forceinline__ void lat_pair(double& ax, double& ay, double& az, const LatVertex& a, const LatVertex& b,
+                                         const LatSegment& r) {
+    const double cry = a.z * b.x - a.x * b.z;
+    const double cry2 = cry * cry;
+    const double d1xz = r.x * a.x + r.z * a.z;
+    const double d2xz = r.x * b.x + r.z * b.z;
+    constexpr double cut = BS<double>::cut_cross;
+    // |r| < RCUT  <=>  1/|r| > 1/RCUT
+    constexpr double rimax = 1.0 / BS<double>::cut_norm;
+    {
+        const double crx = a.y * b.z - a.z * b.y;
+        const double crz = a.x * b.y - a.y * b.x;
+        const double sq = crx * crx + crz * crz + cry2;
+        const double d1 = d1xz + r.y * a.y, d2 = d2xz + r.y * b.y;
+        const bool ok = (sq >= cut) & (a.ri <= rimax) & (b.ri <= rimax);
+        const double t = (d1 * a.ri - d2 * b.ri) * rcp_seeded(sq) * r.g;
+        const double coeff = ok ? t : 0.0;
+        ax += coeff * crx;
+        ay += coeff * cry;
+        az += coeff * crz;
+    }
+    {
+        const double crx = a.ym * b.z - a.z * b.ym;
+        const double crz = a.x * b.ym - a.ym * b.x;
+        const double sq = crx * crx + crz * crz + cry2;
+        const double d1 = d1xz + r.y * a.ym, d2 = d2xz + r.y * b.ym;
+        const bool ok = (sq >= cut) & (a.rim <= rimax) & (b.rim <= rimax);
+        const double t = (d1 * a.rim - d2 * b.rim) * rcp_seeded(sq) * r.g;
+        const double coeff = ok ? t : 0.0;
+        ax += coeff * crx;
+        ay -= coeff * cry;
+        az += coeff * crz;
+    }
+}
 
 // A staged segment for the receiver and its image, as lat_pair but without its cutoffs: low_sq keeps
 // the smallest high word of |r1 x r2|^2 met, so that the walk learns at its end whether any segment came
@@ -754,53 +761,43 @@ __device__ __forceinline__ LatVertex lat_vertex_fast(double cx, double cy, doubl
 
 // The lattice walk of one wave over its span chunk [sa, sb) of a staged tile for the receiver
 // (cx, cy, cz): chordwise segments of each vertex column, spanwise segments of each vertex row, the
-// previous vertex column's terms kept in registers; the tile's right edge only when sb == swe.  Adds
-// the induced velocity to (vx, vy, vz).  This form applies every cutoff where it stands.
-template <int RH>
-__device__ __forceinline__ void lattice_chunk_cutoffs(const LatTile<RH>& t, int swe, int rhe, int sa, int sb, double cx,
-                                                      double cy, double cz, double& ax, double& ay, double& az) {
+// previous vertex column's terms kept in registers; the tile's right edge only when sb == swe.  (ax, ay, az): 4 pi x
+// the induced velocity.  CUT: every cutoff is applied where it stands; else none is, and low_sq and low_r2 are
+// the smallest high words of |r1 x r2|^2 and |r|^2 met.
+template <int RH, bool CUT>
+__device__ __forceinline__ void lattice_walk(const LatTile<RH>& t, int swe, int rhe, int sa, int sb, double cx, double cy,
+                                             double cz, double& ax, double& ay, double& az, uint32_t& low_sq,
+                                             uint32_t& low_r2) {
     const int vw = swe + 1;
-    ax = ay = az = 0.0;  // 4 pi x the induced velocity (lat_pair leaves the factor out)
-    // per vertex column: its rhe chordwise segments, then the rhe + 1 spanwise ones to the next column
-#pragma unroll 1
-    for (int s = sa; s <= sb; s++)
-#pragma unroll 1
-        for (int e = s < sb || sb == swe ? 0 : rhe; e < (s < sb ? 2 * rhe + 1 : rhe); e++) {
-            const bool chord = e < rhe;
-            const int q = chord ? e : e - rhe, from = q * vw + s;
-            lat_pair(ax, ay, az, lat_vertex(cx, cy, cz, t.verts + 3 * from),
-                     lat_vertex(cx, cy, cz, t.verts + 3 * (from + (chord ? vw : 1))),
-                     chord ? t.chord[from].g : t.span[q * swe + s].g);
-        }
-}
-
-// The same walk without the cutoffs (lat_pair_fast); where some lane's smallest |r1 x r2|^2 or |r|^2 is
-// within a rounding of its cutoff or below it, or a result is not finite (an input that is not, or a
-// product that overflowed), the wave walks again with them.  Wakes and wings in use keep clear of the
-// cutoffs (1e-10), so that the second walk is rare.
-// Bound by FP64 VALU issue.  Per (receiver, ring) pair at RH = 4: 2.25 segment pairs of 46 slots and
-// 1.25 vertices of 25 against 58 and 24 with the cutoffs inside.
-template <int RH>
-__device__ __forceinline__ void lattice_chunk(const LatTile<RH>& t, int swe, int rhe, int sa, int sb, double cx,
-                                              double cy, double cz, double& vx, double& vy, double& vz) {
-    const int vw = swe + 1;
-    double ax = 0.0, ay = 0.0, az = 0.0;
-    uint32_t low_sq = 0xffffffffu, low_r2 = 0xffffffffu;
+    auto vertex = [&](int q, int s) {
+        const double* v = t.verts + 3 * (q * vw + s);
+        if constexpr (CUT)
+            return lat_vertex(cx, cy, cz, v);
+        else
+            return lat_vertex_fast(cx, cy, cz, v, low_r2);
+    };
+    auto pair = [&](const LatVertex& a, const LatVertex& b, const LatSegment& r) {
+        if constexpr (CUT)
+            lat_pair(ax, ay, az, a, b, r);
+        else
+            lat_pair_fast(ax, ay, az, a, b, r, low_sq);
+    };
+    ax = ay = az = 0.0;
     LatVertex prev[RH + 1];
 #pragma unroll
     for (int q = 0; q <= RH; q++)
-        if (q <= rhe) prev[q] = lat_vertex_fast(cx, cy, cz, t.verts + 3 * (q * vw + sa), low_r2);
+        if (q <= rhe) prev[q] = vertex(q, sa);
     for (int s = sa; s < sb; s++) {
         // chordwise segments of vertex column s (left edge of ring column s)
 #pragma unroll
         for (int q = 0; q < RH; q++)
-            if (q < rhe) lat_pair_fast(ax, ay, az, prev[q], prev[q + 1], t.chord[q * vw + s], low_sq);
+            if (q < rhe) pair(prev[q], prev[q + 1], t.chord[q * vw + s]);
         // vertex column s+1 and the spanwise segments of ring column s
 #pragma unroll
         for (int q = 0; q <= RH; q++) {
             if (q <= rhe) {
-                const LatVertex cur = lat_vertex_fast(cx, cy, cz, t.verts + 3 * (q * vw + s + 1), low_r2);
-                lat_pair_fast(ax, ay, az, prev[q], cur, t.span[q * swe + s], low_sq);
+                const LatVertex cur = vertex(q, s + 1);
+                pair(prev[q], cur, t.span[q * swe + s]);
                 prev[q] = cur;
             }
         }
@@ -808,12 +805,33 @@ __device__ __forceinline__ void lattice_chunk(const LatTile<RH>& t, int swe, int
     if (sb == swe) {  // right edge of the work-group tile: chordwise segments of vertex column swe
 #pragma unroll
         for (int q = 0; q < RH; q++)
-            if (q < rhe) lat_pair_fast(ax, ay, az, prev[q], prev[q + 1], t.chord[q * vw + swe], low_sq);
+            if (q < rhe) pair(prev[q], prev[q + 1], t.chord[q * vw + swe]);
     }
-    constexpr double cut_r2 = BS<double>::cut_norm * BS<double>::cut_norm;
-    const bool near = (low_sq <= hi_word(BS<double>::cut_cross)) | (low_r2 <= hi_word(cut_r2)) |
-                      !(fabs(ax) + fabs(ay) + fabs(az) < __builtin_huge_val());
-    if (__ballot(near) != 0ull) lattice_chunk_cutoffs<RH>(t, swe, rhe, sa, sb, cx, cy, cz, ax, ay, az);
+}
+
+// A wave's walk without the cutoffs, taken again with them where some lane's smallest |r1 x r2|^2 or |r|^2 is
+// within a rounding of its cutoff or below it, or a result is not finite (an input that is not, or a
+// product that overflowed); tiles of rings so small that this is to be expected (t.small) are walked with
+// them from the start.  Adds the induced velocity to (vx, vy, vz).
+// Bound by FP64 VALU issue.  Per (receiver, ring) pair at RH = 4: 2.25 segment pairs of 46 slots and
+// 1.25 vertices of 25 against 58 and 24 with the cutoffs inside.  The cutoffs are absolute (1e-10): a 10 x 40 wing of
+// chord 1 hardly meets them, one of chord 0.05 or less in nearly every tile beside it.
+// 300 steps of 16 such simulations at chord 1, 0.1, 0.05 and 0.01: 68.3, 68.7, 78.1 and 78.7 ms; with the cutoffs
+// inside throughout 81 to 82, with none inside and t.small not tested 67.9, 68.6, 102 and 166.
+template <int RH>
+__device__ __forceinline__ void lattice_chunk(const LatTile<RH>& t, int swe, int rhe, int sa, int sb, double cx,
+                                              double cy, double cz, double& vx, double& vy, double& vz) {
+    double ax = 0.0, ay = 0.0, az = 0.0;
+    uint32_t low_sq = 0xffffffffu, low_r2 = 0xffffffffu;
+    bool careful = __builtin_amdgcn_readfirstlane(t.small) != 0;
+    if (!careful) {
+        lattice_walk<RH, false>(t, swe, rhe, sa, sb, cx, cy, cz, ax, ay, az, low_sq, low_r2);
+        constexpr double cut_r2 = BS<double>::cut_norm * BS<double>::cut_norm;
+        const bool near = (low_sq <= hi_word(BS<double>::cut_cross)) | (low_r2 <= hi_word(cut_r2)) |
+                          !(fabs(ax) + fabs(ay) + fabs(az) < __builtin_huge_val());
+        careful = __ballot(near) != 0ull;
+    }
+    if (careful) lattice_walk<RH, true>(t, swe, rhe, sa, sb, cx, cy, cz, ax, ay, az, low_sq, low_r2);
     constexpr double inv_fourpi = 1.0 / BS<double>::fourpi;
     vx += ax * inv_fourpi;
     vy += ay * inv_fourpi;
@@ -829,6 +847,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const int64_t zo = (int64_t)blockIdx.z * zs;
     partial += (int64_t)blockIdx.z * wzs;
     __shared__ LatTile<RH> st;
+    if (threadIdx.x == 0) st.small = 0;
     double *const sverts = st.verts, *const sgam = st.gam;
     __shared__ double sred[kWaves][kRecv];
     const int tile = blockIdx.y;
