@@ -19,10 +19,11 @@
 // column-by-column k_panel + k_laswp + k_trsm instead.
 // getrs (n <= 16384): the interchanges are composed (k_solve_prep per block of 64 pivots, k_solve_compose
 // over the blocks) and the 64 x 64 diagonal blocks of L and U inverted (k_solve_prep); then up to n = 256 one
-// work-group per right-hand side does the rest (k_solve_small), above that the interchanges are applied
-// (k_solve_perm) and each 256-row step of a substitution runs on all trailing row blocks at once
-// (k_trsv_step), or, with many right-hand sides, 64-row steps multiply all of them on the matrix cores
-// (k_inv_apply, k_update); larger n uses block-row kernels (k_diag_solve / k_off_update).
+// work-group per right-hand side does the rest (k_solve_small).  Above that solve_route chooses: a work-group per
+// right-hand side in 64-row steps (k_solve_blocked), or the interchanges first (k_solve_perm) and each step of
+// a substitution on all trailing row blocks at once (k_trsv_step by 256 rows, k_trsv_block by 64), or, with
+// many right-hand sides, 64-row steps that multiply all of them on the matrix cores (k_inv_apply, k_update); larger
+// n uses block-row kernels (k_diag_solve / k_off_update).
 #include <atomic>
 #include <map>
 #include <utility>
@@ -2309,6 +2310,8 @@ constexpr int kSB = 64;            // solve block
 constexpr int kSW = 4 * kSB;       // rows of a substitution step
 constexpr int kSolveMaxN = 16384;  // rhs column in LDS
 constexpr int kSolvePairs = 1 + 2 * 2 * kSB;
+constexpr int kBlockedMaxN = 1024;  // rhs column of k_solve_blocked in LDS (two work-groups a CU; with 16384 rows
+                                    // one, and 1.3 times the time)
 
 // y = 0: composes the interchanges of pivot block b (64 positions) into (dst, src) pairs (one wave);
 // y = 1 / 2: inverts the 64 x 64 diagonal block b of L (unit lower) / U (upper): each wave one 16 x 16
@@ -2634,6 +2637,106 @@ __global__ __launch_bounds__(1024) void k_trsv_step(const T* __restrict__ a, int
     if (t < min(kSW, nr)) xc[r0 + t] = xn[t];
 }
 
+// One work-group per right-hand side, its column in LDS, 64 rows at a time: each off-diagonal row of tiles is
+// read where its rows are solved, 64 consecutive rows per column, split over the 16 waves.
+template <typename T>
+__global__ __launch_bounds__(1024) void k_solve_blocked(const T* __restrict__ a, int64_t lda, int n,
+                                                        const int32_t* __restrict__ perm, const T* __restrict__ inv,
+                                                        T* __restrict__ x, int64_t ldx, int64_t sa, int64_t sx) {
+    __shared__ T xs[kBlockedMaxN];
+    __shared__ T red[16][kSB];
+    __shared__ T yb[kSB];
+    const int t = threadIdx.x, r = t & 63, g = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nblk = (n + kSB - 1) / kSB;
+    a += (int64_t)blockIdx.z * sa;  // batch: one matrix per blockIdx.z
+    perm += (int64_t)blockIdx.z * n;
+    inv += (int64_t)blockIdx.z * 2 * nblk * kSB * kSB;
+    T* xc = x + (int64_t)blockIdx.z * sx + (int64_t)blockIdx.x * ldx;
+    for (int i = t; i < n; i += 1024) xs[i] = xc[perm[i]];
+    __syncthreads();
+    for (int e = 0; e < 2 * nblk; e++) {  // L from the first block on, then U from the last
+        const bool lower = e < nblk;
+        const int b = lower ? e : 2 * nblk - 1 - e;
+        const int r0 = b * kSB, rb = min(kSB, n - r0);
+        const T* ib = inv + ((int64_t)(lower ? 0 : nblk) + b) * kSB * kSB;
+        T acc = T(0);
+        if (r < rb)
+            for (int j = (lower ? 0 : r0 + kSB) + g; j < (lower ? r0 : n); j += 16)
+                acc += a[(r0 + r) + (int64_t)j * lda] * xs[j];
+        red[g][r] = acc;
+        __syncthreads();
+        if (t < kSB) {
+            T y = t < rb ? xs[r0 + t] : T(0);
+#pragma unroll
+            for (int q = 0; q < 16; q++) y -= red[q][t];
+            yb[t] = y;
+        }
+        __syncthreads();
+        T s = T(0);
+#pragma unroll
+        for (int p = 4 * g; p < 4 * g + 4; p++) s += ib[r + p * kSB] * yb[p];
+        red[g][r] = s;
+        __syncthreads();
+        if (t < rb) {
+            T v = T(0);
+#pragma unroll
+            for (int q = 0; q < 16; q++) v += red[q][t];
+            xs[r0 + t] = v;
+        }
+        __syncthreads();
+    }
+    for (int i = t; i < n; i += 1024) xc[i] = xs[i];
+}
+
+// k_trsv_step's substitutions by 64 rows: work-group j subtracts the part of block b's rows from the j-th block
+// after it (forward) or before it (backward), group 0 then finishes its block with the inverse.
+template <typename T, bool LOWER>
+__global__ __launch_bounds__(256) void k_trsv_block(const T* __restrict__ a, int64_t lda, int n,
+                                                    const T* __restrict__ inv, T* __restrict__ x, int64_t ldx,
+                                                    int64_t sa, int64_t sx, int b) {
+    __shared__ T xb[kSB];
+    __shared__ T red[4][kSB];
+    __shared__ T yb[kSB];
+    const int t = threadIdx.x, rl = t & 63, g = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nblk = (n + kSB - 1) / kSB;
+    a += (int64_t)blockIdx.z * sa;
+    inv += (int64_t)blockIdx.z * 2 * nblk * kSB * kSB + (LOWER ? 0 : (int64_t)nblk * kSB * kSB);
+    T* xc = x + (int64_t)blockIdx.z * sx + (int64_t)blockIdx.y * ldx;
+    const int j = blockIdx.x;
+    const int r = LOWER ? b + 1 + j : b - 1 - j;  // this group's row block
+    const int r0 = r * kSB, c0 = b * kSB;
+    T y = T(0);
+    if (t < kSB) y = r0 + t < n ? xc[r0 + t] : T(0);
+    if (LOWER ? b >= 0 : b < nblk) {
+        if (t < kSB) xb[t] = c0 + t < n ? xc[c0 + t] : T(0);
+        __syncthreads();
+        T acc = T(0);
+        if (r0 + rl < n) {
+            const T* ab = a + (r0 + rl) + (int64_t)c0 * lda;
+#pragma unroll 4
+            for (int c = 16 * g; c < 16 * g + 16; c++)
+                if (c0 + c < n) acc += ab[(int64_t)c * lda] * xb[c];
+        }
+        red[g][rl] = acc;
+        __syncthreads();
+        if (t < kSB) y -= red[0][t] + red[1][t] + red[2][t] + red[3][t];
+    }
+    if (j != 0) {  // a later block: store the partial update
+        if (t < kSB && r0 + t < n) xc[r0 + t] = y;
+        return;
+    }
+    // the next block in order: finish it with its diagonal-block inverse
+    if (t < kSB) yb[t] = y;
+    __syncthreads();
+    const T* ib = inv + (int64_t)r * kSB * kSB;
+    T s = T(0);
+#pragma unroll
+    for (int p = 16 * g; p < 16 * g + 16; p++) s += ib[rl + p * kSB] * yb[p];
+    red[g][rl] = s;
+    __syncthreads();
+    if (t < kSB && r0 + t < n) xc[r0 + t] = red[0][t] + red[1][t] + red[2][t] + red[3][t];
+}
+
 // X_b = inv X_b for the 64 rows of a diagonal block (rb of them in the matrix) and all right-hand sides, a wave
 // per 16 of them, on the matrix cores
 template <typename T>
@@ -2668,11 +2771,35 @@ __global__ __launch_bounds__(256) void k_inv_apply(const T* __restrict__ inv, T*
     }
 }
 
-// Right-hand sides times rows from which the substitutions run as products over all right-hand sides.  Below,
-// a step per 256 rows and right-hand side is faster or equal.  At the line, steps and products: 128 rhs of 4096
-// FP64 rows 2.80 and 2.64 ms (FP32 1.69 and 1.95), 64 of 8192 rows 6.1 and 5.7 ms (3.86 and 3.89), 1024 of 600 rows
-// 0.49 and 0.42 ms (0.31 and 0.33); at twice that, 256 of 4096 rows, 4.9 and 2.7 ms (3.0 and 2.0).
-constexpr int64_t kManyRhs = 512 * 1024;
+// How a solve past kSW rows runs.  Each line lies about where the two sides measured alike (us; in brackets n,
+// matrices, right-hand sides each):
+//   kRouteBlocked, a work-group per right-hand side: a single launch where the steps' chain has two and more per 256
+//     rows (FP64 [300, 1, 1]: 63 and 36), and enough work-groups with many right-hand sides (FP64 [600, 1, 96]: 122
+//     and 79, [700, 2, 200]: 317 and 169; FP32 [700, 1, 200]: 116 and 77, but [1000, 8, 200]: 939 and 1166);
+//   kRouteProducts, 64 rows at a time as products over all right-hand sides of a matrix ([4096, 1, 200]: steps FP64 4015,
+//     products 2641; FP32 2413 and 1993);
+//   kRouteBlocks, steps of 64 rows: a step of 256 rows and right-hand side holds a work-group of 1024 threads through
+//     its serial part, which many right-hand sides queue for (FP64 [4096, 1, 48]: 1434 and 1198, [4096, 1, 24]: 1018
+//     and 1059; FP32 [8100, 1, 48]: 3318 and 2934);
+//   kRouteSteps otherwise.
+// The route, and with it the rounding, depends on the number of matrices only from 8 matrices and 8 right-hand sides
+// on: a served request gives the same answer in any batch.
+enum SolveRoute { kRouteSteps, kRouteBlocked, kRouteBlocks, kRouteProducts };
+
+template <typename T>
+SolveRoute solve_route(int64_t n, int64_t nrhs, int64_t batch) {
+    constexpr bool f64 = sizeof(T) == 8;
+    const int64_t rows = nrhs * n;
+    if (rows >= (n <= 896 ? 1024 : f64 ? 896 : 768) * 1024) return kRouteProducts;
+    if (n <= 320) return kRouteBlocked;
+    if (n <= kBlockedMaxN) {
+        if (nrhs >= (f64 ? (n <= 640 ? 64 : 200) : n <= 512 ? 512 : n <= 896 ? 160 : INT64_MAX)) return kRouteBlocked;
+        if (batch >= 8 && nrhs >= 8 && nrhs * batch >= 256 && (f64 || (n > 512 && n <= 896))) return kRouteBlocked;
+        return kRouteSteps;
+    }
+    if (f64 ? rows >= (n < 1400 ? 256 : 128) * 1024 : n >= 3072 && rows >= 376 * 1024) return kRouteBlocks;
+    return kRouteSteps;
+}
 
 // What getrs makes of the factors before it sees a right-hand side: inverses of the diagonal blocks, the
 // composed interchanges, and the lists they come from.
@@ -2707,10 +2834,31 @@ struct SolvePrep {
             TVLM_LAUNCHED();
             return TVLM_OK;
         }
+        SolveRoute route = solve_route<T>(n, nrhs, batch);
+        if (route == kRouteProducts && (lda >= kUpdMaxLd || ldx >= kUpdMaxLd)) route = kRouteBlocks;
+        if (route == kRouteBlocked) {
+            hipLaunchKernelGGL(k_solve_blocked<T>, dim3(nrhs, 1, batch), dim3(1024), 0, st, a, lda, n, perm, inv, x, ldx,
+                               sa, sx);
+            TVLM_LAUNCHED();
+            return TVLM_OK;
+        }
         hipLaunchKernelGGL(k_solve_perm<T>, dim3(nrhs, 1, batch), dim3(1024), 0, st, n, perm, x, ldx, sx);
         TVLM_LAUNCHED();
         const int nblk = (n + kSB - 1) / kSB, nst = (n + kSW - 1) / kSW;
-        if ((int64_t)nrhs * n >= kManyRhs && lda < kUpdMaxLd && ldx < kUpdMaxLd) {
+        if (route == kRouteBlocks) {
+            for (int b = -1; b < nblk - 1; b++) {
+                hipLaunchKernelGGL((k_trsv_block<T, true>), dim3(b < 0 ? 1 : nblk - 1 - b, nrhs, batch), dim3(256), 0, st,
+                                   a, lda, n, inv, x, ldx, sa, sx, b);
+                TVLM_LAUNCHED();
+            }
+            for (int b = nblk; b > 0; b--) {
+                hipLaunchKernelGGL((k_trsv_block<T, false>), dim3(b == nblk ? 1 : b, nrhs, batch), dim3(256), 0, st, a, lda,
+                                   n, inv, x, ldx, sa, sx, b);
+                TVLM_LAUNCHED();
+            }
+            return TVLM_OK;
+        }
+        if (route == kRouteProducts) {
             for (int z = 0; z < batch; z++) {
                 const T* az = a + (int64_t)z * sa;
                 const T* iz = inv + (int64_t)z * 2 * nblk * kSB * kSB;
