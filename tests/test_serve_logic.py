@@ -4,6 +4,7 @@ mesh's cap and the lane count, no plan takes a second batch while one is running
 holds (least recently used idle plans are evicted), admission is oldest-first across meshes, and
 unsteady requests run on plans bound to one lane."""
 import itertools
+import time
 
 import numpy as np
 import pytest
@@ -357,3 +358,26 @@ def test_hb_request_errors(S, monkeypatch):
         with pytest.raises(RuntimeError, match="diverged"):
             srv.run([S.Request(0, "wf", kind="hb", hb={"omega": 1, "U": -1, "dyn": np.zeros((3, 3))})],
                     realtime=False)
+
+
+@pytest.mark.parametrize("run,plans", [(0.5, 2), (0.003, 1)])
+def test_lone_request_waits_a_bounded_time(S, monkeypatch, run, plans):
+    """A second request of a mesh, alone in its queue while the first runs: it gets a plan of its own long before a
+    long run ends, and takes the first plan after a short one."""
+    class Timed(FakePlan):
+        def solve(self, *a, **k):
+            super().solve(*a, **k)
+            self.until = time.perf_counter() + run
+
+        def done(self):
+            return time.perf_counter() >= self.until
+
+    monkeypatch.setattr(S, "SteadyPlan", Timed)
+    with S.Server({"a": _mesh(16)}, lanes=3, max_batch=4, budget_bytes=1 << 40) as srv:
+        first, second = S.Request(0, "a", 0.1, arrival=0.0), S.Request(1, "a", 0.1, arrival=0.001)
+        st = srv.run([first, second])
+        assert st.plans_created == plans
+        if plans == 2:
+            assert second.admitted - first.admitted < run / 2
+        else:
+            assert second.admitted >= first.finished

@@ -23,10 +23,10 @@ Structure
   with copies of its first motion, whose results are dropped.
 - admission: whenever a lane is free, the queue (steady: per mesh; unsteady: per mesh) whose oldest
   waiting request arrived first is served: for steady requests an idle plan of that mesh (or a new
-  one, if the mesh has none or at least two of its requests wait) takes up to its cap of that mesh's
-  waiting requests, in arrival order.  Requests that arrive
-  while others are on the device are admitted as soon as a lane and a plan (memory) are free,
-  whatever else is running.
+  one) takes up to its cap of that mesh's waiting requests, in arrival order; a request alone in its
+  queue first waits for the mesh's running plan, until that has run for LONE_WAIT_S.
+  Requests that arrive while others are on the device are admitted as soon as a lane and a plan
+  (memory) are free, whatever else is running.
 
 A request's result does not depend on the batch it shared: each matrix of a batched LU is factored
 independently, and the FP64 refinement drives every solution to the FP64 solution of its own FP64
@@ -221,6 +221,13 @@ def stream_destroy(s: int) -> None:
     H.check(H.lib().tvlm_stream_destroy(ctypes.c_void_p(s)), "tvlm_stream_destroy")
 
 
+# How old a mesh's oldest run may be for a lone request of the mesh to wait for it.  Solves of up to about 2000 panels
+# end within it, and two requests that meet share a batch instead of a further plan with its memory; of longer
+# solves only this much is waited for.  72 requests of the mix on 4 lanes, 2, 0.6 and 0.3 ms apart: mean latency with
+# and without the wait the same within the runs' spread (2.5, 4.8 to 7.3 and 12 to 20 ms), 11 plans instead of 13.
+LONE_WAIT_S = 4e-3
+
+
 @dataclass
 class _Slot:
     plan: object  # SteadyPlan, or UVLMPlan for unsteady requests
@@ -228,6 +235,7 @@ class _Slot:
     busy: bool = False
     last_used: float = 0.0
     unsteady: bool = False
+    started: float = 0.0  # perf_counter when its current run was queued
 
 
 @dataclass
@@ -347,6 +355,14 @@ class Server:
             self.used_bytes -= s.bytes
             self.stats.plans_evicted += 1
         return True
+
+    def _lone_waits(self, key: str, queued: int) -> bool:
+        """Whether a lone request waits for one of its mesh's running plans instead of having a further one
+        created: until the run that began first has lasted LONE_WAIT_S."""
+        slots = self.slots[key]
+        if queued >= 2 or not slots or any(not s.busy for s in slots):
+            return False
+        return time.perf_counter() - min(s.started for s in slots) < LONE_WAIT_S
 
     def _slot_for(self, key: str, lane: int, now: float) -> _Slot | None:
         for s in self.slots[key]:
@@ -526,10 +542,7 @@ class Server:
                     if kind == "unsteady":
                         slot = self._uslot_for(mesh, free_lanes[0], now, self.usims(len(waiting[k])))
                     else:
-                        # A lone request waits for its mesh's running plan: a further plan takes milliseconds
-                        # to create, during which nothing else is admitted, about as long as the running
-                        # solve (72 requests on 4 lanes, 0.6 ms apart: mean latency 9.1 -> 7.4 ms).
-                        if len(waiting[k]) < 2 and self.slots[mesh] and all(s.busy for s in self.slots[mesh]):
+                        if self._lone_waits(mesh, len(waiting[k])):
                             continue
                         slot = self._slot_for(mesh, free_lanes[0], now)
                     if slot is not None:
@@ -560,6 +573,7 @@ class Server:
                 batch = [q.popleft() for _ in range(min(self.cap[mesh], len(q)))]
                 slot.plan.set_stream(self.lanes[lane])
                 slot.busy = True
+                slot.started = time.perf_counter()
                 slot.plan.solve(np.asarray([r.alpha for r in batch]), u_inf=self.u_inf, rho=self.rho)
                 t = time.perf_counter() - t0
                 for r in batch:
