@@ -200,7 +200,8 @@ int tvlm_lu_set_coop_spin_limit(uint32_t limit);
 
 /* Library-wide work-group targets of the wake-induction launches (no counterpart in the reference;
  * tuning knobs that tinyvlm_amd.autotune sets from its cached measurements): wake_groups for the
- * Backend form (Backend::rhs_assemble_wake_influence and the plain UVLM loop, default 2048),
+ * Backend form (Backend::rhs_assemble_wake_influence and the plain UVLM loop, default 2048: tiles take
+ * as few wake rows as stay within it, and two instead of one where that leaves a fifth of it),
  * lattice_groups for UVLM plans created afterwards (fast mode, default 1024; per plan:
  * tvlm_uvlm_set_lattice_target).  0 restores a default; range [64, 65536]. */
 int tvlm_set_tile_targets(int32_t wake_groups, int32_t lattice_groups);

@@ -588,19 +588,22 @@ inline void launch_wake_reduce(T* rhs, int64_t rhs_stride, const T* partial, int
 }
 
 // Tile shape of one wake surface: spans per tile sw <= kMaxSpanTile, rows per tile rh with
-// rh * sw <= kTileRings, as few as give the launch about half of wake_target_groups() work-groups
-// (receiver blocks x tiles).  Half: rows of one tile share the segments between them (400 receivers x 200
-// x 40 rings take two rows and 700 work-groups; one row and 1400 work-groups measured 52 us against
-// 45 us for the whole call).
+// rh * sw <= kTileRings, as few rows as keep the launch within wake_target_groups() work-groups
+// (receiver blocks x tiles).  A tile's rows share the segments between them, so that two rows are taken for one
+// where that leaves a fifth of the target: 400 receivers x 40 spans, 200 rows: 45 us with two rows (700 work-groups),
+// 52 with one; 100 rows: 34 (350) and 31; 85 receivers x 17 spans x 500 rows: 23 (500) and 25.  Three rows are walked
+// as two and one, and four took 194 us where they took 229 (1800 receivers x 60 spans x 200 rows).
 inline void wake_tile_shape(int ns, int rows, int recv_blocks, int& sw, int& rh) {
     sw = ns < kMaxSpanTile ? ns : kMaxSpanTile;
     const int tiles_span = (ns + sw - 1) / sw;
+    const int64_t groups = (int64_t)recv_blocks * tiles_span;  // per row tile
     int rh_max = kTileRings / sw;
     if (rh_max < 1) rh_max = 1;
-    int want_row_tiles = wake_target_groups() / (2 * recv_blocks * tiles_span);
+    int64_t want_row_tiles = wake_target_groups() / groups;
     if (want_row_tiles < 1) want_row_tiles = 1;
-    rh = (rows + want_row_tiles - 1) / want_row_tiles;
-    if (rh < 1) rh = 1;
+    rh = (int)((rows + want_row_tiles - 1) / want_row_tiles);
+    if (rh <= 1) rh = (rows + 1) / 2 * groups * 5 >= wake_target_groups() ? 2 : 1;
+    if (rh == 3) rh = 4;
     if (rh > rh_max) rh = rh_max;
 }
 
