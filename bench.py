@@ -16,7 +16,7 @@ and 1/x from the FP64 hardware estimates plus one Newton step) over the shared-s
 wake, with the far wake aggregated (ring rows older than 80 / 160 / 320 steps merged into 2x4 / 4x8 /
 8x8 rings of mean circulation; --exact-wake turns this off), solves with the FP64 inverse and replays
 the loop as one hipGraph; it is accepted only if |dCL| <= 1e-6 at every step of every simulation
-against the plain FP64 path (exact FP64 Biot-Savart ring by ring over the whole wake, LU substitution
+against the plain FP64 path (exact FP64 Biot-Savart over the whole wake, LU substitution
 each step, one simulation at a time), which is timed too, and so is the served batch with the exact
 wake ("served_exact_wake") and one simulation per plan ("single_simulation": the latency a lone
 request sees).
@@ -25,8 +25,8 @@ Also reported under "served_uvlm": 64 such simulations requested at once through
 (4 lanes, each running up to 8 simulations in one plan).  --batched-only prints only a batch's rate
 and wake roofline (for profiler runs).
 
-Also reported: the roofline of the dominant kernel (wake induction, 398 algorithmic flops per
-receiver x wake-ring pair -- the ring-by-ring count of the reference algorithm -- timed with HIP
+Also reported: the roofline of the dominant kernel (wake induction, 170 algorithmic flops per
+receiver x wake-ring pair -- every segment and vertex of the ring lattice once -- timed with HIP
 events on the plan's stream, against the FP64 VALU peak since it computes in FP64) and the CPU
 baseline (the oracle's FP64 restatement of the reference CPU backend, OpenMP on the host cores).
 
@@ -37,7 +37,7 @@ against the plain FP64 path (one request at a time, exact FP64 assembly, FP64 LU
 them on the same angles, per-batch latency, and one CPU solve of the oracle.
 
 Also reported under "assembly": the influence-matrix assembly of the same elliptic mesh in FP32
-(rsqrt form) and FP64 (exact form), TFLOP/s at 398 flops per pair against the VALU rates.
+(rsqrt form) and FP64 (exact form), TFLOP/s at 170 flops per pair against the VALU rates.
 
 Also reported under "hb": the harmonic-balance driver (the libhbvlm3 interface) on a rectangular
 wing/flap section of chord 2b = 0.254 and span 8 chords (wing 20 + flap 10 chordwise x 20 spanwise =
@@ -65,7 +65,9 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-FLOPS_PER_PAIR = 398  # algorithmic flops per (receiver, ring) pair, both mirror images
+# Flops that a (receiver, ring) pair of a lattice cannot do without: the ring's two own segments and one own vertex
+# (the others are its neighbours'), for the receiver and its mirror image, and the dot product with the normal.
+FLOPS_PER_PAIR = 170
 PEAK_FP64_VALU_TFLOPS = 78.6  # MI355X FP64 vector peak (also non-packed FP32)
 COPY_PROBE_BYTES = 1 << 30
 # HBM bytes per k_wake_lattice launch of this workload (mean over its 499 launches), from the
@@ -456,7 +458,7 @@ PEAK_FP32_VALU_PACKED_TFLOPS = 157.3  # MI355X FP32 vector peak with packed FP32
 
 def assembly_bench(reps=5):
     """Influence-matrix assembly (tvlm_lhs_assemble_*, the reference's lhs_assemble) of the elliptic
-    64 x 64 mesh (N = 4096, 16.8 M receiver x ring pairs, 398 flops each) in FP32 (rsqrt form) and
+    64 x 64 mesh (N = 4096, 16.8 M receiver x ring pairs, 170 flops each) in FP32 (rsqrt form) and
     FP64 (exact form), timed with HIP events on torch's current stream."""
     import torch
 
@@ -1025,8 +1027,8 @@ def main():
     wkey = ("exact" if args.exact_wake else "far") + (f"_sims{B}" if B > 1 else "")
     roofline = counters(wake_roofline(fast, wall / args.steps), wkey)
     roofline["pairs_note"] = (f"pairs = receivers x wake rings evaluated per launch, over all {B} simulations "
-                              "(with far-wake aggregation: the exact rings plus the coarse rings); 398 flops per "
-                              "pair, the ring-by-ring count")
+                              "(with far-wake aggregation: the exact rings plus the coarse rings); 170 flops per "
+                              "pair, every lattice segment and vertex once")
     wake_ms_p, launches_p, pairs_p = plain.time_wake()
     roofline["plain_fp64_wake_tflops"] = round(FLOPS_PER_PAIR * pairs_p / (wake_ms_p * 1e-3) / 1e12, 3)
     fast.close()

@@ -135,8 +135,7 @@ int lhs_assemble(const tvlm_view* lhs, int32_t n_surf, const tvlm_view* colloc, 
 // fixed_bytes (nothing is allocated; a launch that needs more is rejected before any work is
 // queued); when null, to the library's per-stream workspace (grown on demand).
 // lattice (FP64 only): the wake's vortex lattice in the FP64 seeded form (k_wake_lattice, the served
-// UVLM loop's kernel: every lattice segment once, with the difference of the circulations of the
-// two rings beside it) instead of ring by ring.
+// UVLM loop's kernel) instead of the exact form.
 template <typename T>
 int wake_influence(const tvlm_view* rhs, int32_t n_surf, const tvlm_view* gamma_wake, const tvlm_view* colloc,
                    const tvlm_view* normals, const tvlm_view* verts_wake, const uint8_t* lifting, int32_t iteration,

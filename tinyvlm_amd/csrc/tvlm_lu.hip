@@ -286,8 +286,9 @@ __device__ int wave_compose_swaps(int first, int cnt, const int* piv, int* pd, i
 // round 3's, or factors the panel itself where all failed.  A matrix whose panels failed kSpecFails
 // times in a row skips the rounds from then on, up to the panels whose rows are all candidates.
 // On the influence matrices of rectangular and 25-degree swept wings every panel stands in round 1;
-// on the elliptic ones (pivots at the tip panels, up to 1538 rows below the diagonal) up to half in
-// round 1, most others in round 2 and, at 64 x 64, a quarter in round 3.
+// on the elliptic ones (pivots at the tip panels, up to 1538 rows below the diagonal) all (16 x 16, 12 spans
+// x 100), 7 of 17 (100 spans x 12), 3 of 30 (45 x 45) or none (64 x 64) do, most others in round 2 and, at 64 x
+// 64, a quarter in round 3.
 //
 // Every work-group factors the candidates for itself (a 64-step chain in registers and LDS: one
 // launch and no exchange) and then takes its share of the other rows, 16 per wave and step on the
@@ -1234,7 +1235,7 @@ constexpr int kCoopMaxGroups = 64;   // work-groups of one launch; all of them m
 constexpr int kCoopMinRows = 1024;   // shorter panels stay in one work-group (k_panel_reg)
 constexpr unsigned kCoopSpinLimit = 1u << 22;  // default bound of every wait (tvlm_lu_set_coop_spin_limit)
 constexpr int kCoopStalled = -999;
-constexpr int kCoopCtr = NB + 4;                                         // counters per panel and matrix
+constexpr int kCoopCtr = NB + 4;  // ints between the counter sets of a panel and matrix (NB counters each)
 constexpr int64_t kCoopXrow = (int64_t)NB * (kCoopMaxGroups + 1) * NB;  // xrow per matrix
 
 template <typename T>
@@ -2080,12 +2081,12 @@ constexpr int kGroupMinRows = 3072;  // trailing matrices at least this tall are
 // exported as tvlm_getrf_plan so that the schedule and the buffer sizing can be checked without a GPU.
 //   kPathLookahead : batches of >= kWidePanelBatch matrices of <= kFastPanelRows rows (one-group panels
 //                    beside the trailing updates on a side stream);
-//   kPathCoopPairs : the first panel is cooperative; then every panel of more than kCoopMinRows rows is
+//   kPathCoop      : the first panel is cooperative; then every panel of more than kCoopMinRows rows is
 //                    (coop_groups falls with the rows) and takes its own counter set;
 //   kPathPanels    : one work-group per panel throughout (k_panel_reg, or the column-by-column k_panel
 //                    above kFastPanelRows rows) -- also every factorisation with cooperative panels
 //                    switched off.
-enum GetrfPath { kPathLookahead = 0, kPathCoopPairs = 1, kPathPanels = 2 };
+enum GetrfPath { kPathLookahead = 0, kPathCoop = 1, kPathPanels = 2 };
 
 struct GetrfStep {
     int kp, kb;   // first column and width of the panel
@@ -2095,10 +2096,10 @@ struct GetrfStep {
 
 struct GetrfPlan {
     int path = kPathPanels;
-    std::vector<GetrfStep> steps;  // kPathCoopPairs only
+    std::vector<GetrfStep> steps;  // kPathCoop only
     int ctr_sets = 0;              // counter sets allocated (one per cooperative panel)
-    // exchange buffers (kPathCoopPairs): ints (counters, per-matrix attempt state and failure word,
-    // candidate rows, gather lists) and reals (candidate values, published rows and U11)
+    // exchange buffers (kPathCoop): ints (counters, per-matrix failure word, candidate
+    // rows, gather lists) and reals (candidate values, published rows)
     size_t nctr = 0, ncand = 0, nrow = 0, ngat = 0;
     size_t coop_bytes(size_t real_bytes) const {
         return nctr || ncand ? sizeof(int32_t) * (nctr + ncand + ngat) + real_bytes * (ncand + nrow) + 512 : 0;
@@ -2116,14 +2117,14 @@ GetrfPlan getrf_plan(int n, int batch, bool allow_coop) {
         P.path = kPathPanels;
         return P;
     }
-    P.path = kPathCoopPairs;
+    P.path = kPathCoop;
     for (int kp = 0; kp < n; kp += NB) {
         GetrfStep st{kp, n - kp < NB ? n - kp : NB, coop_groups<T>(n - kp, batch), -1};
         if (st.groups > 0) st.ctr_set = P.ctr_sets++;
         P.steps.push_back(st);
     }
     const int panels = (n + NB - 1) / NB;
-    P.nctr = (size_t)P.ctr_sets * batch * kCoopCtr + 2 * (size_t)batch;
+    P.nctr = (size_t)P.ctr_sets * batch * kCoopCtr + 2 * (size_t)batch;  // (batch words would do)
     P.ncand = (size_t)batch * NB * kCoopMaxGroups;
     P.nrow = (size_t)batch * kCoopXrow;
     P.ngat = (size_t)batch * panels * n;
@@ -2131,7 +2132,7 @@ GetrfPlan getrf_plan(int n, int batch, bool allow_coop) {
 }
 
 template <typename T>
-int getrf_coop_pairs(T* a, int64_t lda, int n, int batch, int64_t sb, int32_t* ipiv, int32_t* info, int32_t* perm,
+int getrf_coop(T* a, int64_t lda, int n, int batch, int64_t sb, int32_t* ipiv, int32_t* info, int32_t* perm,
                      hipStream_t st, const GetrfPlan& plan, int32_t* ctr, T* cval, int32_t* crow, T* xrow,
                      int32_t* gtab, int32_t* fail, const SpecWork<T>& spec) {
     if (n > NB) {
@@ -2219,7 +2220,7 @@ int getrf(const tvlm_view* av, int32_t* ipiv, int32_t* info, void* stream, bool 
     int32_t* perm = static_cast<int32_t*>(ws);
     const GetrfPlan plan = getrf_plan<T>(n, batch, allow_coop);
     void* cws = nullptr;
-    if (plan.path == kPathCoopPairs) TVLM_TRY(device_workspace(plan.coop_bytes(sizeof(T)), &cws, kWsLuCoop, st));
+    if (plan.path == kPathCoop) TVLM_TRY(device_workspace(plan.coop_bytes(sizeof(T)), &cws, kWsLuCoop, st));
     // Speculative panels wherever a panel kernel of at most kFastPanelRows rows or a cooperative one
     // follows them.  With a spin limit set (a diagnostic), cooperative factorisations go without, so that
     // the waits it bounds are run.
@@ -2227,7 +2228,7 @@ int getrf(const tvlm_view* av, int32_t* ipiv, int32_t* info, void* stream, bool 
     // Without room for their buffers the panels go without as well.
     void* sws = nullptr;
     if (n > spec_min_rows<T>(batch) && n <= kSpecMaxRows &&
-        (plan.path == kPathCoopPairs ? g_coop_spin_limit.load() == kCoopSpinLimit : n <= kFastPanelRows)) {
+        (plan.path == kPathCoop ? g_coop_spin_limit.load() == kCoopSpinLimit : n <= kFastPanelRows)) {
         const int rc = device_workspace(SpecWork<T>::bytes(n, batch), &sws, kWsLuSpec, st);
         if (rc == TVLM_ERR_NOMEM)
             (void)hipGetLastError();
@@ -2242,11 +2243,10 @@ int getrf(const tvlm_view* av, int32_t* ipiv, int32_t* info, void* stream, bool 
         TVLM_LAUNCHED();
     }
     if (plan.path == kPathLookahead) return getrf_lookahead<T>(a, lda, n, batch, sb, ipiv, info, perm, st, spec);
-    if (plan.path == kPathCoopPairs) {
+    if (plan.path == kPathCoop) {
         // Buffers (sized by the plan): per cooperative panel and matrix kCoopCtr counters, per matrix
-        // the attempt counter and the failure word (all zeroed here, once for the whole
-        // factorisation), the candidates, the published rows and U11, and the deferred
-        // interchanges' gather lists.
+        // the failure word (all zeroed here, once for the whole factorisation), the candidates, the
+        // published rows, and the deferred interchanges' gather lists.
         int32_t* ctr = static_cast<int32_t*>(cws);
         int32_t* crow = ctr + plan.nctr;
         T* cval = reinterpret_cast<T*>((reinterpret_cast<uintptr_t>(crow + plan.ncand) + 255) & ~(uintptr_t)255);
@@ -2257,7 +2257,7 @@ int getrf(const tvlm_view* av, int32_t* ipiv, int32_t* info, void* stream, bool 
                            (int64_t)plan.nctr);
         TVLM_LAUNCHED();
         int32_t* fail = ctr + (size_t)plan.ctr_sets * batch * kCoopCtr;  // per matrix: a wait gave up
-        return getrf_coop_pairs<T>(a, lda, n, batch, sb, ipiv, info, perm, st, plan, ctr, cval, crow, xrow, gtab,
+        return getrf_coop<T>(a, lda, n, batch, sb, ipiv, info, perm, st, plan, ctr, cval, crow, xrow, gtab,
                                    fail, spec);
     }
     for (int k0 = 0; k0 < n;) {

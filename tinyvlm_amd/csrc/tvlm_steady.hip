@@ -7,7 +7,8 @@
 // (iteration 1: the trailing-edge columns also see the one wake row), rhs = -(V_inf . n), solve,
 // circulation differences, steady forces and per-surface CL/CM.
 //   mode 0 (plain FP64): exact FP64 assembly, FP64 LU and substitution, one request after another;
-//                        this is the reference's arithmetic, operation for operation.
+//                        the reference's terms, IEEE square roots and divisions and cutoffs, with the
+//                        segments shared between rings and contracted (SegForm).
 //   mode 1 (served)    : every request's FP64 influence matrix in the seeded form, stored rounded to
 //                        FP32 as well, one batched FP32 LU for all requests, then FP64 iterative refinement
 //                        x += A32^{-1} (b - A64 x) (kRefine + 1 corrections, residual in FP64 against

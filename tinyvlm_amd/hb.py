@@ -189,9 +189,9 @@ class HBVLM:
         # replayed from a hipGraph (use_graph = False: launched call by call, the same kernels)
         self.stream = torch.cuda.Stream()
         self.use_graph = True
-        # wake induction of the map: "exact" (Backend::rhs_assemble_wake_influence ring by ring, the
-        # reference's evaluation) or "lattice" (the same sum over the wake's vortex lattice, every
-        # segment once, FP64 seeded; agrees with "exact" to rounding)
+        # wake induction of the map: "exact" (Backend::rhs_assemble_wake_influence: IEEE square
+        # roots and divisions) or "lattice" (the same sum in the FP64 seeded form; agrees with "exact" to
+        # rounding)
         self.wake_form = "exact"
 
     # ---- HBVLM::init (lib/libhbvlm3.cpp:168-233) ------------------------------------------------
