@@ -298,10 +298,11 @@ __device__ int wave_compose_swaps(int first, int cnt, const int* piv, int* pd, i
 // matrix in FP64), while its multipliers stay below 1; with it the factors are as accurate as column by column
 // up to spec_condition_limit, past which the round fails.  The MFMA output layout is the
 // second operand's layout, so the blocks chain without moving between lanes.  What bounds it is the
-// candidates' chain, 64 dependent pivot steps.  Per 4096-row FP64 panel of one matrix, round 1 takes 21 us
-// (loads 2.3, chain 12.8, inverses and staging 2.8, rows 2.9; FP32 17 us) and a later round 52 us (its
-// chain 41: the pivot search and v_readlane broadcasts); the cooperative panel with an exchange per panel
-// took 153 us, with an exchange per column 327 us.
+// candidates' chain, 64 dependent pivot steps.  Per 4096-row FP64 panel of one matrix, round 1 took 21 us
+// (loads 2.3, chain 12.8, inverses and staging 2.8, rows 2.9; FP32 17 us) before the correction and a later
+// round 52 us (its chain 41: the pivot search and v_readlane broadcasts); over all panels of such a matrix round 1
+// takes 22.0 us without the correction and the condition, 23.6 with them.  The cooperative panel with an exchange
+// per panel took 153 us, with an exchange per column 327 us.
 typedef float vf4 __attribute__((ext_vector_type(4)));
 typedef double vd4 __attribute__((ext_vector_type(4)));
 
